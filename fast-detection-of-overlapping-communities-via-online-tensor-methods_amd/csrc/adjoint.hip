@@ -19,79 +19,352 @@
 
 namespace mmsb {
 
-// per column j: the three K matrices, and the column means needed for kappa and the loss
-__global__ void adj_elem_kernel(int32_t nb, int32_t k, const double* __restrict__ A, const double* __restrict__ B,
-                                const double* __restrict__ C, const double* __restrict__ m, double c3, double c1,
-                                double* __restrict__ KA, double* __restrict__ KB, double* __restrict__ KC,
-                                double* __restrict__ colmean) {
-  const int j = blockIdx.x * blockDim.x + threadIdx.x;
-  if (j >= k) return;
-  const double ma = m[j], mb = m[k + j], mc = m[2 * k + j];
-  double sbc = 0.0, sac = 0.0, sab = 0.0, st = 0.0;
-  for (int x = 0; x < nb; ++x) {
-    const int64_t o = (int64_t)x * k + j;
-    const double a = A[o], b = B[o], c = C[o];
-    KA[o] = c3 * b * c + c1 * (b * mc + mb * c);
-    KB[o] = c3 * a * c + c1 * (a * mc + ma * c);
-    KC[o] = c3 * a * b + c1 * (a * mb + ma * b);
-    sbc += b * c;
-    sac += a * c;
-    sab += a * b;
-    st += c3 * a * b * c + c1 * (a * b * mc + a * mb * c + ma * b * c);
+// ---- FP64 MFMA tiles of the adjoint and the power method -----------------------------------------
+// A T x T block of the output (T = 32 or 64) per workgroup of four waves, each wave a (T/2) x (T/2)
+// quadrant of 16 x 16 v_mfma_f64_16x16x4f64 blocks (lane l supplies A[l % 16][l / 16] and
+// B[l / 16][l % 16]; accumulator register g of lane l holds D[4 g + l / 16][l % 16]). The reduction runs
+// in LDS stages of KS, the next stage's global loads in flight in registers during the MFMAs.
+// Row-major stages pad a row to KS + 4 doubles and k-major ones to T + 16, which spreads the 16 rows
+// (and the 4 k of a lane group) of a fragment read over all banks.
+template <int T>
+constexpr int stage_k() { return T == 32 ? 32 : 16; }
+
+__device__ inline doublex4 mma64(double a, double b, doublex4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
+
+template <int NP, int T>
+struct NnStage {
+  double a[NP][T][stage_k<T>() + 4];
+  double b[stage_k<T>()][T + 16];
+};
+
+template <int T>
+struct TnStage {
+  double a[stage_k<T>()][T + 16];
+  double b[stage_k<T>()][T + 16];
+};
+
+// acc[p] += X_p[row0 .. row0 + T, :] C[:, c0 .. c0 + T) for NP operands sharing C [kk x q] (row-major, leading
+// dimension q); rows from `rows` and columns from q on read as zero. With NM > 0 also msum[s] = the
+// calling thread's part of sum_i mu_s[i] C[i][c0 + threadIdx.x % T].
+template <int NP, int T, int NM, typename TX>
+__device__ inline void nn_tile(doublex4 (&acc)[NP][T / 32][T / 32], NnStage<NP, T>& S, const TX* const (&X)[NP], int64_t ldx,
+                               int64_t row0, int64_t rows, const double* __restrict__ C, int32_t kk, int32_t q, int32_t c0,
+                               const double* const* mu, double* msum) {
+  constexpr int KS = stage_k<T>(), E = T * KS / 256, U = T / 32;
+  const int t = threadIdx.x, l = t & 63, w = t >> 6;
+  const int ai = (T / 2) * (w >> 1), bj = (T / 2) * (w & 1);
+  const int xk = t % KS, xr = t / KS, cc = t % T, ck = T == 64 ? __builtin_amdgcn_readfirstlane(t >> 6) : t / T;
+  TX rx[NP][E];
+  double rc[E];
+  auto load = [&](int kb) {
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        const int64_t row = row0 + xr + (256 / KS) * e;
+        rx[p][e] = (kb + xk < kk && row < rows) ? X[p][row * ldx + kb + xk] : (TX)0;
+      }
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int k = kb + ck + (256 / T) * e;
+      const bool in = k < kk && c0 + cc < q;
+      rc[e] = in ? C[(int64_t)k * q + c0 + cc] : 0.0;
+      if constexpr (NM > 0) {
+#pragma unroll
+        for (int m = 0; m < NM; ++m) msum[m] = fma(k < kk ? mu[m][k] : 0.0, rc[e], msum[m]);
+      }
+    }
+  };
+  load(0);
+  for (int kb = 0; kb < kk; kb += KS) {
+    __syncthreads();
+#pragma unroll
+    for (int p = 0; p < NP; ++p)
+#pragma unroll
+      for (int e = 0; e < E; ++e) S.a[p][xr + (256 / KS) * e][xk] = (double)rx[p][e];
+#pragma unroll
+    for (int e = 0; e < E; ++e) S.b[ck + (256 / T) * e][cc] = rc[e];
+    __syncthreads();
+    if (kb + KS < kk) load(kb + KS);
+#pragma unroll
+    for (int k4 = 0; k4 < KS; k4 += 4) {
+      double b[U];
+#pragma unroll
+      for (int v = 0; v < U; ++v) b[v] = S.b[k4 + (l >> 4)][bj + 16 * v + (l & 15)];
+#pragma unroll
+      for (int p = 0; p < NP; ++p)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const double a = S.a[p][ai + 16 * u + (l & 15)][k4 + (l >> 4)];
+#pragma unroll
+          for (int v = 0; v < U; ++v) acc[p][u][v] = mma64(a, b[v], acc[p][u][v]);
+        }
+    }
   }
-  const double inv = 1.0 / (double)nb;
-  colmean[j] = sbc * inv;
-  colmean[k + j] = sac * inv;
-  colmean[2 * k + j] = sab * inv;
-  colmean[3 * k + j] = st * inv;
 }
 
-// grad = 3 theta PhiH - T; T gets + mu_X kappa_X^T; loss = theta/2 sum G^3 - sum_i (mean_i + c0 ma mb mc)
-__global__ __launch_bounds__(256) void adj_final_kernel(int32_t k, const double* __restrict__ m, const double* __restrict__ mus,
-                                                        const double* __restrict__ colmean, const double* __restrict__ G,
-                                                        const double* __restrict__ PhiH, const double* __restrict__ T,
+// acc += A[r0 .. r1, i0 .. i0 + T)^T B[r0 .. r1, j0 .. j0 + T); columns from p (A) and q (B) on read as zero.
+template <int T, typename TA>
+__device__ inline void tn_tile(doublex4 (&acc)[T / 32][T / 32], TnStage<T>& S, const TA* __restrict__ A, int64_t lda, int32_t p,
+                               int32_t i0, const double* __restrict__ B, int64_t ldb, int32_t q, int32_t j0, int64_t r0,
+                               int64_t r1) {
+  constexpr int KS = stage_k<T>(), E = T * KS / 256, U = T / 32;
+  const int t = threadIdx.x, l = t & 63, w = t >> 6;
+  const int ai = (T / 2) * (w >> 1), bj = (T / 2) * (w & 1);
+  const int cc = t % T, cx = t / T;
+  TA ra[E];
+  double rb[E];
+  auto load = [&](int64_t base) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      const int64_t x = base + cx + (256 / T) * e;
+      ra[e] = (x < r1 && i0 + cc < p) ? A[x * lda + i0 + cc] : (TA)0;
+      rb[e] = (x < r1 && j0 + cc < q) ? B[x * ldb + j0 + cc] : 0.0;
+    }
+  };
+  load(r0);
+  for (int64_t base = r0; base < r1; base += KS) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < E; ++e) {
+      S.a[cx + (256 / T) * e][cc] = (double)ra[e];
+      S.b[cx + (256 / T) * e][cc] = rb[e];
+    }
+    __syncthreads();
+    if (base + KS < r1) load(base + KS);
+#pragma unroll
+    for (int k4 = 0; k4 < KS; k4 += 4) {
+      double a[U], b[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        a[u] = S.a[k4 + (l >> 4)][ai + 16 * u + (l & 15)];
+        b[u] = S.b[k4 + (l >> 4)][bj + 16 * u + (l & 15)];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int v = 0; v < U; ++v) acc[u][v] = mma64(a[u], b[v], acc[u][v]);
+    }
+  }
+}
+
+// Visits the calling lane's elements of a T x T block: f(row, col, u, v, g) with row, col within the block.
+template <int T, typename F>
+__device__ inline void each_elem(F f) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int ai = (T / 2) * (w >> 1), bj = (T / 2) * (w & 1);
+#pragma unroll
+  for (int v = 0; v < T / 32; ++v)
+#pragma unroll
+    for (int u = 0; u < T / 32; ++u)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) f(ai + 16 * u + 4 * g + (l >> 4), bj + 16 * v + (l & 15), u, v, g);
+}
+
+// Column sums of a T x T block from each lane's partials s[v][0..NS) of its columns (bj + 16 v + l % 16):
+// the four lanes of a column, then the two waves that share it; out[i * q + c0 + col]. Fixed order.
+template <int T, int NS>
+__device__ inline void block_colsum(double (&s)[T / 32][NS], double (&red)[2][NS][T], double* __restrict__ out, int32_t q,
+                                    int32_t c0) {
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+  for (int v = 0; v < T / 32; ++v)
+#pragma unroll
+    for (int i = 0; i < NS; ++i) {
+      s[v][i] += __shfl_xor(s[v][i], 16);
+      s[v][i] += __shfl_xor(s[v][i], 32);
+      if (l < 16) red[w >> 1][i][(T / 2) * (w & 1) + 16 * v + l] = s[v][i];
+    }
+  __syncthreads();
+  for (int e = threadIdx.x; e < NS * T; e += 256) {
+    const int i = e / T, c = e % T;
+    if (c0 + c < q) out[(int64_t)i * q + c0 + c] = red[0][i][c] + red[1][i][c];
+  }
+}
+
+// m_s = Phi^T mu_s of the block's columns from the threads' parts (thread t holds column t % T).
+template <int T, int NM>
+__device__ inline void block_m(const double (&ms)[NM], double (&part)[NM][256], double (&m)[NM][T]) {
+#pragma unroll
+  for (int s = 0; s < NM; ++s) part[s][threadIdx.x] = ms[s];
+  __syncthreads();
+  for (int e = threadIdx.x; e < NM * T; e += 256) {
+    const int s = e / T, c = e % T;
+    double v = 0.0;
+    for (int r = 0; r < 256 / T; ++r) v += part[s][c + T * r];
+    m[s][c] = v;
+  }
+  __syncthreads();
+}
+
+// Adjoint, first launch. Workgroups [0, rt * ct): a T x T block of A = Y_A Phi, B = Y_B Phi, C = Y_C Phi (one
+// pass over Phi for the three), turned into K_A, K_B, K_C in registers, with the column sums of B o C,
+// A o C, A o B and of the loss terms over the block's rows (cpart [rt][4][k]) and m = Phi^T mu (by the first row
+// of blocks). The ct * ct workgroups after them: H = (Phi^T Phi)^o2 and the sum of (Phi^T Phi)^o3 per block
+// (gpart). Two workgroups per CU: the 64 x 64 form needs the cap at 256 registers for it (502 -> 395 us per call
+// at k = 500). The element-wise pass this replaces ran k threads over all nb rows (1.49 ms of 3.73 at k = 500,
+// nb = 4000; 0.35 of 0.83 ms at k = 100, nb = 1024), and the products one vector-ALU launch each.
+template <int T, typename TY>
+__global__ __launch_bounds__(256, 2) void adj_products_kernel(int32_t nb, int32_t k, int32_t rt, int32_t ct, const TY* __restrict__ ya,
+                                                           const TY* __restrict__ yb, const TY* __restrict__ yc, int32_t ldy,
+                                                           const double* __restrict__ mua, const double* __restrict__ mub,
+                                                           const double* __restrict__ muc, const double* __restrict__ phi,
+                                                           double c3, double c1, double* __restrict__ KA,
+                                                           double* __restrict__ KB, double* __restrict__ KC,
+                                                           double* __restrict__ cpart, double* __restrict__ m,
+                                                           double* __restrict__ H, double* __restrict__ gpart) {
+  constexpr int U = T / 32;
+  __shared__ union {
+    NnStage<3, T> nn;
+    TnStage<T> tn;
+    struct {
+      double part[3][256];
+      double m[3][T];
+      double red[2][4][T];
+    } e;
+    double red[256];
+  } sm;
+  const int64_t data = (int64_t)rt * ct;
+  if (blockIdx.x >= data) {
+    const int g = (int)(blockIdx.x - data), i0 = g / ct * T, j0 = g % ct * T;
+    doublex4 acc[U][U] = {};
+    tn_tile<T, double>(acc, sm.tn, phi, k, k, i0, phi, k, k, j0, 0, k);
+    double s = 0.0;
+    each_elem<T>([&](int r, int c, int u, int v, int gi) {
+      const double x = acc[u][v][gi];
+      s = fma(x * x, x, s);
+      if (i0 + r < k && j0 + c < k) H[(int64_t)(i0 + r) * k + j0 + c] = x * x;
+    });
+    __syncthreads();
+    sm.red[threadIdx.x] = s;
+    __syncthreads();
+    for (int off = 128; off > 0; off >>= 1) {
+      if ((int)threadIdx.x < off) sm.red[threadIdx.x] += sm.red[threadIdx.x + off];
+      __syncthreads();
+    }
+    if (threadIdx.x == 0) gpart[g] = sm.red[0];
+    return;
+  }
+  const int tr = (int)(blockIdx.x / ct), c0 = (int)(blockIdx.x % ct) * T;
+  const int64_t x0 = (int64_t)tr * T;
+  const TY* const Y[3] = {ya, yb, yc};
+  const double* const mu[3] = {mua, mub, muc};
+  doublex4 acc[3][U][U] = {};
+  double ms[3] = {0.0, 0.0, 0.0};
+  nn_tile<3, T, 3, TY>(acc, sm.nn, Y, ldy, x0, nb, phi, k, k, c0, mu, ms);
+  __syncthreads();
+  block_m<T, 3>(ms, sm.e.part, sm.e.m);
+  double s[U][4] = {};
+  each_elem<T>([&](int r, int c, int u, int v, int g) {
+    const double a = acc[0][u][v][g], b = acc[1][u][v][g], cc = acc[2][u][v][g];
+    const double ma = sm.e.m[0][c], mb = sm.e.m[1][c], mc = sm.e.m[2][c];
+    s[v][0] += b * cc;
+    s[v][1] += a * cc;
+    s[v][2] += a * b;
+    s[v][3] += c3 * a * b * cc + c1 * (a * b * mc + a * mb * cc + ma * b * cc);
+    if (x0 + r < nb && c0 + c < k) {
+      const int64_t o = (x0 + r) * k + c0 + c;
+      KA[o] = c3 * b * cc + c1 * (b * mc + mb * cc);
+      KB[o] = c3 * a * cc + c1 * (a * mc + ma * cc);
+      KC[o] = c3 * a * b + c1 * (a * mb + ma * b);
+    }
+  });
+  block_colsum<T, 4>(s, sm.e.red, cpart + (int64_t)tr * 4 * k, k, c0);
+  if (tr == 0)
+    for (int e = threadIdx.x; e < 3 * T; e += 256)
+      if (c0 + e % T < k) m[(int64_t)(e / T) * k + c0 + e % T] = sm.e.m[e / T][e % T];
+}
+
+// Sums the row blocks' partials of column j (one of ns * k): fixed order, eight loads in flight.
+__device__ inline double part_sum(const double* __restrict__ part, int64_t stride, int32_t n, int64_t j) {
+  double a[8] = {};
+  int32_t i = 0;
+  for (; i + 8 <= n; i += 8)
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a[u] += part[(int64_t)(i + u) * stride + j];
+  for (int u = 0; i < n; ++i, ++u) a[u] += part[(int64_t)i * stride + j];
+  return ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+}
+
+// Adjoint, second launch. Workgroups [0, S * ct * ct): block (i, j) of Y_A^T K_A + Y_B^T K_B + Y_C^T K_C over slice
+// s of the rows (tpart [S][k * k]); then ct * ct blocks of Phi H; the rest sum the column partials into
+// csum [4][k].
+template <int T, typename TY>
+__global__ __launch_bounds__(256) void adj_contract_kernel(int32_t nb, int32_t k, int32_t ct, int32_t S, int32_t rt,
+                                                           const TY* __restrict__ ya, const TY* __restrict__ yb,
+                                                           const TY* __restrict__ yc, int32_t ldy,
+                                                           const double* __restrict__ KA, const double* __restrict__ KB,
+                                                           const double* __restrict__ KC, double* __restrict__ tpart,
+                                                           const double* __restrict__ phi, const double* __restrict__ H,
+                                                           double* __restrict__ PhiH, const double* __restrict__ cpart,
+                                                           double* __restrict__ csum) {
+  constexpr int U = T / 32;
+  __shared__ union {
+    NnStage<1, T> nn;
+    TnStage<T> tn;
+  } sm;
+  const int nt = ct * ct;
+  const int blk = (int)blockIdx.x;
+  if (blk < (S + 1) * nt) {
+    const int tile = blk % nt, i0 = tile / ct * T, j0 = tile % ct * T;
+    doublex4 acc[1][U][U] = {};
+    double* out;
+    if (blk < S * nt) {
+      const int s = blk / nt;
+      const int64_t r0 = (int64_t)nb * s / S, r1 = (int64_t)nb * (s + 1) / S;
+      tn_tile<T, TY>(acc[0], sm.tn, ya, ldy, k, i0, KA, k, k, j0, r0, r1);
+      tn_tile<T, TY>(acc[0], sm.tn, yb, ldy, k, i0, KB, k, k, j0, r0, r1);
+      tn_tile<T, TY>(acc[0], sm.tn, yc, ldy, k, i0, KC, k, k, j0, r0, r1);
+      out = tpart + (int64_t)s * k * k;
+    } else {
+      const double* const X[1] = {phi};
+      nn_tile<1, T, 0, double>(acc, sm.nn, X, k, i0, k, H, k, k, j0, nullptr, nullptr);
+      out = PhiH;
+    }
+    each_elem<T>([&](int r, int c, int u, int v, int g) {
+      if (i0 + r < k && j0 + c < k) out[(int64_t)(i0 + r) * k + j0 + c] = acc[0][u][v][g];
+    });
+    return;
+  }
+  const int64_t j = (int64_t)(blk - (S + 1) * nt) * 256 + threadIdx.x;
+  if (j < 4 * (int64_t)k) csum[j] = part_sum(cpart, 4 * (int64_t)k, rt, j);
+}
+
+// Adjoint, third launch: grad = 3 theta PhiH - (sum_s tpart / nb + mu_X kappa_X^T), one element per thread; the last
+// workgroup forms loss = theta/2 sum G^3 - sum_j (mean_j + c0 m_A m_B m_C).
+__global__ __launch_bounds__(256) void adj_final_kernel(int32_t nb, int32_t k, int32_t S, int32_t ngpart,
+                                                        const double* __restrict__ m, const double* __restrict__ mua,
+                                                        const double* __restrict__ mub, const double* __restrict__ muc,
+                                                        const double* __restrict__ csum, const double* __restrict__ PhiH,
+                                                        const double* __restrict__ tpart, const double* __restrict__ gpart,
                                                         double c1, double c0, double theta, double* __restrict__ grad,
                                                         double* __restrict__ loss) {
-  __shared__ double red[256];
-  const int t = threadIdx.x;
   const int64_t kk = (int64_t)k * k;
-  for (int64_t e = t; e < kk; e += blockDim.x) {
+  const double inv = 1.0 / (double)nb;
+  if (blockIdx.x + 1 < gridDim.x) {
+    const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (e >= kk) return;
     const int i = (int)(e / k), j = (int)(e % k);   // row i (component), column j (eigenvector)
     const double ma = m[j], mb = m[k + j], mc = m[2 * k + j];
-    const double kA = c0 * mb * mc + c1 * colmean[j];
-    const double kB = c0 * ma * mc + c1 * colmean[k + j];
-    const double kC = c0 * ma * mb + c1 * colmean[2 * k + j];
-    const double tt = T[e] + mus[i] * kA + mus[k + i] * kB + mus[2 * k + i] * kC;
-    grad[e] = 3.0 * theta * PhiH[e] - tt;
+    const double kA = c0 * mb * mc + c1 * (csum[j] * inv);
+    const double kB = c0 * ma * mc + c1 * (csum[k + j] * inv);
+    const double kC = c0 * ma * mb + c1 * (csum[2 * k + j] * inv);
+    const double t = part_sum(tpart, kk, S, e) * inv + mua[i] * kA + mub[i] * kB + muc[i] * kC;
+    grad[e] = 3.0 * theta * PhiH[e] - t;
+    return;
   }
+  __shared__ double red[256];
+  const int t = threadIdx.x;
   double acc = 0.0;
-  for (int64_t e = t; e < kk; e += blockDim.x) {
-    const double g = G[e];
-    acc += 0.5 * theta * g * g * g;
-  }
-  for (int j = t; j < k; j += blockDim.x) acc -= colmean[3 * k + j] + c0 * m[j] * m[k + j] * m[2 * k + j];
+  for (int g = t; g < ngpart; g += 256) acc += 0.5 * theta * gpart[g];
+  for (int j = t; j < k; j += 256) acc -= csum[3 * k + j] * inv + c0 * m[j] * m[k + j] * m[2 * k + j];
   red[t] = acc;
   __syncthreads();
-  for (int off = blockDim.x / 2; off > 0; off >>= 1) {
+  for (int off = 128; off > 0; off >>= 1) {
     if (t < off) red[t] += red[t + off];
     __syncthreads();
   }
   if (t == 0) loss[0] = red[0];
-}
-
-__global__ void square_kernel(int64_t n, const double* __restrict__ in, double* __restrict__ out) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) out[t] = in[t] * in[t];
-}
-
-__global__ void pack_mu_kernel(int32_t k, const double* __restrict__ a, const double* __restrict__ b, const double* __restrict__ c,
-                               double* __restrict__ out) {
-  const int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < k) {
-    out[t] = a[t];
-    out[k + t] = b[t];
-    out[2 * k + t] = c[t];
-  }
 }
 
 // Power-method pieces: K_A = c3 B o C + c1 (B o m_C + m_B o C) for a chunk of rows, and the column
@@ -207,11 +480,52 @@ int power_iteration(hipStream_t s, int32_t k, int64_t n, const PowerRows& rows, 
   return MMSB_OK;
 }
 
+// The published workspace size (mmsb_stgd_grad_workspace): callers hold buffers of this size and the fixed
+// scratch of the allocation-free form bounds (k, nb) by it, so it is a formula of its own: 6 b x k and
+// 4 k x k matrices, 12 k-vectors, and the row-slice partials of a k x k product.
+static int64_t grad_slices(int64_t n, int32_t k) {  // slices of a b-row product in that formula
+  const int64_t t64 = ceil_div(k, 64) * ceil_div(k, 64);
+  const int64_t s = std::min<int64_t>(ceil_div(2048, t64), std::max<int64_t>(1, n / 256));
+  int64_t most = std::max<int64_t>(1, std::min<int64_t>(s, 512));
+  if (k == 1 && n >= 65536) most = std::max(most, std::min<int64_t>(1024, n / 256));
+  if (n >= 4096 && k >= 32) {
+    const int64_t tp = ceil_div(k, 128), cap = std::max<int64_t>(1, (256ll << 20) / ((int64_t)k * k * 8));
+    for (int64_t tiles : {tp * tp, tp * (tp + 1) / 2})
+      most = std::max(most, std::max<int64_t>(1, std::min(std::min(std::max<int64_t>(1, 1024 / tiles), cap),
+                                                          std::max<int64_t>(1, n / 1024))));
+  }
+  return most;
+}
+
 size_t grad_workspace_bytes(int32_t k, int32_t nb) {
   const size_t bk = sizeof(double) * (size_t)nb * k, kk = sizeof(double) * (size_t)k * k;
-  size_t tn = std::max(tn_workspace_bytes(nb, k, k), tn_workspace_bytes(k, k, k));
-  tn = std::max(tn, tn_workspace_bytes(k, k, 1));
+  size_t tn = (size_t)std::max(grad_slices(nb, k), grad_slices(k, k)) * kk;
   return 6 * align256(bk) + 4 * align256(kk) + 3 * align256(sizeof(double) * 4 * k) + align256(tn);
+}
+
+// Launch shape of the adjoint, a function of (k, nb) alone so that every entry point sums in the same order.
+// 64 x 64 blocks read each operand half as often as 32 x 32 ones but leave CUs idle on small problems: they are
+// taken for the products once they make 192 workgroups, and for the contraction above k = 256 (below it the
+// k x k output has at most 16 of them): k = 500, nb = 4000 takes 387 us with 64 x 64 products, 431 with 32 x 32.
+// The contraction's rows are cut into S slices of at least 64 rows, about 512 workgroups in all. A whole call
+// (three launches instead of 22): k = 100, nb = 1024 in FP32 828 -> 49 us, of which 28 in kernels; k = 500,
+// nb = 4000 in FP64 3.73 -> 0.39 ms, 32 TFLOP/s of FP64 MFMA.
+struct AdjShape {
+  int t1, rt, ct1, t2, ct2, S;
+};
+
+static AdjShape adj_shape(int32_t k, int32_t nb) {
+  AdjShape a;
+  a.t1 = ceil_div(nb, 64) * ceil_div(k, 64) >= 192 ? 64 : 32;
+  a.rt = (int)ceil_div(nb, a.t1);
+  a.ct1 = (int)ceil_div(k, a.t1);
+  a.t2 = k > 256 ? 64 : 32;
+  a.ct2 = (int)ceil_div(k, a.t2);
+  // the partials lie in what the published size leaves: three b x k matrices less the column partials (at most
+  // b k / 8 + 4 k values), and one k x k matrix
+  const int64_t room = 1 + (3 * (int64_t)nb * k - (int64_t)a.rt * 4 * k) / ((int64_t)k * k);
+  a.S = (int)std::max<int64_t>(1, std::min(std::min<int64_t>(ceil_div(512, a.ct2 * a.ct2), ceil_div(nb, 64)), room));
+  return a;
 }
 
 template <typename TY>
@@ -220,36 +534,33 @@ int stgd_grad(hipStream_t s, int32_t k, int32_t nb, const TY* ya, const TY* yb, 
               double theta, double* grad, double* loss, void* work) {
   MMSB_CHECK_ARG(k >= 1 && nb >= 1 && ldy >= k, "grad: bad shape k=%d nb=%d ldy=%d", k, nb, ldy);
   MMSB_CHECK_ARG(ya && yb && yc && mua && mub && muc && phi && grad && loss && work, "grad: null pointer");
+  const AdjShape a = adj_shape(k, nb);
   unsigned char* w = static_cast<unsigned char*>(work);
-  auto take = [&](size_t bytes) { double* p = reinterpret_cast<double*>(w); w += align256(bytes); return p; };
-  const size_t bk = sizeof(double) * (size_t)nb * k, kk = sizeof(double) * (size_t)k * k;
-  double *A = take(bk), *B = take(bk), *C = take(bk), *KA = take(bk), *KB = take(bk), *KC = take(bk);
-  double *G = take(kk), *H = take(kk), *PhiH = take(kk), *T = take(kk);
-  double *m = take(sizeof(double) * 4 * k), *mus = take(sizeof(double) * 4 * k), *colmean = take(sizeof(double) * 4 * k);
-  double* tn = reinterpret_cast<double*>(w);
-  // A = Y_A Phi etc. (b x k), m = Phi^T mu
-  MMSB_TRY((gemm_nn<TY, double>(s, nb, k, k, 1.0, ya, ldy, phi, k, 0.0, A, k)));
-  MMSB_TRY((gemm_nn<TY, double>(s, nb, k, k, 1.0, yb, ldy, phi, k, 0.0, B, k)));
-  MMSB_TRY((gemm_nn<TY, double>(s, nb, k, k, 1.0, yc, ldy, phi, k, 0.0, C, k)));
-  MMSB_TRY((gemm_tn<double, double>(s, k, k, 1, 1.0, phi, k, mua, 1, 0.0, m, tn)));
-  MMSB_TRY((gemm_tn<double, double>(s, k, k, 1, 1.0, phi, k, mub, 1, 0.0, m + k, tn)));
-  MMSB_TRY((gemm_tn<double, double>(s, k, k, 1, 1.0, phi, k, muc, 1, 0.0, m + 2 * k, tn)));
-  hipLaunchKernelGGL(pack_mu_kernel, dim3((unsigned)ceil_div(k, 256)), dim3(256), 0, s, k, mua, mub, muc, mus);
+  auto take = [&](int64_t n) { double* p = reinterpret_cast<double*>(w); w += align256(sizeof(double) * (size_t)n); return p; };
+  const int64_t bk = (int64_t)nb * k, kk = (int64_t)k * k;
+  double *KA = take(bk), *KB = take(bk), *KC = take(bk);
+  double *H = take(kk), *PhiH = take(kk);
+  double *m = take(3 * (int64_t)k), *csum = take(4 * (int64_t)k), *gpart = take((int64_t)a.ct1 * a.ct1);
+  double *cpart = take((int64_t)a.rt * 4 * k), *tpart = take(a.S * kk);
+  MMSB_CHECK_ARG((size_t)(w - static_cast<unsigned char*>(work)) <= grad_workspace_bytes(k, nb), "grad: workspace layout");
+  const dim3 g1((unsigned)((int64_t)a.rt * a.ct1 + (int64_t)a.ct1 * a.ct1));
+  if (a.t1 == 64)
+    hipLaunchKernelGGL((adj_products_kernel<64, TY>), g1, dim3(256), 0, s, nb, k, a.rt, a.ct1, ya, yb, yc, ldy, mua, mub, muc, phi,
+                       c3, c1, KA, KB, KC, cpart, m, H, gpart);
+  else
+    hipLaunchKernelGGL((adj_products_kernel<32, TY>), g1, dim3(256), 0, s, nb, k, a.rt, a.ct1, ya, yb, yc, ldy, mua, mub, muc, phi,
+                       c3, c1, KA, KB, KC, cpart, m, H, gpart);
   MMSB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(adj_elem_kernel, dim3((unsigned)ceil_div(k, 64)), dim3(64), 0, s, nb, k, A, B, C, m, c3, c1, KA, KB, KC,
-                     colmean);
+  const dim3 g2((unsigned)((int64_t)(a.S + 1) * a.ct2 * a.ct2 + ceil_div(4 * (int64_t)k, 256)));
+  if (a.t2 == 64)
+    hipLaunchKernelGGL((adj_contract_kernel<64, TY>), g2, dim3(256), 0, s, nb, k, a.ct2, a.S, a.rt, ya, yb, yc, ldy, KA, KB, KC,
+                       tpart, phi, H, PhiH, cpart, csum);
+  else
+    hipLaunchKernelGGL((adj_contract_kernel<32, TY>), g2, dim3(256), 0, s, nb, k, a.ct2, a.S, a.rt, ya, yb, yc, ldy, KA, KB, KC,
+                       tpart, phi, H, PhiH, cpart, csum);
   MMSB_LAUNCH_CHECK();
-  // T = (Y_A^T K_A + Y_B^T K_B + Y_C^T K_C) / b
-  const double inv = 1.0 / (double)nb;
-  MMSB_TRY((gemm_tn<TY, double>(s, nb, k, k, inv, ya, ldy, KA, k, 0.0, T, tn)));
-  MMSB_TRY((gemm_tn<TY, double>(s, nb, k, k, inv, yb, ldy, KB, k, 1.0, T, tn)));
-  MMSB_TRY((gemm_tn<TY, double>(s, nb, k, k, inv, yc, ldy, KC, k, 1.0, T, tn)));
-  // G = Phi^T Phi, H = G o G, PhiH
-  MMSB_TRY((gemm_tn<double, double>(s, k, k, k, 1.0, phi, k, phi, k, 0.0, G, tn)));
-  hipLaunchKernelGGL(square_kernel, dim3((unsigned)ceil_div((int64_t)k * k, 256)), dim3(256), 0, s, (int64_t)k * k, G, H);
-  MMSB_LAUNCH_CHECK();
-  MMSB_TRY((gemm_nn<double, double>(s, k, k, k, 1.0, phi, k, H, k, 0.0, PhiH, k)));
-  hipLaunchKernelGGL(adj_final_kernel, dim3(1), dim3(256), 0, s, k, m, mus, colmean, G, PhiH, T, c1, c0, theta, grad, loss);
+  hipLaunchKernelGGL(adj_final_kernel, dim3((unsigned)(ceil_div(kk, 256) + 1)), dim3(256), 0, s, nb, k, a.S, a.ct1 * a.ct1, m, mua,
+                     mub, muc, csum, PhiH, tpart, gpart, c1, c0, theta, grad, loss);
   MMSB_LAUNCH_CHECK();
   return MMSB_OK;
 }
