@@ -95,7 +95,7 @@ int stgd_grad(hipStream_t s, int32_t k, int32_t nb, const TY* ya, const TY* yb, 
               const double* mua, const double* mub, const double* muc, const double* phi, double c3, double c1, double c0,
               double theta, double* grad, double* loss, void* work);
 
-size_t power_workspace_bytes(int32_t k, int32_t chunk);
+size_t power_workspace_bytes(int32_t k, int64_t n, int32_t chunk);
 // rows(r0, nb, &ya, &yb, &yc) enqueues whatever makes rows [r0, r0 + nb) of Y_A, Y_B, Y_C available
 // row-major with leading dimension ldy, and points ya, yb, yc at them (valid until the next call).
 using PowerRows = std::function<int(int64_t r0, int32_t nb, const float** ya, const float** yb, const float** yc)>;

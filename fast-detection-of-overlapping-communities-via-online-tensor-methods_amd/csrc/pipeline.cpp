@@ -1766,7 +1766,7 @@ extern "C" int mmsb_power_method(mmsb_ctx* c, int32_t iters, int32_t orthogonali
   if (e == hipSuccess) e = hipMalloc(&dlam, sizeof(double) * k);
   for (int i = 0; i < (c->have_y ? 1 : 3); ++i)
     if (e == hipSuccess) e = hipMalloc(&yr[i], sizeof(float) * (size_t)chunk * kp);
-  if (e == hipSuccess) e = hipMalloc(&work, power_workspace_bytes(k, chunk));
+  if (e == hipSuccess) e = hipMalloc(&work, power_workspace_bytes(k, c->n[0], chunk));
   if (e == hipSuccess) e = hipMemcpyAsync(dphi, hd.data(), sizeof(double) * k * k, hipMemcpyHostToDevice, c->s);
   if (e != hipSuccess) {
     cleanup();
