@@ -15,6 +15,7 @@
 #include "common.h"
 
 #include "dense.h"
+#include "mfma64.h"
 #include "philox.h"
 
 namespace mmsb {
@@ -66,9 +67,11 @@ int csr_rowsum(hipStream_t s, int32_t m, const int32_t* rowptr, const float* val
 }
 
 // ---- C[p x q] (FP64) = alpha * A^T B, A [n x p], B [n x q] row-major ------------------------
-// Grid: (tiles of C 64 x 64) x S row slices. Each workgroup stages 16-row slabs of A and B through
-// LDS as FP64 and accumulates a 4 x 4 register tile per thread; the S partial tiles are written to
-// a workspace and reduced in a fixed order by a second kernel (deterministic result).
+// The rows are cut into slices; each slice's partial tile of C goes to a workspace and a second kernel sums the
+// slices in order (deterministic result). The slice count is a function of the shape alone and every form below
+// adds the rows of a slice one after another (the MFMA forms four after four), so the form chosen for a call --
+// by how many workgroups its tiles make -- does not change a bit of C.
+// General form: 64 x 64 tiles, 16-row slabs of A and B through LDS as FP64, a 4 x 4 register tile per thread.
 template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void tn_partial_kernel(int64_t n, int32_t p, int32_t q, const TA* __restrict__ A,
                                                          int32_t lda, const TB* __restrict__ B, int32_t ldb,
@@ -114,13 +117,104 @@ __global__ __launch_bounds__(256) void tn_partial_kernel(int64_t n, int32_t p, i
     }
 }
 
-__global__ void tn_reduce_kernel(int64_t pq, int32_t slices, const double* __restrict__ work, double alpha,
-                                 double beta, double* __restrict__ C) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= pq) return;
+// The same with 16 x 16 tiles, one element per thread and 64-row slabs, the next slab's loads in flight: for
+// outputs whose 64 x 64 tiles leave the chip idle.
+template <typename TA, typename TB>
+__global__ __launch_bounds__(256) void tn_small_kernel(int64_t n, int32_t p, int32_t q, const TA* __restrict__ A, int32_t lda,
+                                                       const TB* __restrict__ B, int32_t ldb, int32_t slices,
+                                                       double* __restrict__ work) {
+  constexpr int R = 64;
+  __shared__ double As[R][16];
+  __shared__ double Bs[R][16];
+  const int tp = blockIdx.x * 16, tq = blockIdx.y * 16;
+  const int64_t r0 = n * blockIdx.z / slices, r1 = n * (blockIdx.z + 1) / slices;
+  const int c = threadIdx.x & 15, g = threadIdx.x >> 4;
+  TA ra[4];
+  TB rb[4];
+  auto load = [&](int64_t base) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t row = base + g + 16 * e;
+      ra[e] = (row < r1 && tp + c < p) ? A[row * lda + tp + c] : (TA)0;
+      rb[e] = (row < r1 && tq + c < q) ? B[row * ldb + tq + c] : (TB)0;
+    }
+  };
   double acc = 0.0;
-  for (int s = 0; s < slices; ++s) acc += work[(int64_t)s * pq + t];
+  load(r0);
+  for (int64_t base = r0; base < r1; base += R) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      As[g + 16 * e][c] = (double)ra[e];
+      Bs[g + 16 * e][c] = (double)rb[e];
+    }
+    __syncthreads();
+    if (base + R < r1) load(base + R);
+#pragma unroll 16
+    for (int rr = 0; rr < R; ++rr) acc = fma(As[rr][g], Bs[rr][c], acc);
+  }
+  if (tp + g < p && tq + c < q) work[(int64_t)blockIdx.z * p * q + (int64_t)(tp + g) * q + tq + c] = acc;
+}
+
+// The same for p = 1 or q = 1 (v the column operand, M the other): one thread per column of M walks the slice's
+// rows, sixteen rows of loads in flight. (In 64 x 64 tiles 63 of 64 columns of the slab would be padding.)
+template <typename TM, typename TV>
+__global__ __launch_bounds__(64) void tn_thin_kernel(int64_t n, int32_t m, const TM* __restrict__ M, int32_t ldm,
+                                                     const TV* __restrict__ v, int32_t incv, int32_t slices,
+                                                     double* __restrict__ work) {
+  const int32_t j = blockIdx.x * 64 + threadIdx.x;
+  const int64_t r0 = n * blockIdx.y / slices, r1 = n * (blockIdx.y + 1) / slices;
+  if (j >= m) return;
+  double acc = 0.0;
+  int64_t i = r0;
+  for (; i + 16 <= r1; i += 16) {
+    TV x[16];
+    TM y[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+      x[u] = v[(i + u) * incv];
+      y[u] = M[(i + u) * ldm + j];
+    }
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc = fma((double)x[u], (double)y[u], acc);
+  }
+  for (; i < r1; ++i) acc = fma((double)v[i * incv], (double)M[i * ldm + j], acc);
+  work[(int64_t)blockIdx.y * m + j] = acc;
+}
+
+// C = alpha * sum_s work[s] + beta * C, the slices added in order, sixteen loads in flight per thread; with sym = T the
+// entries of the T x T tiles below the diagonal come from the mirror (sym = 0: none). Bound by the latency of
+// that chain: 64 threads per workgroup spread a small C over the CUs.
+__global__ __launch_bounds__(64) void tn_reduce_kernel(int32_t p, int32_t q, int32_t slices, int32_t sym,
+                                                       const double* __restrict__ work, double alpha, double beta,
+                                                       double* __restrict__ C) {
+  const int64_t pq = (int64_t)p * q;
+  const int64_t t = (int64_t)blockIdx.x * 64 + threadIdx.x;
+  if (t >= pq) return;
+  int64_t src = t;
+  if (sym) {
+    const int i = (int)(t / q), j = (int)(t % q);
+    if (i / sym > j / sym) src = (int64_t)j * q + i;
+  }
+  double acc = 0.0;
+  int s = 0;
+  for (; s + 16 <= slices; s += 16) {
+    double x[16];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) x[u] = work[(int64_t)(s + u) * pq + src];
+#pragma unroll
+    for (int u = 0; u < 16; ++u) acc += x[u];
+  }
+  for (; s < slices; ++s) acc += work[(int64_t)s * pq + src];
   C[t] = (beta == 0.0) ? alpha * acc : alpha * acc + beta * C[t];
+}
+
+static int tn_reduce(hipStream_t s, int32_t p, int32_t q, int32_t slices, int32_t sym, const double* work, double alpha,
+                     double beta, double* C) {
+  hipLaunchKernelGGL(tn_reduce_kernel, dim3((unsigned)ceil_div((int64_t)p * q, 64)), dim3(64), 0, s, p, q, slices, sym, work,
+                     alpha, beta, C);
+  MMSB_LAUNCH_CHECK();
+  return MMSB_OK;
 }
 
 // ---- the vector shapes over many rows: C[1 x m] = v^T M (p = 1) or C[m x 1] = M^T v (q = 1) ----------
@@ -295,60 +389,95 @@ __global__ __launch_bounds__(256) void tn_mfma_kernel(int64_t n, int32_t p, int3
       }
 }
 
-// C = alpha * sum_s work[s] + beta * C; SYM: entries below the diagonal tiles come from the mirror.
-__global__ void tn_mfma_reduce_kernel(int32_t p, int32_t q, int32_t slices, bool sym, const double* __restrict__ work,
-                                      double alpha, double beta, double* __restrict__ C) {
-  const int64_t pq = (int64_t)p * q;
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= pq) return;
-  const int i = (int)(t / q), j = (int)(t % q);
-  const int64_t src = (sym && i / kMT > j / kMT) ? (int64_t)j * q + i : t;
-  double acc = 0.0;
-  for (int s = 0; s < slices; ++s) acc += work[(int64_t)s * pq + src];
-  C[t] = (beta == 0.0) ? alpha * acc : alpha * acc + beta * C[t];
+// The same partials in T x T tiles (T = 64 or 32), for outputs whose 128 x 128 tiles leave CUs idle.
+template <int T, typename TA, typename TB, bool SYM>
+__global__ __launch_bounds__(256) void tn_tile_kernel(int64_t n, int32_t p, int32_t q, const TA* __restrict__ A, int32_t lda,
+                                                      const TB* __restrict__ B, int32_t ldb, int32_t slices,
+                                                      double* __restrict__ work) {
+  __shared__ TnStage<T> sm;
+  int ti, tj;
+  if constexpr (SYM) {
+    const int tp = (p + T - 1) / T;
+    int rem = blockIdx.x;
+    ti = 0;
+    while (rem >= tp - ti) {
+      rem -= tp - ti;
+      ++ti;
+    }
+    tj = ti + rem;
+  } else {
+    const int tq = (q + T - 1) / T;
+    ti = blockIdx.x / tq;
+    tj = blockIdx.x % tq;
+  }
+  const int i0 = ti * T, j0 = tj * T;
+  doublex4 acc[T / 32][T / 32] = {};
+  tn_tile<T, TA, TB>(acc, sm, A, lda, p, i0, B, ldb, q, j0, n * blockIdx.y / slices, n * (blockIdx.y + 1) / slices);
+  double* wp = work + (int64_t)blockIdx.y * p * q;
+  each_elem<T>([&](int r, int c, int u, int v, int g) {
+    if (i0 + r < p && j0 + c < q) wp[(int64_t)(i0 + r) * q + j0 + c] = acc[u][v][g];
+  });
+}
+
+// Tile edge of an MFMA product: the widest of 128, 64, 32 whose tiles x slices make at least 384 workgroups (one and a
+// half per CU), else 32. A 110 x 110 Gram of 50k rows has one 128 tile and 48 slices: 332 us as 48 workgroups, 39 us in
+// 32 x 32 tiles (480 workgroups); the whole whitening of that size 20.1 -> 14.7 ms with the forms above.
+static int tn_tile_edge(int32_t p, int32_t q, bool sym, int slices) {
+  for (int t : {128, 64}) {
+    const int64_t tp = ceil_div(p, t), tq = ceil_div(q, t);
+    if ((sym ? tp * (tp + 1) / 2 : tp * tq) * slices >= 384) return t;
+  }
+  return 32;
 }
 
 template <typename TA, typename TB>
 int gemm_tn(hipStream_t s, int64_t n, int32_t p, int32_t q, double alpha, const TA* A, int32_t lda, const TB* B,
             int32_t ldb, double beta, double* C, double* work) {
   MMSB_CHECK_ARG(n >= 0 && p >= 1 && q >= 1 && lda >= p && ldb >= q, "gemm_tn: bad shape");
-  const int64_t pq = (int64_t)p * q;
-  if ((p == 1 || q == 1) && n >= kVecMinRows) {
+  if (p == 1 || q == 1) {
     const int32_t m = p == 1 ? q : p;
-    const int slices = tn_vec_slices(n, m);
-    const dim3 grid((unsigned)ceil_div(m, 256), (unsigned)slices);
-    if (p == 1)  // C = A^T B with A a column: v = A, M = B
-      hipLaunchKernelGGL((tn_vec_kernel<TB, TA>), grid, dim3(256), 0, s, n, m, B, ldb, A, lda, slices, work);
-    else         // q == 1: v = B, M = A
-      hipLaunchKernelGGL((tn_vec_kernel<TA, TB>), grid, dim3(256), 0, s, n, m, A, lda, B, ldb, slices, work);
+    const bool many = n >= kVecMinRows;
+    const int slices = many ? tn_vec_slices(n, m) : tn_slices(n, p, q);
+    const dim3 grid((unsigned)ceil_div(m, many ? 256 : 64), (unsigned)slices), block(many ? 256 : 64);
+    if (p == 1) {  // C = A^T B with A a column: v = A, M = B
+      if (many) hipLaunchKernelGGL((tn_vec_kernel<TB, TA>), grid, block, 0, s, n, m, B, ldb, A, lda, slices, work);
+      else hipLaunchKernelGGL((tn_thin_kernel<TB, TA>), grid, block, 0, s, n, m, B, ldb, A, lda, slices, work);
+    } else {       // q == 1: v = B, M = A
+      if (many) hipLaunchKernelGGL((tn_vec_kernel<TA, TB>), grid, block, 0, s, n, m, A, lda, B, ldb, slices, work);
+      else hipLaunchKernelGGL((tn_thin_kernel<TA, TB>), grid, block, 0, s, n, m, A, lda, B, ldb, slices, work);
+    }
     MMSB_LAUNCH_CHECK();
-    hipLaunchKernelGGL(tn_reduce_kernel, dim3((unsigned)ceil_div(m, 256)), dim3(256), 0, s, (int64_t)m, slices, work,
-                       alpha, beta, C);
-    MMSB_LAUNCH_CHECK();
-    return MMSB_OK;
+    return tn_reduce(s, 1, m, slices, 0, work, alpha, beta, C);
   }
   if (use_mfma(n, p, q)) {
     const bool sym = std::is_same<TA, TB>::value && (const void*)A == (const void*)B && lda == ldb && p == q;
-    const int slices = tn_mfma_slices(n, p, q, sym);
-    dim3 grid((unsigned)tn_mfma_tiles(p, q, sym), (unsigned)slices);
-    if (sym)
-      hipLaunchKernelGGL((tn_mfma_kernel<TA, TB, true>), grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
-    else
-      hipLaunchKernelGGL((tn_mfma_kernel<TA, TB, false>), grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+    const int slices = tn_mfma_slices(n, p, q, sym), t = tn_tile_edge(p, q, sym, slices);
+    const int64_t tp = ceil_div(p, t), tq = ceil_div(q, t);
+    const dim3 grid((unsigned)(sym ? tp * (tp + 1) / 2 : tp * tq), (unsigned)slices);
+#define MMSB_TN(KERNEL) hipLaunchKernelGGL(KERNEL, grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work)
+    if (sym) {
+      if (t == 128) MMSB_TN((tn_mfma_kernel<TA, TB, true>));
+      else if (t == 64) MMSB_TN((tn_tile_kernel<64, TA, TB, true>));
+      else MMSB_TN((tn_tile_kernel<32, TA, TB, true>));
+    } else {
+      if (t == 128) MMSB_TN((tn_mfma_kernel<TA, TB, false>));
+      else if (t == 64) MMSB_TN((tn_tile_kernel<64, TA, TB, false>));
+      else MMSB_TN((tn_tile_kernel<32, TA, TB, false>));
+    }
+#undef MMSB_TN
     MMSB_LAUNCH_CHECK();
-    hipLaunchKernelGGL(tn_mfma_reduce_kernel, dim3((unsigned)ceil_div(pq, 256)), dim3(256), 0, s, p, q, slices, sym, work,
-                       alpha, beta, C);
-    MMSB_LAUNCH_CHECK();
-    return MMSB_OK;
+    return tn_reduce(s, p, q, slices, sym ? t : 0, work, alpha, beta, C);
   }
   const int slices = tn_slices(n, p, q);
-  dim3 grid((unsigned)ceil_div(p, 64), (unsigned)ceil_div(q, 64), (unsigned)slices);
-  hipLaunchKernelGGL((tn_partial_kernel<TA, TB>), grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+  if (ceil_div(p, 64) * ceil_div(q, 64) * slices < 256) {
+    dim3 grid((unsigned)ceil_div(p, 16), (unsigned)ceil_div(q, 16), (unsigned)slices);
+    hipLaunchKernelGGL((tn_small_kernel<TA, TB>), grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+  } else {
+    dim3 grid((unsigned)ceil_div(p, 64), (unsigned)ceil_div(q, 64), (unsigned)slices);
+    hipLaunchKernelGGL((tn_partial_kernel<TA, TB>), grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+  }
   MMSB_LAUNCH_CHECK();
-  hipLaunchKernelGGL(tn_reduce_kernel, dim3((unsigned)ceil_div(pq, 256)), dim3(256), 0, s, pq, slices, work, alpha,
-                     beta, C);
-  MMSB_LAUNCH_CHECK();
-  return MMSB_OK;
+  return tn_reduce(s, p, q, slices, 0, work, alpha, beta, C);
 }
 
 template int gemm_tn<float, float>(hipStream_t, int64_t, int32_t, int32_t, double, const float*, int32_t, const float*,
@@ -622,7 +751,7 @@ int gemm_nn_f32(hipStream_t s, int64_t n, int32_t p, int32_t q, double alpha, co
 // C [p x q] (FP64) = alpha A^T B + beta C with A [n x p], B [n x q] FP32: the rows are cut into the
 // slices of tn_mfma_slices; each workgroup sums its slice of one 128 x 128 tile on
 // v_mfma_f32_32x32x2f32 (FP32 sums over at most n / slices rows), the partials are written as FP64
-// and reduced in FP64 by tn_mfma_reduce_kernel. For products whose relative accuracy need not beat
+// and reduced in FP64 by tn_reduce_kernel. For products whose relative accuracy need not beat
 // ~sqrt(n / slices) eps_32 (the operator applications of the randomized range finder).
 __global__ __launch_bounds__(256, 2) void tn_f32mfma_kernel(int64_t n, int32_t p, int32_t q, const float* __restrict__ A,
                                                            int32_t lda, const float* __restrict__ B, int32_t ldb,
@@ -691,18 +820,66 @@ __global__ __launch_bounds__(256, 2) void tn_f32mfma_kernel(int64_t n, int32_t p
       }
 }
 
+// The same partials in 64 x 64 tiles (each wave one 32 x 32 block, 32-deep stages): the widths of mid-size problems
+// make one 128 tile, i.e. one workgroup per slice.
+__global__ __launch_bounds__(256) void tn_f32mfma64_kernel(int64_t n, int32_t p, int32_t q, const float* __restrict__ A,
+                                                           int32_t lda, const float* __restrict__ B, int32_t ldb,
+                                                           int32_t slices, double* __restrict__ work) {
+  constexpr int T = 64, KS = 32;
+  __shared__ float As[KS][T + 4];
+  __shared__ float Bs[KS][T + 4];
+  const int tq = (q + T - 1) / T;
+  const int i0 = (int)blockIdx.x / tq * T, j0 = (int)blockIdx.x % tq * T;
+  const int64_t r0 = n * blockIdx.y / slices, r1 = n * (blockIdx.y + 1) / slices;
+  const int t = threadIdx.x, w = t >> 6, l = t & 63;
+  const int ai = 32 * (w >> 1), bj = 32 * (w & 1);
+  float ra[8], rb[8];
+  auto load = [&](int64_t base) {  // wave w stages rows w + 4 e
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int64_t row = base + w + 4 * e;
+      ra[e] = (row < r1 && i0 + l < p) ? A[row * lda + i0 + l] : 0.f;
+      rb[e] = (row < r1 && j0 + l < q) ? B[row * ldb + j0 + l] : 0.f;
+    }
+  };
+  floatx16 acc = {};
+  load(r0);
+  for (int64_t base = r0; base < r1; base += KS) {
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      As[w + 4 * e][l] = ra[e];
+      Bs[w + 4 * e][l] = rb[e];
+    }
+    __syncthreads();
+    if (base + KS < r1) load(base + KS);
+#pragma unroll
+    for (int kk = 0; kk < KS; kk += 2) {
+      const int kl = kk + (l >> 5);
+      acc = __builtin_amdgcn_mfma_f32_32x32x2f32(As[kl][ai + (l & 31)], Bs[kl][bj + (l & 31)], acc, 0, 0, 0);
+    }
+  }
+  double* wp = work + (int64_t)blockIdx.y * p * q;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int ri = i0 + ai + 8 * (i >> 2) + 4 * (l >> 5) + (i & 3), cj = j0 + bj + (l & 31);
+    if (ri < p && cj < q) wp[(int64_t)ri * q + cj] = (double)acc[i];
+  }
+}
+
 int gemm_tn_f32(hipStream_t s, int64_t n, int32_t p, int32_t q, double alpha, const float* A, int32_t lda, const float* B,
                 int32_t ldb, double beta, double* C, double* work) {
   MMSB_CHECK_ARG(n >= 0 && p >= 1 && q >= 1 && lda >= p && ldb >= q, "gemm_tn_f32: bad shape");
   const int slices = tn_mfma_slices(n, p, q, false);
-  const dim3 grid((unsigned)(ceil_div(p, kFT) * ceil_div(q, kFT)), (unsigned)slices);
-  hipLaunchKernelGGL(tn_f32mfma_kernel, grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+  const bool wide = tn_tile_edge(p, q, false, slices) == 128;
+  const int t = wide ? kFT : 64;
+  const dim3 grid((unsigned)(ceil_div(p, t) * ceil_div(q, t)), (unsigned)slices);
+  if (wide)
+    hipLaunchKernelGGL(tn_f32mfma_kernel, grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
+  else
+    hipLaunchKernelGGL(tn_f32mfma64_kernel, grid, dim3(256), 0, s, n, p, q, A, lda, B, ldb, slices, work);
   MMSB_LAUNCH_CHECK();
-  const int64_t pq = (int64_t)p * q;
-  hipLaunchKernelGGL(tn_mfma_reduce_kernel, dim3((unsigned)ceil_div(pq, 256)), dim3(256), 0, s, p, q, slices, false, work,
-                     alpha, beta, C);
-  MMSB_LAUNCH_CHECK();
-  return MMSB_OK;
+  return tn_reduce(s, p, q, slices, 0, work, alpha, beta, C);
 }
 
 // ---- Cholesky factor and its inverse (CholeskyQR of the tall whitening sketches) ----------------
@@ -995,19 +1172,30 @@ __global__ void fill_u64_kernel(int64_t n, unsigned long long* p, unsigned long 
 
 // ---- column sign canonicalisation: largest-|.| entry of each column made positive ----------
 // key = (|v| bits << 32) | ~row: atomicMax picks the largest magnitude, then the smallest row.
+// 64 columns per workgroup, the rows of its slab dealt over four waves (loads of a wave are coalesced and
+// independent); one atomic per column and slab.
 template <typename T>
-__global__ void colmax_kernel(int64_t n, int32_t c, const T* __restrict__ M, int32_t ld,
-                              unsigned long long* __restrict__ best) {
-  const int col = blockIdx.y * blockDim.x + threadIdx.x;
-  if (col >= c) return;
+__global__ __launch_bounds__(256) void colmax_kernel(int64_t n, int32_t c, const T* __restrict__ M, int32_t ld,
+                                                     unsigned long long* __restrict__ best) {
+  __shared__ unsigned long long red[4][64];
+  const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+  const int col = blockIdx.y * 64 + l;
   const int64_t r0 = n * blockIdx.x / gridDim.x, r1 = n * (blockIdx.x + 1) / gridDim.x;
   unsigned long long b = 0;
-  for (int64_t i = r0; i < r1; ++i) {
-    const float a = fabsf((float)M[i * ld + col]);
-    const unsigned long long key = ((unsigned long long)__float_as_uint(a) << 32) | (0xFFFFFFFFull - (unsigned long long)i);
-    b = key > b ? key : b;
+  if (col < c) {
+#pragma unroll 4
+    for (int64_t i = r0 + w; i < r1; i += 4) {
+      const float a = fabsf((float)M[i * ld + col]);
+      const unsigned long long key = ((unsigned long long)__float_as_uint(a) << 32) | (0xFFFFFFFFull - (unsigned long long)i);
+      b = key > b ? key : b;
+    }
   }
-  atomicMax(best + col, b);
+  red[w][l] = b;
+  __syncthreads();
+  if (w == 0 && col < c) {
+    for (int i = 1; i < 4; ++i) b = red[i][l] > b ? red[i][l] : b;
+    atomicMax(best + col, b);
+  }
 }
 
 template <typename T>
@@ -1033,9 +1221,9 @@ int col_sign(hipStream_t s, int64_t n, int32_t c, const T* M, int32_t ld, unsign
   MMSB_CHECK_ARG(n >= 1 && n < 0xFFFFFFFFll && c >= 1, "col_sign: bad shape");
   hipLaunchKernelGGL(fill_u64_kernel, dim3((unsigned)ceil_div(c, 256)), dim3(256), 0, s, (int64_t)c, best, 0ull);
   MMSB_LAUNCH_CHECK();
-  const int slabs = (int)std::min<int64_t>(256, ceil_div(n, 1024));
+  const int slabs = (int)std::min<int64_t>(256, ceil_div(n, 64));  // n = 50k, c = 100: 48 slabs of one wave took 324 us, 256 of four waves 13
   dim3 grid((unsigned)slabs, (unsigned)ceil_div(c, 64));
-  hipLaunchKernelGGL((colmax_kernel<T>), grid, dim3(64), 0, s, n, c, M, ld, best);
+  hipLaunchKernelGGL((colmax_kernel<T>), grid, dim3(256), 0, s, n, c, M, ld, best);
   MMSB_LAUNCH_CHECK();
   hipLaunchKernelGGL((colsign_kernel<T>), dim3((unsigned)ceil_div(c, 64)), dim3(64), 0, s, c, M, ld, best, sign);
   MMSB_LAUNCH_CHECK();
