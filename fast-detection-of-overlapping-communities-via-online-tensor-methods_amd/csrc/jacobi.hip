@@ -10,12 +10,13 @@
 // of disjoint block pairs per sweep. One launch per round: the workgroup of block pair (P, Q) loads
 // their 2B columns of A (and of V when it is accumulated) into LDS, orthogonalises every column pair
 // among them (one inner sweep of 2B - 1 inner rounds of B disjoint pairs, one wave per pair), writes
-// them back and adds its rotation count to the sweep's counter. After each sweep a one-thread kernel
-// marks convergence (a sweep without rotations) and the host reads the mark. Plain launches keep the
+// them back and adds its rotation count to the sweep's counter, which the host reads from the fourth
+// sweep on (one without rotations ends the factorisation). Plain launches keep the
 // factorisation free of cooperative launches, whose global-wave-sync resource only one process on a
 // GPU can hold, and a launch boundary costs less than a grid-wide barrier on this part.
 #include "common.h"
 #include "dense.h"
+#include "wave.h"
 
 namespace mmsb {
 
@@ -25,11 +26,11 @@ static constexpr int kMaxSweeps = 40;
 #ifndef MMSB_JACOBI_BMAX
 #define MMSB_JACOBI_BMAX 8
 #endif
-// counters: [0, kMaxSweeps) rotations per sweep, [kMaxSweeps] sweeps run, [kMaxSweeps + 1] converged
-static constexpr int kSweepsRun = kMaxSweeps, kDone = kMaxSweeps + 1;
+// counters: [0, kMaxSweeps) rotations per sweep. A sweep without rotations ends the factorisation: every later
+// round sees its predecessor's zero and returns.
 
 size_t jacobi_workspace_bytes(int32_t r) {
-  return sizeof(double) * ((size_t)r * r + (size_t)r) + sizeof(int32_t) * (kMaxSweeps + 2) + 64;
+  return sizeof(double) * ((size_t)r * r + (size_t)r) + sizeof(int32_t) * kMaxSweeps + 64;
 }
 
 __device__ inline double block_sum(double v, double* red) {
@@ -66,22 +67,31 @@ __global__ void jacobi_init_kernel(int32_t r, double* __restrict__ Vw, int32_t* 
   const int64_t gsz = (int64_t)gridDim.x * blockDim.x;
   if (Vw)
     for (int64_t e = gtid; e < rr; e += gsz) Vw[e] = ((e / r) == (e % r)) ? 1.0 : 0.0;
-  for (int64_t e = gtid; e < kMaxSweeps + 2; e += gsz) counters[e] = 0;
+  for (int64_t e = gtid; e < kMaxSweeps; e += gsz) counters[e] = 0;
 }
 
-// One round of a sweep: workgroup b handles block pair b of the round (grid = block pairs).
-template <int B, bool WV>
+// One round of a sweep: workgroup b handles block pair b of the round (grid = block pairs), wave g the pair g of
+// every inner round. Bound by the chain of one inner round -- dot products, three wave sums, the rotation's
+// divisions and square roots, the barrier -- 15 times per launch. MIN <= r <= 64 RM: a lane keeps its RM entries
+// of both columns in registers from the dot products to the rotation (RM = 0: any r, entries re-read); the wave
+// sums stay out of LDS (wave.h), V's columns are read while the rotation is formed, and every wave moves two
+// columns between HBM and LDS with all its loads in flight. The arithmetic and its order are those of a
+// lane-strided sum and a shuffle butterfly. With 8 waves two share a SIMD, so every instruction of that chain
+// counts twice: 3000 cycles per inner round at r = 110 before the sums were packed and the square roots paired,
+// 1600 after. A launch at r = 110 takes 16.9 us with V and 15.8 without (33.6 and 30.8 with re-read columns, LDS
+// shuffles and loads in turn); a 50k-node, k = 100 whitening 14.7 -> 10.7 ms.
+template <int B, bool WV, int RM, int MIN>
 __global__ __launch_bounds__(64 * B) void jacobi_round_kernel(int32_t r, double* __restrict__ A, double* __restrict__ Vw,
                                                               int32_t* __restrict__ counters, int32_t sweep, int32_t round) {
-  constexpr int TPG = 64;                  // one wave per column pair (64 B threads per workgroup)
+  constexpr int M = RM > 0 ? RM : 1;
   extern __shared__ double lds[];          // [2B][r] columns of A, then (WV) [2B][r] columns of V
   __shared__ int nrot;
-  if (counters[kDone]) return;             // converged in an earlier sweep (uniform)
+  const int32_t live = sweep > 0 ? counters[sweep - 1] : 1;  // tested once the columns' loads are on their way
   double* la = lds;
   double* lv = lds + (int64_t)2 * B * r;
   const int nblk = (r + B - 1) / B;
   const int nbp = nblk + (nblk & 1);
-  const int g = threadIdx.x / TPG, tg = threadIdx.x % TPG;
+  const int g = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tg = threadIdx.x & 63;
   int P, Q;
   pair_of(nbp, round, blockIdx.x, P, Q);
   auto gcol = [&](int lc) -> int {  // global column of local column lc, or -1
@@ -89,52 +99,119 @@ __global__ __launch_bounds__(64 * B) void jacobi_round_kernel(int32_t r, double*
     const int c = blkid * B + (lc % B);
     return (blkid < nblk && c < r) ? c : -1;
   };
-  for (int lc = 0; lc < 2 * B; ++lc) {
-    const int c = gcol(lc);
-    if (c < 0) continue;
-    for (int i = threadIdx.x; i < r; i += blockDim.x) {
-      la[(int64_t)lc * r + i] = A[(int64_t)c * r + i];
-      if constexpr (WV) lv[(int64_t)lc * r + i] = Vw[(int64_t)c * r + i];
+  const int c0 = gcol(g), c1 = gcol(g + B);  // the columns this wave moves
+  for (int base = 0; base < r; base += 64 * M) {
+    double a0[M], a1[M], v0[M], v1[M];
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int i = base + 64 * m + tg;
+      a0[m] = (c0 >= 0 && i < r) ? A[(int64_t)c0 * r + i] : 0.0;
+      a1[m] = (c1 >= 0 && i < r) ? A[(int64_t)c1 * r + i] : 0.0;
+      if constexpr (WV) {
+        v0[m] = (c0 >= 0 && i < r) ? Vw[(int64_t)c0 * r + i] : 0.0;
+        v1[m] = (c1 >= 0 && i < r) ? Vw[(int64_t)c1 * r + i] : 0.0;
+      }
+    }
+    if (live == 0) return;  // converged in an earlier sweep (uniform)
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      const int i = base + 64 * m + tg;
+      if (i < r) {
+        la[g * r + i] = a0[m];
+        la[(g + B) * r + i] = a1[m];
+        if constexpr (WV) {
+          lv[g * r + i] = v0[m];
+          lv[(g + B) * r + i] = v1[m];
+        }
+      }
     }
   }
   if (threadIdx.x == 0) nrot = 0;
   __syncthreads();
+  // entry 64 m + lane of a column, the last one for lanes past the end (whose value is then zeroed)
+  int at[M];
+  bool in[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    in[m] = 64 * m + tg < r;
+    at[m] = in[m] ? 64 * m + tg : r - 1;
+  }
   int myrot = 0;
   for (int ir = 0; ir < 2 * B - 1; ++ir) {
     int lp, lq;
     pair_of(2 * B, ir, g, lp, lq);
     if (gcol(lp) >= 0 && gcol(lq) >= 0) {
-      double* ap = la + (int64_t)lp * r;
-      double* aq = la + (int64_t)lq * r;
+      double* ap = la + lp * r;
+      double* aq = la + lq * r;
+      double* vp = lv + lp * r;
+      double* vq = lv + lq * r;
+      double x[M], y[M], vx[M], vy[M];
       double a = 0.0, b = 0.0, gg = 0.0;
-      for (int i = tg; i < r; i += TPG) {
-        const double x = ap[i], y = aq[i];
-        a = fma(x, x, a);
-        b = fma(y, y, b);
-        gg = fma(x, y, gg);
-      }
-      for (int off = TPG / 2; off > 0; off >>= 1) {
-        a += __shfl_xor(a, off);
-        b += __shfl_xor(b, off);
-        gg += __shfl_xor(gg, off);
-      }
-      if (gg != 0.0 && fabs(gg) > 1e-15 * sqrt(a * b)) {
-        const double zeta = (b - a) / (2.0 * gg);
-        const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + sqrt(1.0 + zeta * zeta));
-        const double c = 1.0 / sqrt(1.0 + t * t);
-        const double sn = c * t;
-        for (int i = tg; i < r; i += TPG) {
-          const double x = ap[i], y = aq[i];
-          ap[i] = c * x - sn * y;
-          aq[i] = sn * x + c * y;
+      if constexpr (RM > 0) {
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          x[m] = ap[at[m]];
+          y[m] = aq[at[m]];
         }
         if constexpr (WV) {
-          double* vp = lv + (int64_t)lp * r;
-          double* vq = lv + (int64_t)lq * r;
-          for (int i = tg; i < r; i += TPG) {
-            const double x = vp[i], y = vq[i];
-            vp[i] = c * x - sn * y;
-            vq[i] = sn * x + c * y;
+#pragma unroll
+          for (int m = 0; m < M; ++m) {
+            vx[m] = vp[at[m]];
+            vy[m] = vq[at[m]];
+          }
+        }
+#pragma unroll
+        for (int m = 0; m < M; ++m) {
+          if (64 * m + 64 > MIN) {
+            x[m] = in[m] ? x[m] : 0.0;
+            y[m] = in[m] ? y[m] : 0.0;
+          }
+          a = fma(x[m], x[m], a);
+          b = fma(y[m], y[m], b);
+          gg = fma(x[m], y[m], gg);
+        }
+      } else {
+        for (int i = tg; i < r; i += 64) {
+          const double p = ap[i], q = aq[i];
+          a = fma(p, p, a);
+          b = fma(q, q, b);
+          gg = fma(p, q, gg);
+        }
+      }
+      wave_sum3(a, b, gg);
+      // the two square roots of the test and of the rotation's first step in one go, in the wave's two halves
+      // (gg = 0 gives an infinite or undefined zeta that nothing uses)
+      const double zeta = (b - a) / (2.0 * gg);
+      const double root = sqrt(tg < 32 ? fma(zeta, zeta, 1.0) : a * b);
+      if (gg != 0.0 && fabs(gg) > 1e-15 * read_lane(root, 32)) {
+        const double t = (zeta >= 0.0 ? 1.0 : -1.0) / (fabs(zeta) + read_lane(root, 0));
+        const double c = 1.0 / sqrt(fma(t, t, 1.0));
+        const double sn = c * t;
+        if constexpr (RM > 0) {
+#pragma unroll
+          for (int m = 0; m < M; ++m) {
+            const int i = 64 * m + tg;
+            if (64 * m + 64 <= MIN || in[m]) {
+              ap[i] = fma(c, x[m], -(sn * y[m]));
+              aq[i] = fma(sn, x[m], c * y[m]);
+              if constexpr (WV) {
+                vp[i] = fma(c, vx[m], -(sn * vy[m]));
+                vq[i] = fma(sn, vx[m], c * vy[m]);
+              }
+            }
+          }
+        } else {
+          for (int i = tg; i < r; i += 64) {
+            const double p = ap[i], q = aq[i];
+            ap[i] = fma(c, p, -(sn * q));
+            aq[i] = fma(sn, p, c * q);
+          }
+          if constexpr (WV) {
+            for (int i = tg; i < r; i += 64) {
+              const double p = vp[i], q = vq[i];
+              vp[i] = fma(c, p, -(sn * q));
+              vq[i] = fma(sn, p, c * q);
+            }
           }
         }
         if (tg == 0) ++myrot;
@@ -143,22 +220,16 @@ __global__ __launch_bounds__(64 * B) void jacobi_round_kernel(int32_t r, double*
     __syncthreads();
   }
   if (tg == 0 && myrot) atomicAdd(&nrot, myrot);
-  for (int lc = 0; lc < 2 * B; ++lc) {
-    const int c = gcol(lc);
-    if (c < 0) continue;
-    for (int i = threadIdx.x; i < r; i += blockDim.x) {
-      A[(int64_t)c * r + i] = la[(int64_t)lc * r + i];
-      if constexpr (WV) Vw[(int64_t)c * r + i] = lv[(int64_t)lc * r + i];
+  for (int i = tg; i < r; i += 64) {
+    if (c0 >= 0) A[(int64_t)c0 * r + i] = la[g * r + i];
+    if (c1 >= 0) A[(int64_t)c1 * r + i] = la[(g + B) * r + i];
+    if constexpr (WV) {
+      if (c0 >= 0) Vw[(int64_t)c0 * r + i] = lv[g * r + i];
+      if (c1 >= 0) Vw[(int64_t)c1 * r + i] = lv[(g + B) * r + i];
     }
   }
   __syncthreads();
   if (threadIdx.x == 0 && nrot) atomicAdd(counters + sweep, nrot);
-}
-
-__global__ void jacobi_sweep_end_kernel(int32_t* __restrict__ counters, int32_t sweep) {
-  if (threadIdx.x != 0 || counters[kDone]) return;
-  counters[kSweepsRun] = sweep + 1;
-  if (counters[sweep] == 0) counters[kDone] = 1;
 }
 
 // sw[j] = ||A_j||, one workgroup per column.
@@ -197,32 +268,54 @@ __global__ __launch_bounds__(256) void jacobi_sort_kernel(int32_t r, const doubl
     if (threadIdx.x == 0) sigma[rank] = sj;
     __syncthreads();
   }
-  if (blockIdx.x == 0 && threadIdx.x == 0) sweeps_out[0] = counters[kSweepsRun];
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    int sweeps = 0;
+    while (sweeps < kMaxSweeps && counters[sweeps]) ++sweeps;
+    sweeps_out[0] = sweeps + 1;  // the last one rotated nothing
+  }
 }
 
-template <int B, bool WV>
-static int run_sweeps(hipStream_t s, int32_t r, double* A, double* Vw, int32_t* counters) {
-  const void* fn = reinterpret_cast<const void*>(jacobi_round_kernel<B, WV>);
+template <int B, bool WV, int RM, int MIN>
+static int run_sweeps_rm(hipStream_t s, int32_t r, double* A, double* Vw, int32_t* counters) {
+  const void* fn = reinterpret_cast<const void*>(jacobi_round_kernel<B, WV, RM, MIN>);
   const size_t shm = sizeof(double) * (size_t)(WV ? 4 : 2) * B * r;
   MMSB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)shm));
   const int nblk = (r + B - 1) / B;
   const int nbp = nblk + (nblk & 1);
   const int npairs = nbp / 2;
-  int32_t done = 0;
-  for (int sweep = 0; sweep < kMaxSweeps && !done; ++sweep) {
+  int32_t rotations = 1;
+  for (int sweep = 0; sweep < kMaxSweeps && rotations; ++sweep) {
     for (int round = 0; round < nbp - 1; ++round) {
-      hipLaunchKernelGGL((jacobi_round_kernel<B, WV>), dim3(npairs), dim3(64 * B), shm, s, r, A, Vw, counters, sweep,
+      hipLaunchKernelGGL((jacobi_round_kernel<B, WV, RM, MIN>), dim3(npairs), dim3(64 * B), shm, s, r, A, Vw, counters, sweep,
                          round);
       MMSB_LAUNCH_CHECK();
     }
-    hipLaunchKernelGGL(jacobi_sweep_end_kernel, dim3(1), dim3(64), 0, s, counters, sweep);
-    MMSB_LAUNCH_CHECK();
-    MMSB_HIP(hipMemcpyAsync(&done, counters + kDone, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+    // No matrix that is not already orthogonal converges in four sweeps (random ones take 10 at r = 110, 30 at 510):
+    // until then the host does not wait, and the rounds after an early convergence return at once.
+    if (sweep < 3) continue;
+    MMSB_HIP(hipMemcpyAsync(&rotations, counters + sweep, sizeof(int32_t), hipMemcpyDeviceToHost, s));
     MMSB_HIP(hipStreamSynchronize(s));
   }
-  if (!done)  // every sweep still rotated: the factors are not converged, so say so instead of using them
+  if (rotations)  // every sweep still rotated: the factors are not converged, so say so instead of using them
     return set_error(MMSB_ERR_NUMERIC, "jacobi: no convergence after %d sweeps (r = %d)", kMaxSweeps, r);
   return MMSB_OK;
+}
+
+template <int B, bool WV>
+static int run_sweeps(hipStream_t s, int32_t r, double* A, double* Vw, int32_t* counters) {
+  if constexpr (B >= 4) {  // columns in registers: up to 20 entries per lane
+#define MMSB_RM(RM, MIN) \
+  if (r <= 64 * RM) return run_sweeps_rm<B, WV, RM, MIN>(s, r, A, Vw, counters);
+    MMSB_RM(1, 1)
+    MMSB_RM(2, 65)
+    MMSB_RM(4, 129)
+    MMSB_RM(6, 257)
+    MMSB_RM(8, 385)
+    MMSB_RM(12, 513)
+    MMSB_RM(20, 769)
+#undef MMSB_RM
+  }
+  return run_sweeps_rm<B, WV, 0, 0>(s, r, A, Vw, counters);
 }
 
 int jacobi_svd(hipStream_t s, int32_t r, double* A, double* U, double* sigma, double* V, void* work, int32_t* sweeps_out) {
