@@ -37,11 +37,13 @@
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
+#include <cstring>
 #include <type_traits>
 #include <vector>
 
 #include "common.h"
 #include "stgd.h"
+#include "wave.h"
 
 namespace cg = cooperative_groups;
 
@@ -438,10 +440,11 @@ struct TileShm {
 // Writes block (i0, j0) of a new kp x kp iterate held as v[e] = element (i0 + r, j0 + c4 + e), with
 // r = thread / 8 and c4 = 4 (thread % 8): Out row-major (FP32 and, with SPLIT, BF16 pairs), OutT
 // transposed (FP32 without SPLIT, BF16 pairs with it: the transposes are only ever MFMA operands, and
-// a later FP32 run rebuilds its FP32 transpose in SETUP), *fslot = ||Out - prev||_F^2 over the block when fslot is given (prev in pre.pv; the step's
-// log entry is the sum of its tiles' slots, see frob_sum), and, when
+// a later FP32 run rebuilds its FP32 transpose in SETUP), *fslot = ||Out - prev||_F^2 over the block when fslot
+// is given (prev in pre.pv; the step's log entry is the sum of its tiles' slots, see frob_sum), and, when
 // mpart is given, mpart[(ti * 2 + s) * kp + j] = sum over the block's rows i of mu_s[i] Out[i][j]
-// (s = A, B; mu in pre.ua, pre.ub). Every thread of the block calls it.
+// (s = A, B; mu in pre.ua, pre.ub). Every thread of the block calls it. The stores go first: what the next
+// kernel waits for is their way to memory, under which the sums are taken.
 template <bool SPLIT>
 __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64_t j0, const float v[4], float* Out,
                                    uint16_t* Out16, float* OutT, uint16_t* OutT16, const TilePre& pre, double* fslot,
@@ -450,40 +453,11 @@ __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
   const int64_t nel = (int64_t)kp * kp;
   const int64_t off = (i0 + r) * kp + j0 + c4;
-  const bool act = epi_thread();  // waves 4.. hold no elements; they only meet the barrier
+  const bool act = epi_thread();  // waves 4.. hold no elements; they only meet the barriers
   if (act) {
-  put4<SPLIT>(Out, Out16, nel, off, v);
 #pragma unroll
-  for (int e = 0; e < 4; ++e) S.t[c4 + e][r] = v[e];
-  if (fslot) {
-    double d = 0.0;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const double dd = (double)v[e] - (double)pre.pv[e];
-      d += dd * dd;
-    }
-    for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o);
-    if (lane == 0) S.d[w] = d;
-  }
-  if (mpart) {
-    float sa[4], sb[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      sa[e] = pre.ua * v[e];
-      sb[e] = pre.ub * v[e];
-      for (int o = 8; o < 64; o <<= 1) {  // lanes with equal lane % 8 hold the same columns
-        sa[e] += __shfl_xor(sa[e], o);
-        sb[e] += __shfl_xor(sb[e], o);
-      }
-    }
-    if (lane < 8) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        S.m[w][0][c4 + e] = sa[e];
-        S.m[w][1][c4 + e] = sb[e];
-      }
-    }
-  }
+    for (int e = 0; e < 4; ++e) S.t[c4 + e][r] = v[e];
+    put4<SPLIT>(Out, Out16, nel, off, v);
   }
   __syncthreads();
   if (act) {
@@ -491,6 +465,35 @@ __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64
     const float t[4] = {S.t[c][r4], S.t[c][r4 + 1], S.t[c][r4 + 2], S.t[c][r4 + 3]};
     put4<SPLIT>(SPLIT ? nullptr : OutT, OutT16, nel, (j0 + c) * kp + i0 + r4, t);
   }
+  if (!fslot && !mpart) return;  // uniform over the block
+  if (act && fslot) {
+    double d = 0.0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const double dd = (double)v[e] - (double)pre.pv[e];
+      d = fma(dd, dd, d);
+    }
+    d = wave_sum(d);
+    if (lane == 0) S.d[w] = d;
+  }
+  if (act && mpart) {
+    // lanes with equal lane % 8 hold the same columns: their eight rows are summed over offsets 8, 16, 32, the last
+    // two packed (the odd rows of 16 lanes carry s = B, the upper half the columns 2 and 3)
+    float q[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float pa = pre.ua * v[e], pb = pre.ub * v[e];
+      const float sa = fmaf(pre.ua, v[e], dpp_mov<kDppRor8>(pa)), sb = fmaf(pre.ub, v[e], dpp_mov<kDppRor8>(pb));
+      q[e] = swap_add16(sa, sb);
+    }
+    const float s01 = swap_add32(q[0], q[2]), s23 = swap_add32(q[1], q[3]);
+    if ((lane & 15) < 8) {
+      const int h = lane >> 5, sx = (lane >> 4) & 1, c = 4 * (lane & 7) + 2 * h;
+      S.m[w][sx][c] = s01;
+      S.m[w][sx][c + 1] = s23;
+    }
+  }
+  __syncthreads();
   if (fslot && threadIdx.x == 0) *fslot = (S.d[0] + S.d[1]) + (S.d[2] + S.d[3]);
   if (mpart && threadIdx.x < 64) {
     const int s = threadIdx.x >> 5, c = threadIdx.x & 31;
@@ -521,25 +524,124 @@ __device__ inline void store4(T* p, const float v[4]) {
 enum StgdPhase { PH_SETUP = 0, PH_P1 = 1, PH_P2 = 2, PH_GRAM = 3, PH_UPDATE = 4, PH_COPY = 5, PH_QPOLY = 6, PH_QRFIN = 7,
                  PH_FROB = 8 };
 
-// Everything the phases of one step of one instance read or write.
-struct StepCtx {
-  StgdArgs a;          // a.phi = B.phi[cur], a.phit = B.phit
-  StgdBuffers B;
-  const void* YA;
-  const void* YB;
-  const void* YCt;
-  int32_t cur;         // B.phi[cur] holds the step's input Phi
-  int32_t ns_iters;
-  int32_t ns_degree;   // 3 or 5
-  int64_t row0;        // first X row of the minibatch
-  int64_t yrow0;       // its first row in the Y buffers (row0, or 0 when they hold only the minibatch)
-  int32_t nb;          // rows in the minibatch
-  int64_t st;          // step index within the run
-  double* frob_prev;   // the previous step's log entry within the run (null for the run's first), formed by
-                       // this step's P1 from the previous step's tile partials
-  double* frob;        // this step's ||Phi_{t+1} - Phi_t||_F^2 (written by FROB after a run's last step)
-  double* frob_zero;   // SETUP: the run's frob entries, cleared by tile 0
+// What one phase of one step reads and writes, resolved on the host: every pointer is the one to use (the Phi
+// ping-pong, the Newton-Schulz scratch of the iteration, the minibatch's first row), so that a kernel fetches
+// its arguments in one go instead of walking a context. Operands are FP32 or split BF16 ([hi | lo]) by the run's
+// mode; the *16 outputs are null in FP32 runs.
+struct P1Args {
+  const void *ya, *yb;   // the minibatch's first row, leading dimension kp
+  const void* phiT;      // operand
+  const float* mpart;
+  void* cgt;
+  float *cs_part, *mab;
+  float* h;
+  uint16_t* h16;
+  double* frob_prev;     // the previous step's log entry within the run (null for the run's first), formed here from
+  const double* fpart;   // the previous step's tile partials
+  int32_t kp, b, nb;
+  float c3, c1;
+};
+struct P2Args {
+  const void *phi_op, *h_op;
+  const float* phi;
+  const void* yct;       // the minibatch's first column, leading dimension n_pad
+  const void* cgt;
+  const float *cs_part, *mab;
+  const double* mu_c;
+  float* out;
+  uint16_t* out16;
+  float* outT;
+  uint16_t* outT16;
+  unsigned long long* rowsum;  // cleared for the first Newton-Schulz iteration
+  double* fpart;               // null unless the log is taken before the renormalisation
+  int64_t n_pad;
+  int32_t kp, b, nb, aligned;  // aligned: yct rows start on 16 bytes
+  float eta, theta, c0, c1;
+};
+struct GramArgs {
+  const void* xT;
+  float* g;
+  uint16_t* g16;
+  unsigned long long* rowsum;
+  int32_t kp;
+};
+struct QpolyArgs {
+  const void* g_op;
+  const float* g;
+  float* q;
+  uint16_t* q16;
+  const unsigned long long* rowsum;
+  int32_t kp;
+};
+struct UpdateArgs {
+  const void *x_op, *g_op;     // g_op: G (degree 3) or Q (degree 5)
+  const float* x;
+  float* out;
+  uint16_t* out16;
+  float* outT;
+  uint16_t* outT16;
+  const float* prev;           // the last iteration logs ||out - prev||^2 (fpart) and the m partials (mpart); else null
+  const double *mu_a, *mu_b;
+  double* fpart;
+  float* mpart;
+  const unsigned long long* rowsum;
+  unsigned long long* rowsum_next;
+  int32_t kp, quintic;
+};
+struct CopyArgs {              // COPY, QRFIN and SETUP
+  const float* x;
+  float* out;                  // null in SETUP
+  uint16_t* out16;
+  float* outT;
+  uint16_t* outT16;
+  const float* prev;
+  const double *mu_a, *mu_b;
+  double* fpart;
+  float* mpart;
+  double* frob_zero;           // SETUP: the run's log entries, cleared by tile 0
   int64_t nfrob;
+  int32_t kp, kmax;            // rows and columns from kmax on become zero
+};
+struct FrobArgs {
+  double* frob;
+  const double* fpart;
+  int32_t kp;
+};
+union PhaseArgs {
+  P1Args p1;
+  P2Args p2;
+  GramArgs gram;
+  QpolyArgs qpoly;
+  UpdateArgs update;
+  CopyArgs copy;
+  FrobArgs frob;
+};
+
+template <int PHASE>
+__host__ __device__ inline const auto& phase_args(const PhaseArgs& a) {
+  if constexpr (PHASE == PH_P1) return a.p1;
+  else if constexpr (PHASE == PH_P2) return a.p2;
+  else if constexpr (PHASE == PH_GRAM) return a.gram;
+  else if constexpr (PHASE == PH_QPOLY) return a.qpoly;
+  else if constexpr (PHASE == PH_UPDATE) return a.update;
+  else if constexpr (PHASE == PH_FROB) return a.frob;
+  else return a.copy;
+}
+template <int PHASE>
+struct ArgsOf { using type = CopyArgs; };
+template <> struct ArgsOf<PH_P1> { using type = P1Args; };
+template <> struct ArgsOf<PH_P2> { using type = P2Args; };
+template <> struct ArgsOf<PH_GRAM> { using type = GramArgs; };
+template <> struct ArgsOf<PH_QPOLY> { using type = QpolyArgs; };
+template <> struct ArgsOf<PH_UPDATE> { using type = UpdateArgs; };
+template <> struct ArgsOf<PH_FROB> { using type = FrobArgs; };
+
+// The end test of a step (per-phase launches only).
+struct StopArgs {
+  StgdStop* stop;
+  int64_t st;        // step index within the run
+  double thresh;
+  int64_t iter_min, iter_max;
 };
 
 union StgdSmem {
@@ -568,15 +670,16 @@ __host__ __device__ inline int phase_tiles(int phase, int kp, int b) {
   }
 }
 
-// Block (ti, tj), ti <= tj, of upper-triangle tile t (row-major over the triangle).
+// Block (ti, tj), ti <= tj, of upper-triangle tile t (row-major over the triangle): the row from the root of its
+// first tile's index i (2 ntk + 1 - i) / 2 <= t, corrected by one where the rounded root is off.
 __device__ inline void tri_tile(int t, int ntk, int& ti, int& tj) {
-  int i = 0;
-  while (t >= ntk - i) {
-    t -= ntk - i;
-    ++i;
-  }
-  ti = i;
-  tj = i + t;
+  const float n = (float)(2 * ntk + 1);
+  int i = (int)((n - sqrtf(fmaxf(n * n - 8.f * (float)t, 0.f))) * 0.5f);
+  i = min(max(i, 0), ntk - 1);
+  if (i * (2 * ntk + 1 - i) / 2 > t) --i;
+  if ((i + 1) * (2 * ntk - i) / 2 <= t) ++i;
+  ti = __builtin_amdgcn_readfirstlane(i);
+  tj = ti + t - ti * (2 * ntk + 1 - ti) / 2;
 }
 
 // The log entry ||Phi_{t+1} - Phi_t||_F^2 of a finished step from its tiles' partials fpart[0 .. n):
@@ -585,50 +688,17 @@ __device__ inline void tri_tile(int t, int ntk, int& ti, int& tj) {
 __device__ inline double frob_sum(const double* fpart, int n) {
   const int lane = threadIdx.x & 63;
   double s = 0.0;
+#pragma unroll 4
   for (int t = lane; t < n; t += 64) s += fpart[t];
-  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-  return s;
+  return wave_sum(s);
 }
 
-// Newton-Schulz iteration `it` reads (x, xT) and writes (dst, dstT): phit -> phia -> phit -> ...;
-// the last iteration writes phi[cur ^ 1] and phiT.
-struct NsBufs {
-  float *x, *xT, *dst, *dstT;
-  uint16_t *x16, *xT16, *dst16, *dstT16;
-};
-
-__host__ __device__ inline NsBufs ns_bufs(const StgdBuffers& B, int cur, int it, int ns_iters) {
-  NsBufs n;
-  const bool from_t = (it & 1) == 0;
-  const bool last = it == ns_iters - 1;
-  n.x = from_t ? B.phit : B.phia;
-  n.xT = from_t ? B.phitT : B.phiaT;
-  n.x16 = from_t ? B.phit16 : B.phia16;
-  n.xT16 = from_t ? B.phitT16 : B.phiaT16;
-  n.dst = last ? B.phi[cur ^ 1] : (from_t ? B.phia : B.phit);
-  n.dstT = last ? B.phiT : (from_t ? B.phiaT : B.phitT);
-  n.dst16 = last ? B.phi16[cur ^ 1] : (from_t ? B.phia16 : B.phit16);
-  n.dstT16 = last ? B.phiT16 : (from_t ? B.phiaT16 : B.phitT16);
-  return n;
-}
-
-// The operand view of a kp x kp matrix for one mode: FP32 data, or the BF16 (hi, lo) pair.
+// A kp x kp operand of one mode: FP32 data, or the BF16 (hi, lo) pair.
 template <int MODE>
-__host__ __device__ inline Opnd<op_t<MODE>> pick(const float* f32, const uint16_t* s16, int64_t nel, int64_t ld) {
-  if constexpr (MODE == MM_F32) {
-    (void)s16;
-    (void)nel;
-    return opnd<float>(f32, nullptr, ld);
-  } else {
-    (void)f32;
-    const __bf16* p = reinterpret_cast<const __bf16*>(s16);
-    return opnd<__bf16>(p, p + nel, ld);
-  }
-}
-
-template <bool SPLIT>
-__device__ inline uint16_t* sp(uint16_t* p) {
-  return SPLIT ? p : nullptr;
+__device__ inline Opnd<op_t<MODE>> pick(const void* p, int64_t nel, int64_t ld) {
+  const op_t<MODE>* q = static_cast<const op_t<MODE>*>(p);
+  if constexpr (MODE == MM_F32) return opnd<float>(q, nullptr, ld);
+  else return opnd<__bf16>(q, q + nel, ld);
 }
 
 // Sums of strided partials, one per output column: out[o] = sum_{t < nt} src[t * stride + off(o)]
@@ -660,9 +730,7 @@ __device__ inline float mpart_reduce(const PartSum& ps, const float* mpart, int 
   float m = (ps.v[0] + ps.v[1]) + (ps.v[2] + ps.v[3]);
   if (ps.extra)
     for (int ti = q + 4 * kPartRegs; ti < ntk; ti += 4) m += mpart[((int64_t)ti * 2 + s) * kp + j0 + c];
-  m += __shfl_xor(m, 1);
-  m += __shfl_xor(m, 2);
-  return m;  // valid in every lane of the output's group of four
+  return quad_sum(m);  // valid in every lane of the output's group of four
 }
 
 // P2: column sums of the b/32 row-tile partials cs_part[tb][j0 + c]: thread -> c = t / 8,
@@ -682,18 +750,14 @@ __device__ inline float cspart_reduce(const PartSum& ps, const float* cs_part, i
   float m = (ps.v[0] + ps.v[1]) + (ps.v[2] + ps.v[3]);
   if (ps.extra)
     for (int tb = q + 8 * kPartRegs; tb < ntb; tb += 8) m += cs_part[(int64_t)tb * kp + j0 + c];
-  m += __shfl_xor(m, 1);
-  m += __shfl_xor(m, 2);
-  m += __shfl_xor(m, 4);
-  return m;
+  return oct_sum(m);
 }
 
 // P1 tiles [0, ntk (ntk + 1) / 2): upper-triangle H tiles; the rest: a 32-row slice of the minibatch x
-// 32 columns of C_g.
+// 32 columns of C_g. Tile 0 also forms the previous step's log entry (wave 0; the partials' loads go first).
 template <int DMODE, int KMODE, typename TY, typename TPH>
-__device__ __forceinline__ void p1_tile(const StepCtx& P, int tile, StgdSmem& sm) {
+__device__ __forceinline__ void p1_tile(const P1Args& a, int tile, StgdSmem& sm, bool log) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
-  const StgdArgs& a = P.a;
   const int kp = a.kp;
   const int ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
@@ -706,15 +770,14 @@ __device__ __forceinline__ void p1_tile(const StepCtx& P, int tile, StgdSmem& sm
     const int tb = tile / ntk, tj = tile % ntk;
     const int64_t x0 = (int64_t)tb * 32, j0 = (int64_t)tj * 32;
     PartSum ps;
-    if (epi_thread()) mpart_load(ps, P.B.mpart, kp, ntk, j0);  // m_A, m_B of the block's columns
+    if (epi_thread()) mpart_load(ps, a.mpart, kp, ntk, j0);  // m_A, m_B of the block's columns
     // every wave: P_A and P_B over its part of the k reduction, sharing the Phi^T fragments
     floatx16 acc_b = {};
     kslice<DMODE>(kp, kWaves, w, k0, kl);
-    wave_mm_pair<DMODE>(acc, acc_b, static_cast<const TY*>(P.YA) + P.yrow0 * (int64_t)kp,
-                        static_cast<const TY*>(P.YB) + P.yrow0 * (int64_t)kp, kp, pick<DMODE>(P.B.phiT, P.B.phiT16, nel, kp).hi,
-                        kp, x0, j0, k0, kl);
+    wave_mm_pair<DMODE>(acc, acc_b, static_cast<const TY*>(a.ya), static_cast<const TY*>(a.yb), kp,
+                        pick<DMODE>(a.phiT, nel, kp).hi, kp, x0, j0, k0, kl);
     if (epi_thread()) {
-      const float m = mpart_reduce(ps, P.B.mpart, kp, ntk, j0);
+      const float m = mpart_reduce(ps, a.mpart, kp, ntk, j0);
       const int o = threadIdx.x >> 2;
       if ((threadIdx.x & 3) == 0) sm.p1.mvec[o >> 5][o & 31] = m;
     }
@@ -731,13 +794,13 @@ __device__ __forceinline__ void p1_tile(const StepCtx& P, int tile, StgdSmem& sm
       const int r = r4 + e;
       const float p = red_sum4(sm.p1.red[0], r, c);
       const float q = red_sum4(sm.p1.red[1], r, c);
-      const bool valid = (x0 + r) < P.nb;
+      const bool valid = (x0 + r) < a.nb;
       const float ab = p * q;
       cs += valid ? ab : 0.f;
       cg[e] = valid ? a.c3 * ab + a.c1 * (p * mB + mA * q) : 0.f;
     }
-    store4(static_cast<TPH*>(P.B.cgt) + (j0 + c) * (int64_t)a.b + x0 + r4, cg);
-    for (int off = 1; off < 8; off <<= 1) cs += __shfl_xor(cs, off);
+    store4(static_cast<TPH*>(a.cgt) + (j0 + c) * (int64_t)a.b + x0 + r4, cg);
+    cs = oct_sum(cs);
     if ((threadIdx.x & 7) == 0) {
       a.cs_part[(int64_t)tb * kp + j0 + c] = cs;
       if (tb == 0) {
@@ -746,12 +809,22 @@ __device__ __forceinline__ void p1_tile(const StepCtx& P, int tile, StgdSmem& sm
       }
     }
   } else {
+    log = log && tile == 0 && a.frob_prev && w == 0;
+    double fs = 0.0;
+    if (log) {
+#pragma unroll 4
+      for (int t = threadIdx.x; t < ntk * ntk; t += 64) fs += a.fpart[t];
+    }
     int ti, tj;
     tri_tile(tile, ntk, ti, tj);
     const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
-    const Opnd<op_t<KMODE>> phiT_k = pick<KMODE>(P.B.phiT, P.B.phiT16, nel, kp);
+    const Opnd<op_t<KMODE>> phiT_k = pick<KMODE>(a.phiT, nel, kp);
     kslice<KMODE>(kp, kWaves, w, k0, kl);
     wave_mm<KMODE, true>(acc, phiT_k, phiT_k, i0, j0, k0, kl);  // G = Phi^T Phi
+    if (log) {
+      const double f = wave_sum(fs);
+      if (threadIdx.x == 0) *a.frob_prev = f;
+    }
     Red4& red = sm.p1.red[0];
     red_put(red, acc);
     __syncthreads();
@@ -763,23 +836,21 @@ __device__ __forceinline__ void p1_tile(const StepCtx& P, int tile, StgdSmem& sm
       g[e] = red_sum4(red, r, c4 + e);
       g[e] *= g[e];
     }
-    put4<SPLIT>(P.B.h, sp<SPLIT>(P.B.h16), nel, (i0 + r) * kp + j0 + c4, g);
+    put4<SPLIT>(a.h, a.h16, nel, (i0 + r) * kp + j0 + c4, g);
     if (ti != tj) {  // the mirror block (j, i): thread -> row c of it, columns r4 .. r4 + 3
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
         g[e] = red_sum4(red, c4 + e, r);
         g[e] *= g[e];
       }
-      put4<SPLIT>(P.B.h, sp<SPLIT>(P.B.h16), nel, (j0 + r) * kp + i0 + c4, g);
+      put4<SPLIT>(a.h, a.h16, nel, (j0 + r) * kp + i0 + c4, g);
     }
   }
 }
 
 template <int DMODE, int KMODE, typename TY, typename TPH>
-__device__ __forceinline__ void p2_tile(const StepCtx& P, int tile, StgdSmem& sm) {
+__device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
-  constexpr int VEC = 16 / sizeof(TY);  // Y_C^T elements per 16-byte load
-  const StgdArgs& a = P.a;
   const int kp = a.kp, ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
   const int w = wave_id();
@@ -805,13 +876,12 @@ __device__ __forceinline__ void p2_tile(const StepCtx& P, int tile, StgdSmem& sm
   const int part = (w & 1) + 2 * (w >> 2);
   if ((w & 2) == 0) {  // Phi H (H symmetric: row j of H is column j)
     kslice<KMODE>(kp, kWaves / 2, part, k0, kl);
-    wave_mm<KMODE, true>(acc, pick<KMODE>(a.phi, P.B.phi16[P.cur], nel, kp), pick<KMODE>(P.B.h, P.B.h16, nel, kp), i0, j0,
-                         k0, kl);
+    wave_mm<KMODE, true>(acc, pick<KMODE>(a.phi_op, nel, kp), pick<KMODE>(a.h_op, nel, kp), i0, j0, k0, kl);
   } else {             // Y_C^T C_g over parts of the minibatch tile
     kslice<DMODE>(a.b, kWaves / 2, part, k0, kl);
-    const Opnd<TY> yc = opnd<TY>(static_cast<const TY*>(P.YCt) + P.yrow0, nullptr, a.n_pad);
-    const Opnd<TPH> cg = opnd<TPH>(static_cast<const TPH*>(P.B.cgt), nullptr, a.b);
-    if (P.yrow0 % VEC == 0)
+    const Opnd<TY> yc = opnd<TY>(static_cast<const TY*>(a.yct), nullptr, a.n_pad);
+    const Opnd<TPH> cg = opnd<TPH>(static_cast<const TPH*>(a.cgt), nullptr, a.b);
+    if (a.aligned)
       wave_mm<DMODE, true>(acc, yc, cg, i0, j0, k0, kl);
     else
       wave_mm<DMODE, false>(acc, yc, cg, i0, j0, k0, kl);
@@ -819,13 +889,13 @@ __device__ __forceinline__ void p2_tile(const StepCtx& P, int tile, StgdSmem& sm
   if (epi) {
     const int c = threadIdx.x >> 3;
     const float ssum = cspart_reduce(ps, a.cs_part, kp, a.b / 32, j0);
-    if ((threadIdx.x & 7) == 0) sm.p2.cmu[c] = a.c0 * mab_a * mab_b + a.c1 * ssum / (float)P.nb;
+    if ((threadIdx.x & 7) == 0) sm.p2.cmu[c] = a.c0 * mab_a * mab_b + a.c1 * ssum / (float)a.nb;
   }
   if (tile == 0)
-    for (int t = threadIdx.x; t < kp; t += blockDim.x) P.B.rowsum[t] = 0ull;
+    for (int t = threadIdx.x; t < kp; t += blockDim.x) a.rowsum[t] = 0ull;
   red_put(red, acc);
   __syncthreads();
-  const float eta = a.eta, inv_b = 1.f / (float)P.nb;
+  const float eta = a.eta, inv_b = 1.f / (float)a.nb;
   const float p0[4] = {ph.x, ph.y, ph.z, ph.w};
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (epi) {
@@ -837,11 +907,10 @@ __device__ __forceinline__ void p2_tile(const StepCtx& P, int tile, StgdSmem& sm
       v[e] = p0[e] - eta * a.theta * phh + eta * (t * inv_b + muc * sm.p2.cmu[c]);
     }
   }
-  TilePre pre{};  // the reference's log: ||Phi~ - Phi||^2 before the renormalisation (frob_pre)
+  TilePre pre{};  // the reference's log: ||Phi~ - Phi||^2 before the renormalisation
 #pragma unroll
   for (int e = 0; e < 4; ++e) pre.pv[e] = p0[e];
-  finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, a.phit, sp<SPLIT>(P.B.phit16), P.B.phitT, sp<SPLIT>(P.B.phitT16),
-                     pre, a.frob_pre ? P.B.fpart + tile : nullptr, nullptr);
+  finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, a.out, a.out16, a.outT, a.outT16, pre, a.fpart ? a.fpart + tile : nullptr, nullptr);
 }
 
 // The Newton-Schulz scale guard c = min(1, sqrt(2 / ||G||_inf)) from the row sums of |G|, computed
@@ -850,97 +919,95 @@ __device__ __forceinline__ void p2_tile(const StepCtx& P, int tile, StgdSmem& sm
 // The row sums are accumulated across tiles as fixed-point integers (units of 2^-32): integer
 // addition is associative, so the sums -- and the guard they decide -- do not depend on the order in
 // which the tiles' atomics land, and Phi is bit-reproducible from run to run. Partial sums are
-// clamped at 2^30, far beyond the point where the guard acts.
+// clamped at 2^30, far beyond the point where the guard acts. The largest is found among the integers and
+// converted once (conversion is monotone): converted one by one under a branch each, eight loads of a wave came
+// back one after another, 2.3 us of an UPDATE at kp = 512.
 __device__ inline unsigned long long fix32(float s) {
   return (unsigned long long)(long long)llrintf(fminf(s, 1073741824.f) * 4294967296.f);
 }
 
-__device__ inline float unfix32(unsigned long long v) { return (float)((double)v * 2.3283064365386963e-10); }
-
-__device__ inline void guard_load(float rs[8], const unsigned long long* rowsum, int kp) {
+__device__ inline void guard_load(unsigned long long rs[8], const unsigned long long* rowsum, int kp) {
   const int lane = threadIdx.x & 63;
 #pragma unroll
-  for (int u = 0; u < 8; ++u) rs[u] = lane + 64 * u < kp ? unfix32(rowsum[lane + 64 * u]) : 0.f;
+  for (int u = 0; u < 8; ++u) rs[u] = rowsum[min(lane + 64 * u, kp - 1)];
 }
 
-__device__ inline void guard_scale(const float rs[8], const unsigned long long* rowsum, int kp, float* cscale) {
+__device__ inline void guard_scale(const unsigned long long rs[8], const unsigned long long* rowsum, int kp, float* cscale) {
   const int lane = threadIdx.x & 63;
-  float mx = 0.f;
+  unsigned long long m = 0;
 #pragma unroll
-  for (int u = 0; u < 8; ++u) mx = fmaxf(mx, rs[u]);
-  for (int t = lane + 512; t < kp; t += 64) mx = fmaxf(mx, unfix32(rowsum[t]));
-  for (int off = 32; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off));
+  for (int u = 0; u < 8; ++u) m = rs[u] > m ? rs[u] : m;
+  for (int t = lane + 512; t < kp; t += 64) m = rowsum[t] > m ? rowsum[t] : m;
+  const float mx = (float)(wave_max((double)m) * 2.3283064365386963e-10);
   if (lane == 0) *cscale = mx > 2.f ? sqrtf(2.f / mx) : 1.f;
 }
 
-// G = X^T X of Newton-Schulz iteration `it` on upper-triangle tile `tile` (block and mirror), and
-// rowsum[i] += sum over the block's columns of |G_ij| for every row i the block and its mirror cover.
+// G = X^T X of a Newton-Schulz iteration on upper-triangle tile `tile` (block and mirror), and
+// rowsum[i] += sum over the block's columns of |G_ij| for every row i the block and its mirror cover (the atomics
+// go out before the stores, whose way to memory is the shorter).
 template <int KMODE>
-__device__ __forceinline__ void gram_tile(const StepCtx& P, int it, int tile, StgdSmem& sm) {
+__device__ __forceinline__ void gram_tile(const GramArgs& a, int tile, StgdSmem& sm) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
-  const int kp = P.a.kp, ntk = kp / 32;
+  const int kp = a.kp, ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
   const int w = wave_id();
   int ti, tj;
   tri_tile(tile, ntk, ti, tj);
   const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
-  const NsBufs nb = ns_bufs(P.B, P.cur, it, P.ns_iters);
-  unsigned long long* rowsum = P.B.rowsum + (it & 1) * kp;
   Red4& red = sm.p2.red;
   floatx16 acc = {};
   int64_t k0, kl;
-  const Opnd<op_t<KMODE>> xT = pick<KMODE>(nb.xT, nb.xT16, nel, kp);
+  const Opnd<op_t<KMODE>> xT = pick<KMODE>(a.xT, nel, kp);
   kslice<KMODE>(kp, kWaves, w, k0, kl);
   wave_mm<KMODE, true>(acc, xT, xT, i0, j0, k0, kl);
   red_put(red, acc);
   __syncthreads();
   if (!epi_thread()) return;
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
-  float g[4], s = 0.f;
+  float g[4], t[4], s = 0.f;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     g[e] = red_sum4(red, r, c4 + e);
     s += fabsf(g[e]);
   }
-  put4<SPLIT>(P.B.gt, sp<SPLIT>(P.B.gt16), nel, (i0 + r) * kp + j0 + c4, g);
-  for (int off = 1; off < 8; off <<= 1) s += __shfl_xor(s, off);
-  if ((threadIdx.x & 7) == 0) atomicAdd(rowsum + i0 + r, fix32(s));
+  s = oct_sum(s);
+  if ((threadIdx.x & 7) == 0) atomicAdd(a.rowsum + i0 + r, fix32(s));
   if (ti != tj) {  // the mirror block (j, i): thread -> row r of it, columns c4 .. c4 + 3
-    float t = 0.f;
+    s = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      g[e] = red_sum4(red, c4 + e, r);
-      t += fabsf(g[e]);
+      t[e] = red_sum4(red, c4 + e, r);
+      s += fabsf(t[e]);
     }
-    put4<SPLIT>(P.B.gt, sp<SPLIT>(P.B.gt16), nel, (j0 + r) * kp + i0 + c4, g);
-    for (int off = 1; off < 8; off <<= 1) t += __shfl_xor(t, off);
-    if ((threadIdx.x & 7) == 0) atomicAdd(rowsum + j0 + r, fix32(t));
+    s = oct_sum(s);
+    if ((threadIdx.x & 7) == 0) atomicAdd(a.rowsum + j0 + r, fix32(s));
   }
+  put4<SPLIT>(a.g, a.g16, nel, (i0 + r) * kp + j0 + c4, g);
+  if (ti != tj) put4<SPLIT>(a.g, a.g16, nel, (j0 + r) * kp + i0 + c4, t);
 }
 
 // Degree-5 iteration, second stage: Q = -(5/4) c^2 G + (3/8) c^4 G^2 (symmetric, as G), so that the
 // update is Xout = c X (15/8 I + Q).
 template <int KMODE>
-__device__ __forceinline__ void qpoly_tile(const StepCtx& P, int it, int tile, StgdSmem& sm) {
+__device__ __forceinline__ void qpoly_tile(const QpolyArgs& a, int tile, StgdSmem& sm) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
-  const int kp = P.a.kp, ntk = kp / 32;
+  const int kp = a.kp, ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
   const int w = wave_id();
   const int ti = tile / ntk, tj = tile % ntk;
   const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
-  const unsigned long long* rowsum = P.B.rowsum + (it & 1) * kp;
   Red4& red = sm.p2.red;
   floatx16 acc = {};
   int64_t k0, kl;
   kslice<KMODE>(kp, kWaves, w, k0, kl);
-  float rs[8];
-  if (w == 3) guard_load(rs, rowsum, kp);
+  unsigned long long rs[8];
+  if (w == 3) guard_load(rs, a.rowsum, kp);
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
   float4 gv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (epi_thread()) gv = *reinterpret_cast<const float4*>(P.B.gt + (i0 + r) * kp + j0 + c4);
-  const Opnd<op_t<KMODE>> g = pick<KMODE>(P.B.gt, P.B.gt16, nel, kp);
+  if (epi_thread()) gv = *reinterpret_cast<const float4*>(a.g + (i0 + r) * kp + j0 + c4);
+  const Opnd<op_t<KMODE>> g = pick<KMODE>(a.g_op, nel, kp);
   wave_mm<KMODE, true>(acc, g, g, i0, j0, k0, kl);  // (G G)_ij = G[i,:] . G[j,:] (G symmetric)
-  if (w == 3) guard_scale(rs, rowsum, kp, &sm.p2.cscale);
+  if (w == 3) guard_scale(rs, a.rowsum, kp, &sm.p2.cscale);
   red_put(red, acc);
   __syncthreads();
   if (!epi_thread()) return;
@@ -950,41 +1017,35 @@ __device__ __forceinline__ void qpoly_tile(const StepCtx& P, int it, int tile, S
   float v[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = a1 * gg[e] + a2 * red_sum4(red, r, c4 + e);
-  put4<SPLIT>(P.B.q, sp<SPLIT>(P.B.q16), nel, (i0 + r) * kp + j0 + c4, v);
+  put4<SPLIT>(a.q, a.q16, nel, (i0 + r) * kp + j0 + c4, v);
 }
 
 // Degree 3: Xout = c (1.5 X - 0.5 c^2 X G); degree 5: Xout = c (1.875 X + X Q). The outputs are those
 // of finish_tile (the last iteration also logs ||Phi_next - Phi||^2 and the partial sums of m_A, m_B).
 template <int KMODE>
-__device__ __forceinline__ void update_tile(const StepCtx& P, int it, int tile, StgdSmem& sm) {
+__device__ __forceinline__ void update_tile(const UpdateArgs& a, int tile, StgdSmem& sm) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
-  const int kp = P.a.kp, ntk = kp / 32;
+  const int kp = a.kp, ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
   const int w = wave_id();
   const int ti = tile / ntk, tj = tile % ntk;
   const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
-  const NsBufs nb = ns_bufs(P.B, P.cur, it, P.ns_iters);
-  const bool last = it == P.ns_iters - 1;
-  const unsigned long long* rowsum = P.B.rowsum + (it & 1) * kp;
-  unsigned long long* rowsum_next = P.B.rowsum + ((it + 1) & 1) * kp;
   Red4& red = sm.p2.red;
   floatx16 acc = {};
   int64_t k0, kl;
   kslice<KMODE>(kp, kWaves, w, k0, kl);
-  float rs[8];
-  if (w == 3) guard_load(rs, rowsum, kp);
-  const bool quintic = P.ns_degree == 5;
+  unsigned long long rs[8];
+  if (w == 3) guard_load(rs, a.rowsum, kp);
+  const bool quintic = a.quintic;
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
   float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (epi_thread()) xv = *reinterpret_cast<const float4*>(nb.x + (i0 + r) * kp + j0 + c4);
+  if (epi_thread()) xv = *reinterpret_cast<const float4*>(a.x + (i0 + r) * kp + j0 + c4);
   TilePre pre;
-  tile_pre(pre, kp, i0, j0, last ? P.a.phi : nullptr, last ? P.a.mu_a : nullptr, P.a.mu_b);
-  wave_mm<KMODE, true>(acc, pick<KMODE>(nb.x, nb.x16, nel, kp),
-                       quintic ? pick<KMODE>(P.B.q, P.B.q16, nel, kp) : pick<KMODE>(P.B.gt, P.B.gt16, nel, kp), i0, j0,
-                       k0, kl);  // X G or X Q (both symmetric)
-  if (w == 3) guard_scale(rs, rowsum, kp, &sm.p2.cscale);
+  tile_pre(pre, kp, i0, j0, a.prev, a.prev ? a.mu_a : nullptr, a.mu_b);
+  wave_mm<KMODE, true>(acc, pick<KMODE>(a.x_op, nel, kp), pick<KMODE>(a.g_op, nel, kp), i0, j0, k0, kl);  // X G or X Q (both symmetric)
+  if (w == 3) guard_scale(rs, a.rowsum, kp, &sm.p2.cscale);
   if (tile == 0)
-    for (int t = threadIdx.x; t < kp; t += blockDim.x) rowsum_next[t] = 0ull;
+    for (int t = threadIdx.x; t < kp; t += blockDim.x) a.rowsum_next[t] = 0ull;
   red_put(red, acc);
   __syncthreads();
   const float cs = sm.p2.cscale;
@@ -994,8 +1055,8 @@ __device__ __forceinline__ void update_tile(const StepCtx& P, int it, int tile, 
   if (epi_thread())
 #pragma unroll
     for (int e = 0; e < 4; ++e) v[e] = c1 * x[e] + c3 * red_sum4(red, r, c4 + e);
-  finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, nb.dst, sp<SPLIT>(nb.dst16), nb.dstT, sp<SPLIT>(nb.dstT16), pre,
-                     last ? P.B.fpart + tile : nullptr, last ? P.B.mpart : nullptr);
+  finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, a.out, a.out16, a.outT, a.outT16, pre, a.fpart ? a.fpart + tile : nullptr,
+                     a.mpart);
 }
 
 // COPY: Phi_next = Phi~ with the outputs of a last update; QRFIN: Phi_next = the QR factor the host
@@ -1003,118 +1064,246 @@ __device__ __forceinline__ void update_tile(const StepCtx& P, int it, int tile, 
 // before its QR). SETUP: the derived copies of the current Phi (split pairs, Phi^T, the m partial
 // sums), and tile 0 clears the run's frob entries.
 template <bool SPLIT>
-__device__ __forceinline__ void copy_tile(const StepCtx& P, bool setup, int tile, StgdSmem& sm, bool qrfin = false) {
-  const int kp = P.a.kp, ntk = kp / 32;
+__device__ __forceinline__ void copy_tile(const CopyArgs& a, int tile, StgdSmem& sm) {
+  const int kp = a.kp, ntk = kp / 32;
   const int ti = tile / ntk, tj = tile % ntk;
   const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
-  const float* X = setup ? P.B.phi[P.cur] : (qrfin ? P.B.phia : P.B.phit);
   float4 xv = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (epi_thread()) xv = *reinterpret_cast<const float4*>(X + (i0 + r) * kp + j0 + c4);
+  if (epi_thread()) xv = *reinterpret_cast<const float4*>(a.x + (i0 + r) * kp + j0 + c4);
   float v[4] = {xv.x, xv.y, xv.z, xv.w};
-  if (qrfin)
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
-      if (i0 + r >= P.a.k || j0 + c4 + e >= P.a.k) v[e] = 0.f;
-  if (setup && tile == 0)
-    for (int64_t t = threadIdx.x; t < P.nfrob; t += blockDim.x) P.frob_zero[t] = 0.0;
+  for (int e = 0; e < 4; ++e)
+    if (i0 + r >= a.kmax || j0 + c4 + e >= a.kmax) v[e] = 0.f;
+  if (a.frob_zero && tile == 0)
+    for (int64_t t = threadIdx.x; t < a.nfrob; t += blockDim.x) a.frob_zero[t] = 0.0;
   TilePre pre;
-  tile_pre(pre, kp, i0, j0, setup ? nullptr : P.a.phi, P.a.mu_a, P.a.mu_b);
-  if (setup)
-    finish_tile<SPLIT>(sm.S, kp, ti, i0, j0, v, nullptr, sp<SPLIT>(P.B.phi16[P.cur]), P.B.phiT, sp<SPLIT>(P.B.phiT16),
-                       pre, nullptr, P.B.mpart);
-  else
-    finish_tile<SPLIT>(sm.S, kp, ti, i0, j0, v, P.B.phi[P.cur ^ 1], sp<SPLIT>(P.B.phi16[P.cur ^ 1]), P.B.phiT,
-                       sp<SPLIT>(P.B.phiT16), pre, (qrfin || P.a.frob_pre) ? nullptr : P.B.fpart + tile, P.B.mpart);
+  tile_pre(pre, kp, i0, j0, a.prev, a.mu_a, a.mu_b);
+  finish_tile<SPLIT>(sm.S, kp, ti, i0, j0, v, a.out, a.out16, a.outT, a.outT16, pre, a.fpart ? a.fpart + tile : nullptr, a.mpart);
 }
 
 // FROB: the log entry of a run's last step from its tiles' partials (one wave).
-__device__ __forceinline__ void frob_final(const StepCtx& P) {
+__device__ __forceinline__ void frob_final(const FrobArgs& a) {
   if (threadIdx.x >= 64) return;
-  const int ntk = P.a.kp / 32;
-  const double f = frob_sum(P.B.fpart, ntk * ntk);
-  if (threadIdx.x == 0) *P.frob = f;
+  const int ntk = a.kp / 32;
+  const double f = frob_sum(a.fpart, ntk * ntk);
+  if (threadIdx.x == 0) *a.frob = f;
 }
 
-// P1's tile 0 also forms the previous step's log entry (wave 0, after its tile work).
-__device__ __forceinline__ void p1_log(const StepCtx& P) {
-  if (!P.frob_prev || threadIdx.x >= 64) return;
-  const int ntk = P.a.kp / 32;
-  const double f = frob_sum(P.B.fpart, ntk * ntk);
-  if (threadIdx.x == 0) *P.frob_prev = f;
+template <int DMODE, int KMODE, typename TY, typename TPH, int PHASE>
+__device__ __forceinline__ void phase_tile(const typename ArgsOf<PHASE>::type& a, int tile, StgdSmem& sm, bool log = true) {
+  constexpr bool SPLIT = KMODE == MM_BF16X3;
+  if constexpr (PHASE == PH_P1) p1_tile<DMODE, KMODE, TY, TPH>(a, tile, sm, log);
+  else if constexpr (PHASE == PH_P2) p2_tile<DMODE, KMODE, TY, TPH>(a, tile, sm);
+  else if constexpr (PHASE == PH_GRAM) gram_tile<KMODE>(a, tile, sm);
+  else if constexpr (PHASE == PH_QPOLY) qpoly_tile<KMODE>(a, tile, sm);
+  else if constexpr (PHASE == PH_UPDATE) update_tile<KMODE>(a, tile, sm);
+  else if constexpr (PHASE == PH_FROB) frob_final(a);
+  else copy_tile<SPLIT>(a, tile, sm);
 }
 
 template <int DMODE, int KMODE, typename TY, typename TPH>
-__device__ __forceinline__ void run_tile(const StepCtx& P, int phase, int it, int tile, StgdSmem& sm) {
-  constexpr bool SPLIT = KMODE == MM_BF16X3;
+__device__ __forceinline__ void run_tile(const PhaseArgs& a, int phase, int tile, StgdSmem& sm) {
   switch (phase) {
-    case PH_SETUP: copy_tile<SPLIT>(P, true, tile, sm); break;
-    case PH_P1:
-      p1_tile<DMODE, KMODE, TY, TPH>(P, tile, sm);
-      if (tile == 0) p1_log(P);
-      break;
-    case PH_FROB: frob_final(P); break;
-    case PH_P2: p2_tile<DMODE, KMODE, TY, TPH>(P, tile, sm); break;
-    case PH_GRAM: gram_tile<KMODE>(P, it, tile, sm); break;
-    case PH_UPDATE: update_tile<KMODE>(P, it, tile, sm); break;
-    case PH_QPOLY: qpoly_tile<KMODE>(P, it, tile, sm); break;
-    case PH_QRFIN: copy_tile<SPLIT>(P, false, tile, sm, true); break;
-    default: copy_tile<SPLIT>(P, false, tile, sm); break;
+    case PH_P1: phase_tile<DMODE, KMODE, TY, TPH, PH_P1>(a.p1, tile, sm); break;
+    case PH_FROB: phase_tile<DMODE, KMODE, TY, TPH, PH_FROB>(a.frob, tile, sm); break;
+    case PH_P2: phase_tile<DMODE, KMODE, TY, TPH, PH_P2>(a.p2, tile, sm); break;
+    case PH_GRAM: phase_tile<DMODE, KMODE, TY, TPH, PH_GRAM>(a.gram, tile, sm); break;
+    case PH_UPDATE: phase_tile<DMODE, KMODE, TY, TPH, PH_UPDATE>(a.update, tile, sm); break;
+    case PH_QPOLY: phase_tile<DMODE, KMODE, TY, TPH, PH_QPOLY>(a.qpoly, tile, sm); break;
+    default: phase_tile<DMODE, KMODE, TY, TPH, PH_COPY>(a.copy, tile, sm); break;
   }
 }
 
 // The end test of the reference's STGD loop after step t (sgd_iter, 0-based) with log value f
 // (stpm.c:747-765): converged, or past the cap.
-__device__ inline bool stop_test(const StgdArgs& a, int64_t t, double f) {
+__device__ inline bool stop_test(const StopArgs& a, int64_t t, double f) {
   return (a.iter_min > 0 && f < a.thresh && t > a.iter_min) || (a.iter_max > 0 && t > a.iter_max);
 }
 
 // One phase of one step, one kernel per phase (each with its own register allocation):
 // blockIdx.x = tile. (An XCD-aware order that gave each XCD a compact group of tiles cut the HBM
 // fetches of P1 from 24 to 9 MiB per launch, but the step took 2.6 % longer: the waves of a group
-// then request the same lines at the same moment.)
-// With the end test on (P.a.stop), every phase of step g = base + st first checks whether the loop
+// then request the same lines at the same moment.) At b = 1024 a phase is bound by latency, not by its products:
+// with the products taken out, UPDATE kept 6.8 of its 9.2 us at k = 500 (P1 5.6 of 10.4, P2 4.6 of 8.9, GRAM 4.0
+// of 6.3) -- argument and guard loads that came back one after another, sums through LDS shuffles ahead of the stores.
+// Arguments resolved on the host, independent loads and sums in registers after the stores took a step at k = 500 from
+// 55 to 48 us (UPDATE 9.2 -> 6.5) and at k = 100 in FP32 from 45 to 39.
+// With the end test on (STOP), every phase of step g = base + st first checks whether the loop
 // has ended; P1 of each step but a run's first forms the previous step's log entry in every wave
 // (its kernels have finished), workgroup 0 stores it, and every workgroup applies the test to it and
 // marks the end -- each reaches the same decision from the same bits, so the whole launch returns
 // together. P1 returns early only when an earlier step ended the loop (stop_at < g): stop_at == g
 // was set by a sibling workgroup, and workgroup 0 must still store the entry. The skipped kernels
 // write nothing, and the host reads stop_at after the run.
-template <int DMODE, int KMODE, typename TY, typename TPH, int PHASE>
-__global__ __launch_bounds__(kThreads) void stgd_phase_kernel(StepCtx P, int32_t it) {
+template <int DMODE, int KMODE, typename TY, typename TPH, int PHASE, bool STOP>
+__global__ __launch_bounds__(kThreads) void stgd_phase_kernel(typename ArgsOf<PHASE>::type a, StopArgs s) {
   __shared__ StgdSmem sm;
-  constexpr bool SPLIT = KMODE == MM_BF16X3;
-  if constexpr (PHASE != PH_SETUP) {
-    if (P.a.stop) {
-      const int64_t g = P.a.stop->base + P.st;
-      const int64_t sa = P.a.stop->stop_at;
-      if (sa < g || (PHASE != PH_P1 && sa == g)) return;  // an earlier step ended the loop (checked
-                                                           // first: the log of a skipped step is never written)
-      if constexpr (PHASE == PH_P1) {
-        if (P.frob_prev) {
-          const int ntk = P.a.kp / 32;
-          const double f = frob_sum(P.B.fpart, ntk * ntk);
-          if (blockIdx.x == 0 && threadIdx.x == 0) *P.frob_prev = f;
-          if (stop_test(P.a, g - 1, f)) {
-            if (threadIdx.x == 0) P.a.stop->stop_at = g;
-            return;
-          }
+  if constexpr (STOP && PHASE != PH_SETUP) {
+    const int64_t g = s.stop->base + s.st;
+    const int64_t sa = s.stop->stop_at;
+    if (sa < g || (PHASE != PH_P1 && sa == g)) return;  // an earlier step ended the loop (checked
+                                                         // first: the log of a skipped step is never written)
+    if constexpr (PHASE == PH_P1) {
+      if (a.frob_prev) {
+        const int ntk = a.kp / 32;
+        const double f = frob_sum(a.fpart, ntk * ntk);
+        if (blockIdx.x == 0 && threadIdx.x == 0) *a.frob_prev = f;
+        if (stop_test(s, g - 1, f)) {
+          if (threadIdx.x == 0) s.stop->stop_at = g;
+          return;
         }
       }
     }
   }
-  if constexpr (PHASE == PH_SETUP) copy_tile<SPLIT>(P, true, blockIdx.x, sm);
-  else if constexpr (PHASE == PH_P1) {
-    p1_tile<DMODE, KMODE, TY, TPH>(P, blockIdx.x, sm);
-    if (!P.a.stop && blockIdx.x == 0) p1_log(P);
-  } else if constexpr (PHASE == PH_FROB) frob_final(P);
-  else if constexpr (PHASE == PH_P2) p2_tile<DMODE, KMODE, TY, TPH>(P, blockIdx.x, sm);
-  else if constexpr (PHASE == PH_GRAM) gram_tile<KMODE>(P, it, blockIdx.x, sm);
-  else if constexpr (PHASE == PH_UPDATE) update_tile<KMODE>(P, it, blockIdx.x, sm);
-  else if constexpr (PHASE == PH_QPOLY) qpoly_tile<KMODE>(P, it, blockIdx.x, sm);
-  else if constexpr (PHASE == PH_QRFIN) copy_tile<SPLIT>(P, false, blockIdx.x, sm, true);
-  else copy_tile<SPLIT>(P, false, blockIdx.x, sm);
+  phase_tile<DMODE, KMODE, TY, TPH, PHASE>(a, blockIdx.x, sm, !STOP);
 }
+
+// ---- resolving the arguments (host) ------------------------------------------------------------------
+// One instance's buffers and settings, as the plan of a run or of a batch holds them.
+struct StepPlan {
+  StgdArgs a;
+  StgdBuffers B;
+  const void *YA, *YB, *YCt;
+  int32_t ns_iters, ns_degree;
+  bool bf16;
+  int64_t esz() const { return bf16 ? 2 : 4; }
+  const void* op(const float* f32, const uint16_t* s16) const { return bf16 ? (const void*)s16 : (const void*)f32; }
+  uint16_t* out16(uint16_t* p) const { return bf16 ? p : nullptr; }
+  const void* at(const void* p, int64_t elems) const { return static_cast<const char*>(p) + elems * esz(); }
+
+  // Newton-Schulz iteration `it` reads x, xT and writes dst, dstT: phit -> phia -> phit -> ...; the last
+  // iteration writes phi[cur ^ 1] and phiT.
+  struct Ns {
+    float *x, *xT, *dst, *dstT;
+    uint16_t *x16, *xT16, *dst16, *dstT16;
+  };
+  Ns ns(int cur, int it) const {
+    Ns n;
+    const bool from_t = (it & 1) == 0, last = it == ns_iters - 1;
+    n.x = from_t ? B.phit : B.phia;
+    n.xT = from_t ? B.phitT : B.phiaT;
+    n.x16 = from_t ? B.phit16 : B.phia16;
+    n.xT16 = from_t ? B.phitT16 : B.phiaT16;
+    n.dst = last ? B.phi[cur ^ 1] : (from_t ? B.phia : B.phit);
+    n.dstT = last ? B.phiT : (from_t ? B.phiaT : B.phitT);
+    n.dst16 = last ? B.phi16[cur ^ 1] : (from_t ? B.phia16 : B.phit16);
+    n.dstT16 = last ? B.phiT16 : (from_t ? B.phiaT16 : B.phitT16);
+    return n;
+  }
+
+  // Arguments of `phase` (iteration `it` of a renormalisation) of a step that reads phi[cur] and the minibatch of nb
+  // rows at row yrow0 of the Y buffers. log / log_prev: its and the previous step's log entries (log_prev null
+  // for a run's first step); log0, nlog: all of the run's (SETUP).
+  PhaseArgs resolve(int phase, int it, int cur, int64_t yrow0, int32_t nb, double* log, double* log_prev, double* log0,
+                    int64_t nlog) const {
+    PhaseArgs out;
+    std::memset(static_cast<void*>(&out), 0, sizeof(out));
+    const int kp = a.kp;
+    switch (phase) {
+      case PH_P1: {
+        P1Args& p = out.p1;
+        p.ya = at(YA, yrow0 * kp);
+        p.yb = at(YB, yrow0 * kp);
+        p.phiT = op(B.phiT, B.phiT16);
+        p.mpart = B.mpart;
+        p.cgt = B.cgt;
+        p.cs_part = a.cs_part;
+        p.mab = a.mab;
+        p.h = B.h;
+        p.h16 = out16(B.h16);
+        p.frob_prev = log_prev;
+        p.fpart = B.fpart;
+        p.kp = kp;
+        p.b = a.b;
+        p.nb = nb;
+        p.c3 = a.c3;
+        p.c1 = a.c1;
+        break;
+      }
+      case PH_P2: {
+        P2Args& p = out.p2;
+        p.phi_op = op(B.phi[cur], B.phi16[cur]);
+        p.h_op = op(B.h, B.h16);
+        p.phi = B.phi[cur];
+        p.yct = at(YCt, yrow0);
+        p.cgt = B.cgt;
+        p.cs_part = a.cs_part;
+        p.mab = a.mab;
+        p.mu_c = a.mu_c;
+        p.out = B.phit;
+        p.out16 = out16(B.phit16);
+        p.outT = B.phitT;
+        p.outT16 = out16(B.phitT16);
+        p.rowsum = B.rowsum;
+        p.fpart = a.frob_pre ? B.fpart : nullptr;
+        p.n_pad = a.n_pad;
+        p.kp = kp;
+        p.b = a.b;
+        p.nb = nb;
+        p.aligned = yrow0 % (16 / esz()) == 0;
+        p.eta = a.eta;
+        p.theta = a.theta;
+        p.c0 = a.c0;
+        p.c1 = a.c1;
+        break;
+      }
+      case PH_GRAM: {
+        const Ns n = ns(cur, it);
+        out.gram = GramArgs{op(n.xT, n.xT16), B.gt, out16(B.gt16), B.rowsum + (it & 1) * kp, kp};
+        break;
+      }
+      case PH_QPOLY:
+        out.qpoly = QpolyArgs{op(B.gt, B.gt16), B.gt, B.q, out16(B.q16), B.rowsum + (it & 1) * kp, kp};
+        break;
+      case PH_UPDATE: {
+        const Ns n = ns(cur, it);
+        const bool last = it == ns_iters - 1, quintic = ns_degree == 5;
+        UpdateArgs& p = out.update;
+        p.x_op = op(n.x, n.x16);
+        p.g_op = quintic ? op(B.q, B.q16) : op(B.gt, B.gt16);
+        p.x = n.x;
+        p.out = n.dst;
+        p.out16 = out16(n.dst16);
+        p.outT = n.dstT;
+        p.outT16 = out16(n.dstT16);
+        p.prev = last ? B.phi[cur] : nullptr;
+        p.mu_a = a.mu_a;
+        p.mu_b = a.mu_b;
+        p.fpart = last ? B.fpart : nullptr;
+        p.mpart = last ? B.mpart : nullptr;
+        p.rowsum = B.rowsum + (it & 1) * kp;
+        p.rowsum_next = B.rowsum + ((it + 1) & 1) * kp;
+        p.kp = kp;
+        p.quintic = quintic;
+        break;
+      }
+      case PH_FROB:
+        out.frob = FrobArgs{log, B.fpart, kp};
+        break;
+      default: {  // COPY, QRFIN, SETUP
+        CopyArgs& p = out.copy;
+        const bool setup = phase == PH_SETUP, qrfin = phase == PH_QRFIN;
+        p.x = setup ? B.phi[cur] : (qrfin ? B.phia : B.phit);
+        p.out = setup ? nullptr : B.phi[cur ^ 1];
+        p.out16 = out16(B.phi16[setup ? cur : cur ^ 1]);
+        p.outT = B.phiT;
+        p.outT16 = out16(B.phiT16);
+        p.prev = setup ? nullptr : B.phi[cur];
+        p.mu_a = a.mu_a;
+        p.mu_b = a.mu_b;
+        p.fpart = setup || qrfin || a.frob_pre ? nullptr : B.fpart;
+        p.mpart = B.mpart;
+        p.frob_zero = setup ? log0 : nullptr;
+        p.nfrob = nlog;
+        p.kp = kp;
+        p.kmax = qrfin ? a.k : kp;
+        break;
+      }
+    }
+    return out;
+  }
+};
 
 // ---- many instances in one persistent launch -------------------------------------------------------
 // The host lays the phases of every instance's steps out slot by slot: slot s holds the s-th phase
@@ -1122,83 +1311,42 @@ __global__ __launch_bounds__(kThreads) void stgd_phase_kernel(StepCtx P, int32_t
 // slot. The cooperative grid walks the slots; in each, the workgroups share the slot's tiles
 // (tile t of the slot goes to workgroup t mod grid), and a grid barrier separates consecutive
 // slots. Every workgroup executes every barrier, and no workgroup waits on another except there.
-struct BatchSeg {
-  int32_t inst;
+struct BatchSeg {      // host only: the plan before it is laid out
   int32_t phase;
-  int32_t it;
   int32_t ntiles;
-  int64_t step;     // step index within the launch
-  int64_t first;    // index of the segment's first tile within its slot
-  int64_t ctx;      // its step's context in the plan's context array
+  PhaseArgs args;
 };
 
-struct BatchInst {
-  StgdArgs a;
-  StgdBuffers B;
-  const void* YA;
-  const void* YB;
-  const void* YCt;
-  int32_t cur0;       // phi[cur0] holds Phi at the start of the launch
-  int32_t ns_iters;
-  int32_t ns_degree;
-  int64_t step0;      // global index of the launch's first step
-  int64_t spe;        // steps per epoch
-  double* frob_log;   // [steps of the launch]
-  int64_t nfrob;
-};
-
-__host__ __device__ inline void make_step(const BatchInst& I, int64_t st, StepCtx& P) {
-  P.a = I.a;
-  P.B = I.B;
-  P.YA = I.YA;
-  P.YB = I.YB;
-  P.YCt = I.YCt;
-  P.cur = I.cur0 ^ (int)(st & 1);
-  P.ns_iters = I.ns_iters;
-  P.ns_degree = I.ns_degree;
-  const int64_t g = I.step0 + st;
-  P.row0 = (g % I.spe) * I.a.bl;
-  P.yrow0 = P.row0;
-  P.nb = (int32_t)min((int64_t)I.a.bl, I.a.n_x - P.row0);
-  P.st = st;
-  P.frob_prev = st > 0 ? I.frob_log + st - 1 : nullptr;
-  P.a.phi = I.B.phi[P.cur];
-  P.a.phit = I.B.phit;
-  P.frob = I.frob_log + st;
-  P.frob_zero = I.frob_log;
-  P.nfrob = I.nfrob;
-}
-
-// The segment of a slot that holds slot tile t (the last with first <= t). Every lane runs the same
-// search on the same addresses, so it stays in scalar registers.
-__device__ inline int32_t find_seg(const BatchSeg* segs, int32_t s0, int32_t s1, int64_t t) {
-  int32_t lo = s0, hi = s1 - 1;
-  while (lo < hi) {
-    const int32_t mid = (lo + hi + 1) >> 1;
-    if (segs[mid].first <= t) lo = mid;
-    else hi = mid - 1;
+// The segment of slot segments [s0, s1) that holds slot tile t (the last with first <= t): the lanes compare 64
+// segments at a time, one load deep. (A binary search walked its probes one load after another.)
+__device__ inline int32_t find_seg(const int32_t* __restrict__ first, int32_t s0, int32_t s1, int32_t t) {
+  const int lane = threadIdx.x & 63;
+  int32_t n = 0;
+  for (int32_t s = s0; s < s1; s += 64) {
+    const bool le = first[min(s + lane, s1 - 1)] <= t && s + lane < s1;
+    n += __popcll(__ballot(le));
   }
-  return lo;
+  return __builtin_amdgcn_readfirstlane(s0 + n - 1);
 }
 
-// The step contexts are built on the host with the plan, one per (member, step), and read here through
+// The arguments are resolved on the host with the plan, one PhaseArgs per segment, and read here through
 // a uniform reference into global memory, as the per-phase kernels read theirs from the kernel
 // arguments: in scalar registers. (A context held in LDS is per-lane data to the compiler, which costs
 // the scalar operand bases and doubles the register footprint; one built in registers goes to the
 // stack, as it is indexed at run time. The tile functions are forced inline for the same reason: an
 // out-of-line call passes the context as a per-lane pointer.)
 template <int DMODE, int KMODE, typename TY, typename TPH>
-__global__ __launch_bounds__(kThreads) void stgd_batch_kernel(const StepCtx* __restrict__ ctxs, const BatchSeg* __restrict__ segs,
-                                                         const int32_t* slot_seg, const int64_t* slot_tiles,
-                                                         int32_t nslots) {
+__global__ __launch_bounds__(kThreads) void stgd_batch_kernel(const PhaseArgs* __restrict__ args, const int32_t* __restrict__ first,
+                                                         const int32_t* __restrict__ phase, const int32_t* slot_seg,
+                                                         const int64_t* slot_tiles, int32_t nslots) {
   cg::grid_group grid = cg::this_grid();
   __shared__ StgdSmem sm;
   for (int32_t sl = 0; sl < nslots; ++sl) {
     const int32_t s0 = slot_seg[sl], s1 = slot_seg[sl + 1];
     const int64_t ntiles = slot_tiles[sl];
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-      const BatchSeg sg = segs[find_seg(segs, s0, s1, t)];
-      run_tile<DMODE, KMODE, TY, TPH>(ctxs[sg.ctx], sg.phase, sg.it, (int)(t - sg.first), sm);
+      const int32_t sg = find_seg(first, s0, s1, (int32_t)t);
+      run_tile<DMODE, KMODE, TY, TPH>(args[sg], phase[sg], (int)t - first[sg], sm);
       __syncthreads();
     }
     grid.sync();
@@ -1208,35 +1356,22 @@ __global__ __launch_bounds__(kThreads) void stgd_batch_kernel(const StepCtx* __r
 // One phase slot of the plan as its own launch (blockIdx.x = tile of the slot): the grouped
 // alternative to the persistent kernel, where the kernel boundary orders consecutive slots.
 template <int DMODE, int KMODE, typename TY, typename TPH>
-__global__ __launch_bounds__(kThreads) void stgd_slot_kernel(const StepCtx* __restrict__ ctxs, const BatchSeg* __restrict__ segs, int32_t s0, int32_t s1) {
+__global__ __launch_bounds__(kThreads) void stgd_slot_kernel(const PhaseArgs* __restrict__ args, const int32_t* __restrict__ first,
+                                                        const int32_t* __restrict__ phase, int32_t s0, int32_t s1) {
   __shared__ StgdSmem sm;
-  const int64_t t = blockIdx.x;
-  const BatchSeg sg = segs[find_seg(segs, s0, s1, t)];
-  run_tile<DMODE, KMODE, TY, TPH>(ctxs[sg.ctx], sg.phase, sg.it, (int)(t - sg.first), sm);
+  const int32_t sg = find_seg(first, s0, s1, blockIdx.x);
+  run_tile<DMODE, KMODE, TY, TPH>(args[sg], phase[sg], (int)blockIdx.x - first[sg], sm);
 }
 
 // A slot whose segments are all of one phase, launched with that phase's code only: the generic slot
 // kernel holds every phase and gets the register budget of the largest (one wave per SIMD), this one
 // that of its phase, as the per-phase kernels of single instances.
 template <int DMODE, int KMODE, typename TY, typename TPH, int PHASE>
-__global__ __launch_bounds__(kThreads) void stgd_slot_phase_kernel(const StepCtx* __restrict__ ctxs, const BatchSeg* __restrict__ segs, int32_t s0,
-                                                                  int32_t s1) {
+__global__ __launch_bounds__(kThreads) void stgd_slot_phase_kernel(const PhaseArgs* __restrict__ args, const int32_t* __restrict__ first,
+                                                              int32_t s0, int32_t s1) {
   __shared__ StgdSmem sm;
-  constexpr bool SPLIT = KMODE == MM_BF16X3;
-  const int64_t t = blockIdx.x;
-  const BatchSeg sg = segs[find_seg(segs, s0, s1, t)];
-  const StepCtx& P = ctxs[sg.ctx];
-  const int tile = (int)(t - sg.first);
-  if constexpr (PHASE == PH_SETUP) copy_tile<SPLIT>(P, true, tile, sm);
-  else if constexpr (PHASE == PH_P1) {
-    p1_tile<DMODE, KMODE, TY, TPH>(P, tile, sm);
-    if (tile == 0) p1_log(P);
-  } else if constexpr (PHASE == PH_P2) p2_tile<DMODE, KMODE, TY, TPH>(P, tile, sm);
-  else if constexpr (PHASE == PH_GRAM) gram_tile<KMODE>(P, sg.it, tile, sm);
-  else if constexpr (PHASE == PH_UPDATE) update_tile<KMODE>(P, sg.it, tile, sm);
-  else if constexpr (PHASE == PH_QPOLY) qpoly_tile<KMODE>(P, sg.it, tile, sm);
-  else if constexpr (PHASE == PH_FROB) frob_final(P);
-  else copy_tile<SPLIT>(P, false, tile, sm);
+  const int32_t sg = find_seg(first, s0, s1, blockIdx.x);
+  phase_tile<DMODE, KMODE, TY, TPH, PHASE>(phase_args<PHASE>(args[sg]), (int)blockIdx.x - first[sg], sm);
 }
 
 __global__ void set_i64_kernel(int64_t* p, int64_t v) {
@@ -1278,48 +1413,45 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
                      int& cur, double* frob_log, StgdTiming* timing, const StgdFill& fill, const StgdRenorm& renorm) {
   const int kp = args.kp;
   const int64_t spe = ceil_div(args.n_x, args.bl);
-  StepCtx P{};
-  P.a = args;
-  P.B = B;
-  P.YA = YA;
-  P.YB = YB;
-  P.YCt = YCt;
-  P.ns_iters = ns_iters;
-  P.ns_degree = ns_degree;
+  const StepPlan P{args, B, YA, YB, YCt, ns_iters, ns_degree, KMODE == MM_BF16X3};
+  StopArgs stop{args.stop, 0, args.thresh, args.iter_min, args.iter_max};
+  int64_t yrow0 = 0;
+  int32_t nb = 0;
   auto launch = [&](int phase, int it) -> int {
     const dim3 grid(phase_tiles(phase, kp, args.b)), block(kThreads);
+    const int64_t st = stop.st;
+    const PhaseArgs a = P.resolve(phase, it, cur, yrow0, nb, frob_log + st, st > 0 ? frob_log + st - 1 : nullptr, frob_log, nsteps);
+#define MMSB_PHASE(PH)                                                                                                      \
+  case PH:                                                                                                                  \
+    if (stop.stop)                                                                                                          \
+      hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH, true>), grid, block, 0, s, phase_args<PH>(a), stop);   \
+    else                                                                                                                    \
+      hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH, false>), grid, block, 0, s, phase_args<PH>(a), stop);  \
+    break;
     switch (phase) {
-      case PH_SETUP: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_SETUP>), grid, block, 0, s, P, it); break;
-      case PH_P1: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_P1>), grid, block, 0, s, P, it); break;
-      case PH_P2: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_P2>), grid, block, 0, s, P, it); break;
-      case PH_GRAM: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_GRAM>), grid, block, 0, s, P, it); break;
-      case PH_UPDATE: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_UPDATE>), grid, block, 0, s, P, it); break;
-      case PH_QPOLY: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_QPOLY>), grid, block, 0, s, P, it); break;
-      case PH_QRFIN: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_QRFIN>), grid, block, 0, s, P, it); break;
-      case PH_FROB: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_FROB>), grid, block, 0, s, P, it); break;
-      default: hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_COPY>), grid, block, 0, s, P, it); break;
+      MMSB_PHASE(PH_SETUP)
+      MMSB_PHASE(PH_P1)
+      MMSB_PHASE(PH_P2)
+      MMSB_PHASE(PH_GRAM)
+      MMSB_PHASE(PH_UPDATE)
+      MMSB_PHASE(PH_QPOLY)
+      MMSB_PHASE(PH_QRFIN)
+      MMSB_PHASE(PH_FROB)
+      MMSB_PHASE(PH_COPY)
     }
+#undef MMSB_PHASE
     MMSB_LAUNCH_CHECK();
     return MMSB_OK;
   };
-  P.cur = cur;
-  P.a.phi = B.phi[cur];
-  P.a.phit = B.phit;
-  P.frob_zero = frob_log;
-  P.nfrob = nsteps;
   MMSB_TRY(launch(PH_SETUP, 0));
   for (int64_t st = 0; st < nsteps; ++st) {
     const int64_t gstep = step0 + st;
-    P.cur = cur;
-    P.row0 = (gstep % spe) * args.bl;
-    P.nb = (int32_t)std::min<int64_t>(args.bl, args.n_x - P.row0);
-    P.yrow0 = args.y_window ? 0 : P.row0;
-    P.a.phi = B.phi[cur];
-    P.st = st;
-    P.frob_prev = st > 0 ? frob_log + st - 1 : nullptr;
-    P.frob = frob_log + st;
+    const int64_t row0 = (gstep % spe) * args.bl;
+    nb = (int32_t)std::min<int64_t>(args.bl, args.n_x - row0);
+    yrow0 = args.y_window ? 0 : row0;
+    stop.st = st;
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[0], s));
-    if (args.y_window) MMSB_TRY(fill(P.row0, P.nb));
+    if (args.y_window) MMSB_TRY(fill(row0, nb));
     MMSB_TRY(launch(PH_P1, 0));
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[1], s));
     MMSB_TRY(launch(PH_P2, 0));
@@ -1347,10 +1479,7 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
     }
     cur ^= 1;
   }
-  P.st = nsteps - 1;  // the last step's log entry
-  P.frob = frob_log + nsteps - 1;
-  MMSB_TRY(launch(PH_FROB, 0));
-  return MMSB_OK;
+  return launch(PH_FROB, 0);  // the last step's log entry
 }
 
 static int check_args(const StgdArgs& args, int32_t ns_iters, int32_t ns_degree) {
@@ -1397,8 +1526,9 @@ struct StgdBatch {
   int32_t nslots = 0;
   int32_t grid = 0;
   int32_t grid_max = 0;
-  StepCtx* d_ctx = nullptr;        // [contexts]: one per (member, step)
-  BatchSeg* d_segs = nullptr;      // [segments]
+  PhaseArgs* d_args = nullptr;     // [segments]
+  int32_t* d_first = nullptr;      // [segments]: index of the segment's first tile within its slot
+  int32_t* d_phase = nullptr;      // [segments]
   int32_t* d_slot_seg = nullptr;   // [nslots + 1]: first segment of each slot
   int64_t* d_slot_tiles = nullptr; // [nslots]
   std::vector<int32_t> h_slot_seg;  // host copies for the per-slot launches
@@ -1420,10 +1550,7 @@ int stgd_batch_plan(StgdBatch*& out, int32_t precision, const std::vector<StgdBa
   out = nullptr;
   MMSB_CHECK_ARG(!members.empty(), "stgd batch: no instances");
   MMSB_CHECK_ARG(precision == MMSB_PREC_FP32 || precision == MMSB_PREC_BF16, "stgd batch: unknown precision %d", precision);
-  std::vector<BatchInst> insts(members.size());
   std::vector<std::vector<BatchSeg>> per(members.size());
-  std::vector<StepCtx> ctxs;                  // one per (member, step)
-  std::vector<int64_t> ctx0(members.size());  // each member's first
   for (size_t i = 0; i < members.size(); ++i) {
     const StgdBatchMember& m = members[i];
     MMSB_TRY(check_args(m.args, ns_iters, ns_degree));
@@ -1431,33 +1558,15 @@ int stgd_batch_plan(StgdBatch*& out, int32_t precision, const std::vector<StgdBa
     MMSB_CHECK_ARG(!m.args.stop && !m.args.frob_pre, "stgd batch: instance %zu uses the per-step end test or QR mode", i);
     if (precision == MMSB_PREC_BF16) MMSB_TRY(check_split(m.bufs));
     MMSB_CHECK_ARG(m.nsteps >= 1, "stgd batch: instance %zu has no steps", i);
-    BatchInst& I = insts[i];
-    I.a = m.args;
-    I.B = m.bufs;
-    I.YA = m.YA;
-    I.YB = m.YB;
-    I.YCt = m.YCt;
-    I.cur0 = m.cur;
-    I.ns_iters = ns_iters;
-    I.ns_degree = ns_degree;
-    I.step0 = m.step0;
-    I.spe = ceil_div(m.args.n_x, m.args.bl);
-    I.frob_log = m.frob_log;
-    I.nfrob = m.nsteps;
-    ctx0[i] = (int64_t)ctxs.size();
-    for (int64_t st = 0; st < m.nsteps; ++st) {
-      StepCtx P{};
-      make_step(I, st, P);
-      ctxs.push_back(P);
-    }
+    const StepPlan P{m.args, m.bufs, m.YA, m.YB, m.YCt, ns_iters, ns_degree, precision == MMSB_PREC_BF16};
+    const int64_t spe = ceil_div(m.args.n_x, m.args.bl);
     auto add = [&](int phase, int it, int64_t st) {
-      BatchSeg sg{};
-      sg.inst = (int32_t)i;
+      const int64_t row0 = ((m.step0 + st) % spe) * m.args.bl;
+      BatchSeg sg;
       sg.phase = phase;
-      sg.it = it;
       sg.ntiles = phase_tiles(phase, m.args.kp, m.args.b);
-      sg.step = st;
-      sg.ctx = ctx0[i] + st;
+      sg.args = P.resolve(phase, it, m.cur ^ (int)(st & 1), row0, (int32_t)std::min<int64_t>(m.args.bl, m.args.n_x - row0),
+                          m.frob_log + st, st > 0 ? m.frob_log + st - 1 : nullptr, m.frob_log, m.nsteps);
       per[i].push_back(sg);
     };
     add(PH_SETUP, 0, 0);
@@ -1474,46 +1583,41 @@ int stgd_batch_plan(StgdBatch*& out, int32_t precision, const std::vector<StgdBa
         add(PH_COPY, 0, st);
       }
     }
+    add(PH_FROB, 0, m.nsteps - 1);
   }
-  std::vector<BatchSeg> segs;
+  std::vector<PhaseArgs> args;
+  std::vector<int32_t> first, phases;
   std::vector<int32_t> slot_seg;
   std::vector<int64_t> slot_tiles;
   std::vector<int32_t> slot_phase;
-  // every member's log entry of its last step in one final slot: nothing writes a member's tile
-  // partials after its last step, and the other slots keep one phase each
-  for (size_t i = 0; i < members.size(); ++i) {
-    BatchSeg sg{};
-    sg.inst = (int32_t)i;
-    sg.phase = PH_FROB;
-    sg.ntiles = 1;
-    sg.step = members[i].nsteps - 1;
-    sg.ctx = ctx0[i] + sg.step;
-    per[i].push_back(sg);
-  }
+  // every member's log entry of its last step is the last segment of its list and goes into one final slot: nothing
+  // writes a member's tile partials after its last step, and the other slots keep one phase each
   size_t maxlen = 0;
   for (auto& v : per) maxlen = std::max(maxlen, v.size() - 1);
   for (size_t sl = 0; sl <= maxlen; ++sl) {
-    slot_seg.push_back((int32_t)segs.size());
+    slot_seg.push_back((int32_t)args.size());
     int64_t t = 0;
     int32_t phase = -2;
     for (size_t i = 0; i < per.size(); ++i) {
       const size_t last = per[i].size() - 1;  // the FROB segment
       const size_t at = sl == maxlen ? last : sl;
       if (sl < maxlen && sl >= last) continue;
-      BatchSeg sg = per[i][at];
-      sg.first = t;
+      const BatchSeg& sg = per[i][at];
+      args.push_back(sg.args);
+      first.push_back((int32_t)t);
+      phases.push_back(sg.phase);
       t += sg.ntiles;
-      segs.push_back(sg);
       phase = phase == -2 ? sg.phase : (phase == sg.phase ? phase : -1);
     }
+    MMSB_CHECK_ARG(t < INT32_MAX, "stgd batch: too many tiles in a slot");
     slot_tiles.push_back(t);
     slot_phase.push_back(phase < 0 ? -1 : phase);
   }
-  slot_seg.push_back((int32_t)segs.size());
-  MMSB_CHECK_ARG(segs.size() < (size_t)INT32_MAX, "stgd batch: too many segments");
+  slot_seg.push_back((int32_t)args.size());
+  MMSB_CHECK_ARG(args.size() < (size_t)INT32_MAX, "stgd batch: too many segments");
   auto* b = new StgdBatch();
   b->precision = precision;
-  b->ninst = (int32_t)insts.size();
+  b->ninst = (int32_t)members.size();
   b->nslots = (int32_t)slot_tiles.size();
   b->h_slot_seg = slot_seg;
   b->h_slot_tiles = slot_tiles;
@@ -1523,18 +1627,14 @@ int stgd_batch_plan(StgdBatch*& out, int32_t precision, const std::vector<StgdBa
     return set_error(MMSB_ERR_HIP, "stgd batch: %s", hipGetErrorString(e));
   };
   hipError_t e;
-  if ((e = hipMalloc(&b->d_ctx, sizeof(StepCtx) * ctxs.size())) != hipSuccess) return fail(e);
-  if ((e = hipMalloc(&b->d_segs, sizeof(BatchSeg) * segs.size())) != hipSuccess) return fail(e);
-  if ((e = hipMalloc(&b->d_slot_seg, sizeof(int32_t) * slot_seg.size())) != hipSuccess) return fail(e);
-  if ((e = hipMalloc(&b->d_slot_tiles, sizeof(int64_t) * slot_tiles.size())) != hipSuccess) return fail(e);
-  if ((e = hipMemcpy(b->d_ctx, ctxs.data(), sizeof(StepCtx) * ctxs.size(), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e);
-  if ((e = hipMemcpy(b->d_segs, segs.data(), sizeof(BatchSeg) * segs.size(), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e);
-  if ((e = hipMemcpy(b->d_slot_seg, slot_seg.data(), sizeof(int32_t) * slot_seg.size(), hipMemcpyHostToDevice)) != hipSuccess)
-    return fail(e);
-  if ((e = hipMemcpy(b->d_slot_tiles, slot_tiles.data(), sizeof(int64_t) * slot_tiles.size(), hipMemcpyHostToDevice)) !=
-      hipSuccess)
+  auto put = [](auto** dst, const auto& src) -> hipError_t {
+    const size_t bytes = sizeof(src[0]) * src.size();
+    const hipError_t me = hipMalloc(dst, bytes);
+    return me != hipSuccess ? me : hipMemcpy(*dst, src.data(), bytes, hipMemcpyHostToDevice);
+  };
+  if ((e = put(&b->d_args, args)) != hipSuccess || (e = put(&b->d_first, first)) != hipSuccess ||
+      (e = put(&b->d_phase, phases)) != hipSuccess || (e = put(&b->d_slot_seg, slot_seg)) != hipSuccess ||
+      (e = put(&b->d_slot_tiles, slot_tiles)) != hipSuccess)
     return fail(e);
   int dev = 0, per_cu = 0, cus = 0;
   if ((e = hipGetDevice(&dev)) != hipSuccess) return fail(e);
@@ -1559,7 +1659,7 @@ int32_t stgd_batch_grid_max(const StgdBatch* b) { return b ? b->grid_max : 0; }
 
 int stgd_batch_launch(hipStream_t s, StgdBatch* b) {
   MMSB_CHECK_ARG(b, "stgd batch: null plan");
-  void* args[] = {&b->d_ctx, &b->d_segs, &b->d_slot_seg, &b->d_slot_tiles, &b->nslots};
+  void* args[] = {&b->d_args, &b->d_first, &b->d_phase, &b->d_slot_seg, &b->d_slot_tiles, &b->nslots};
   MMSB_HIP(hipLaunchCooperativeKernel(batch_kernel(b->precision), dim3(b->grid), dim3(kThreads), args, 0, s));
   return MMSB_OK;
 }
@@ -1571,7 +1671,7 @@ static void launch_slot(hipStream_t s, const StgdBatch* b, int32_t sl) {
   switch (b->h_slot_phase[sl]) {
 #define MMSB_SLOT(PH)                                                                                              \
   case PH:                                                                                                         \
-    hipLaunchKernelGGL((stgd_slot_phase_kernel<DMODE, KMODE, TY, TPH, PH>), grid, block, 0, s, b->d_ctx, b->d_segs, s0, s1); \
+    hipLaunchKernelGGL((stgd_slot_phase_kernel<DMODE, KMODE, TY, TPH, PH>), grid, block, 0, s, b->d_args, b->d_first, s0, s1); \
     break;
     MMSB_SLOT(PH_SETUP)
     MMSB_SLOT(PH_P1)
@@ -1583,7 +1683,7 @@ static void launch_slot(hipStream_t s, const StgdBatch* b, int32_t sl) {
     MMSB_SLOT(PH_FROB)
 #undef MMSB_SLOT
     default:  // segments of different phases
-      hipLaunchKernelGGL((stgd_slot_kernel<DMODE, KMODE, TY, TPH>), grid, block, 0, s, b->d_ctx, b->d_segs, s0, s1);
+      hipLaunchKernelGGL((stgd_slot_kernel<DMODE, KMODE, TY, TPH>), grid, block, 0, s, b->d_args, b->d_first, b->d_phase, s0, s1);
   }
 }
 
@@ -1599,8 +1699,9 @@ int stgd_batch_launch_slots(hipStream_t s, StgdBatch* b) {
 
 void stgd_batch_free(StgdBatch* b) {
   if (!b) return;
-  (void)hipFree(b->d_ctx);
-  (void)hipFree(b->d_segs);
+  (void)hipFree(b->d_args);
+  (void)hipFree(b->d_first);
+  (void)hipFree(b->d_phase);
   (void)hipFree(b->d_slot_seg);
   (void)hipFree(b->d_slot_tiles);
   delete b;

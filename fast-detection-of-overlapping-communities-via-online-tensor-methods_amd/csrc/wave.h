@@ -11,7 +11,13 @@
 
 namespace mmsb {
 
-enum { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRor4 = 0x124, kDppRor8 = 0x128 };
+// kDppHalfMirror reverses each group of 8 lanes: once the values of a quad agree, lane 7 - i holds what lane i ^ 4 does.
+enum { kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppRor4 = 0x124, kDppRor8 = 0x128, kDppHalfMirror = 0x141 };
+
+template <int CTRL>
+__device__ inline float dpp_mov(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
+}
 
 __device__ inline uint32_t lo32(double v) { return (uint32_t)__builtin_bit_cast(uint64_t, v); }
 __device__ inline uint32_t hi32(double v) { return (uint32_t)(__builtin_bit_cast(uint64_t, v) >> 32); }
@@ -43,6 +49,18 @@ __device__ inline double swap_add16(double p, double q) {
   return join32(l[0], h[0]) + join32(l[1], h[1]);
 }
 
+__device__ inline float swap_add32(float p, float q) {
+#pragma clang fp contract(off)
+  const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, q), false, false);
+  return __builtin_bit_cast(float, (uint32_t)x[0]) + __builtin_bit_cast(float, (uint32_t)x[1]);
+}
+
+__device__ inline float swap_add16(float p, float q) {
+#pragma clang fp contract(off)
+  const auto x = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(uint32_t, p), __builtin_bit_cast(uint32_t, q), false, false);
+  return __builtin_bit_cast(float, (uint32_t)x[0]) + __builtin_bit_cast(float, (uint32_t)x[1]);
+}
+
 __device__ inline double row_sum(double v) {  // over the row's 16 lanes
 #pragma clang fp contract(off)
   v += dpp_mov<kDppRor8>(v);
@@ -59,6 +77,32 @@ __device__ inline void wave_sum3(double& a, double& b, double& c) {
   a = read_lane(v, 0);
   c = read_lane(v, 16);
   b = read_lane(v, 32);
+}
+
+__device__ inline double wave_sum(double v) { return row_sum(swap_add16(swap_add32(v, v), swap_add32(v, v))); }
+
+// The largest of the wave's values (not negative).
+__device__ inline double wave_max(double v) {
+  v = fmax(v, dpp_mov<kDppRor8>(v));
+  v = fmax(v, dpp_mov<kDppRor4>(v));
+  v = fmax(v, dpp_mov<kDppXor2>(v));
+  v = fmax(v, dpp_mov<kDppXor1>(v));
+  return fmax(fmax(read_lane(v, 0), read_lane(v, 16)), fmax(read_lane(v, 32), read_lane(v, 48)));
+}
+
+// Sums over the lanes of a quad, and of a group of eight (offsets 1, 2, 4).
+__device__ inline float quad_sum(float v) {
+#pragma clang fp contract(off)
+  v += dpp_mov<kDppXor1>(v);
+  v += dpp_mov<kDppXor2>(v);
+  return v;
+}
+
+__device__ inline float oct_sum(float v) {
+#pragma clang fp contract(off)
+  v = quad_sum(v);
+  v += dpp_mov<kDppHalfMirror>(v);
+  return v;
 }
 
 }  // namespace mmsb
