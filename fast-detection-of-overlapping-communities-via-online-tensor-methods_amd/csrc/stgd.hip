@@ -407,10 +407,11 @@ __device__ inline void put4(float* f32, uint16_t* s16, int64_t nel, int64_t off,
 
 // Inputs of finish_tile that do not depend on the tile's products, loaded before the MFMA loop so
 // that their latency overlaps the operand loads: the previous iterate's block values (for the frob
-// log) and mu_A, mu_B of the thread's row (for the m partial sums).
+// log) and mu_A, mu_B of the thread's row (for the m partial sums; as loaded -- a conversion before the loop would
+// wait for them ahead of the operand loads).
 struct TilePre {
   float pv[4];
-  float ua, ub;
+  double ua, ub;
 };
 
 __device__ inline void tile_pre(TilePre& t, int kp, int64_t i0, int64_t j0, const float* prev, const double* mu_a,
@@ -425,9 +426,16 @@ __device__ inline void tile_pre(TilePre& t, int kp, int64_t i0, int64_t j0, cons
     t.pv[3] = p.w;
   }
   if (mu_a) {
-    t.ua = (float)mu_a[i0 + r];
-    t.ub = (float)mu_b[i0 + r];
+    t.ua = mu_a[i0 + r];
+    t.ub = mu_b[i0 + r];
   }
+}
+
+// Keeps what is computed from a value loaded early behind this point (the compiler would move it up to the load,
+// and the wait for it ahead of the operand loads).
+template <typename T>
+__device__ inline void late(T& v) {
+  asm volatile("" : "+v"(v));
 }
 
 // Shared memory of the tile epilogue.
@@ -447,7 +455,7 @@ struct TileShm {
 // kernel waits for is their way to memory, under which the sums are taken.
 template <bool SPLIT>
 __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64_t j0, const float v[4], float* Out,
-                                   uint16_t* Out16, float* OutT, uint16_t* OutT16, const TilePre& pre, double* fslot,
+                                   uint16_t* Out16, float* OutT, uint16_t* OutT16, TilePre& pre, double* fslot,
                                    float* mpart) {
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
@@ -479,11 +487,13 @@ __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64
   if (act && mpart) {
     // lanes with equal lane % 8 hold the same columns: their eight rows are summed over offsets 8, 16, 32, the last
     // two packed (the odd rows of 16 lanes carry s = B, the upper half the columns 2 and 3)
+    late(pre.ua);
+    late(pre.ub);
+    const float ua = (float)pre.ua, ub = (float)pre.ub;
     float q[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float pa = pre.ua * v[e], pb = pre.ub * v[e];
-      const float sa = fmaf(pre.ua, v[e], dpp_mov<kDppRor8>(pa)), sb = fmaf(pre.ub, v[e], dpp_mov<kDppRor8>(pb));
+      const float sa = fmaf(ua, v[e], dpp_mov<kDppRor8>(ua * v[e])), sb = fmaf(ub, v[e], dpp_mov<kDppRor8>(ub * v[e]));
       q[e] = swap_add16(sa, sb);
     }
     const float s01 = swap_add32(q[0], q[2]), s23 = swap_add32(q[1], q[3]);
@@ -862,13 +872,14 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
   PartSum ps;  // column sums of P_A o P_B and m_A, m_B for c_mu, gathered during the MFMA loop
   const bool epi = epi_thread();
   const int r = threadIdx.x >> 3, c4 = 4 * (threadIdx.x & 7);
-  float mab_a = 0.f, mab_b = 0.f, muc = 0.f;
+  float mab_a = 0.f, mab_b = 0.f;
+  double muc_d = 0.0;  // converted after the MFMA loop
   float4 ph = make_float4(0.f, 0.f, 0.f, 0.f);
   if (epi) {  // epilogue inputs, loaded ahead of the MFMA loop
     cspart_load(ps, a.cs_part, kp, a.b / 32, j0);
     mab_a = a.mab[j0 + (threadIdx.x >> 3)];
     mab_b = a.mab[kp + j0 + (threadIdx.x >> 3)];
-    muc = (float)a.mu_c[i0 + r];
+    muc_d = a.mu_c[i0 + r];
     ph = *reinterpret_cast<const float4*>(a.phi + (i0 + r) * kp + j0 + c4);
   }
   // waves with (w & 2) == 0 take Phi H, the others Y_C^T C_g, each over kWaves / 2 parts of its range;
@@ -895,7 +906,8 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
     for (int t = threadIdx.x; t < kp; t += blockDim.x) a.rowsum[t] = 0ull;
   red_put(red, acc);
   __syncthreads();
-  const float eta = a.eta, inv_b = 1.f / (float)a.nb;
+  late(muc_d);
+  const float eta = a.eta, inv_b = 1.f / (float)a.nb, muc = (float)muc_d;
   const float p0[4] = {ph.x, ph.y, ph.z, ph.w};
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (epi) {
@@ -932,11 +944,14 @@ __device__ inline void guard_load(unsigned long long rs[8], const unsigned long 
   for (int u = 0; u < 8; ++u) rs[u] = rowsum[min(lane + 64 * u, kp - 1)];
 }
 
-__device__ inline void guard_scale(const unsigned long long rs[8], const unsigned long long* rowsum, int kp, float* cscale) {
+__device__ inline void guard_scale(unsigned long long rs[8], const unsigned long long* rowsum, int kp, float* cscale) {
   const int lane = threadIdx.x & 63;
   unsigned long long m = 0;
 #pragma unroll
-  for (int u = 0; u < 8; ++u) m = rs[u] > m ? rs[u] : m;
+  for (int u = 0; u < 8; ++u) {
+    late(rs[u]);
+    m = rs[u] > m ? rs[u] : m;
+  }
   for (int t = lane + 512; t < kp; t += 64) m = rowsum[t] > m ? rowsum[t] : m;
   const float mx = (float)(wave_max((double)m) * 2.3283064365386963e-10);
   if (lane == 0) *cscale = mx > 2.f ? sqrtf(2.f / mx) : 1.f;
