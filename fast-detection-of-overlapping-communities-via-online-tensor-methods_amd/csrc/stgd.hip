@@ -127,9 +127,8 @@ __device__ inline u32x4* wave_stage() {
   return buf[wave_id()];
 }
 
-// Rearranges a block loaded by stage_load into the MFMA layout, in place.
-__device__ inline void stage_swap(u32x4 v[4]) {
-  u32x4* buf = wave_stage();
+// Rearranges a block loaded by stage_load into the MFMA layout, in place, through the wave's buffer.
+__device__ inline void stage_swap(u32x4 v[4], u32x4* buf) {
   const int lane = threadIdx.x & 63;
   const int q = lane >> 3, s = lane & 7, r = lane & 31, h = lane >> 5;
 #pragma unroll
@@ -142,6 +141,8 @@ __device__ inline void stage_swap(u32x4 v[4]) {
   for (int c = 0; c < 4; ++c) v[c] = buf[r * 8 + ((2 * c + h) ^ ((r >> 1) & 7))];
   asm volatile("" ::: "memory");  // ... and the next block's writes follow these reads
 }
+
+__device__ inline void stage_swap(u32x4 v[4]) { stage_swap(v, wave_stage()); }
 
 __device__ inline floatx4 as_f32(const u32x4& v) { return __builtin_bit_cast(floatx4, v); }
 __device__ inline bf16x8 as_bf16(const u32x4& v) { return __builtin_bit_cast(bf16x8, v); }
@@ -389,6 +390,7 @@ __device__ inline float red_sum4(const Red4& R, int r, int c) {
 // SPLIT, the (hi, lo) BF16 pair stored as [hi | lo] blocks of nel elements each (if s16).
 template <bool SPLIT>
 __device__ inline void put4(float* f32, uint16_t* s16, int64_t nel, int64_t off, const float v[4]) {
+#pragma clang fp contract(off)  // lo is of the rounded v, also where v is a product
   if (f32) *reinterpret_cast<float4*>(f32 + off) = make_float4(v[0], v[1], v[2], v[3]);
   if constexpr (SPLIT) {
     if (s16) {
@@ -510,6 +512,27 @@ __device__ inline void finish_tile(TileShm& S, int kp, int ti, int64_t i0, int64
     mpart[((int64_t)ti * 2 + s) * kp + j0 + c] = (S.m[0][s][c] + S.m[1][s][c]) + (S.m[2][s][c] + S.m[3][s][c]);
   }
 }
+
+// ---- the element-wise formulas of the phases, with their roundings fixed (every form of a phase gives the same bits)
+__device__ inline float cg_value(float c3, float c1, float p, float q, float ab, float mA, float mB) {
+  return fmaf(c3, ab, c1 * fmaf(p, mB, mA * q));
+}
+__device__ inline float cmu_value(float c0, float c1, float mA, float mB, float ssum, int nb) {
+  return fmaf(c0 * mA, mB, c1 * ssum / (float)nb);
+}
+__device__ inline float step_value(float p0, float eta, float theta, float phh, float t, float inv_b, float muc, float cmu) {
+  return fmaf(eta, fmaf(t, inv_b, muc * cmu), fmaf(-(eta * theta), phh, p0));
+}
+__device__ inline float update_value(float cs, bool quintic, float x, float y) {
+  const float c1 = (quintic ? 1.875f : 1.5f) * cs, c3 = quintic ? cs : -0.5f * cs * cs * cs;
+  return fmaf(c1, x, c3 * y);
+}
+__device__ inline float qpoly_value(float cs, float g, float gg) {
+  const float c2 = cs * cs;
+  const float a1 = -1.25f * c2, a2 = 0.375f * c2 * c2;
+  return fmaf(a2, gg, a1 * g);
+}
+__device__ inline float guard_value(float mx) { return mx > 2.f ? sqrtf(2.f / mx) : 1.f; }
 
 template <typename T>
 __device__ inline void store4(T* p, const float v[4]) {
@@ -807,7 +830,7 @@ __device__ __forceinline__ void p1_tile(const P1Args& a, int tile, StgdSmem& sm,
       const bool valid = (x0 + r) < a.nb;
       const float ab = p * q;
       cs += valid ? ab : 0.f;
-      cg[e] = valid ? a.c3 * ab + a.c1 * (p * mB + mA * q) : 0.f;
+      cg[e] = valid ? cg_value(a.c3, a.c1, p, q, ab, mA, mB) : 0.f;
     }
     store4(static_cast<TPH*>(a.cgt) + (j0 + c) * (int64_t)a.b + x0 + r4, cg);
     cs = oct_sum(cs);
@@ -900,14 +923,14 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
   if (epi) {
     const int c = threadIdx.x >> 3;
     const float ssum = cspart_reduce(ps, a.cs_part, kp, a.b / 32, j0);
-    if ((threadIdx.x & 7) == 0) sm.p2.cmu[c] = a.c0 * mab_a * mab_b + a.c1 * ssum / (float)a.nb;
+    if ((threadIdx.x & 7) == 0) sm.p2.cmu[c] = cmu_value(a.c0, a.c1, mab_a, mab_b, ssum, a.nb);
   }
   if (tile == 0)
     for (int t = threadIdx.x; t < kp; t += blockDim.x) a.rowsum[t] = 0ull;
   red_put(red, acc);
   __syncthreads();
   late(muc_d);
-  const float eta = a.eta, inv_b = 1.f / (float)a.nb, muc = (float)muc_d;
+  const float inv_b = 1.f / (float)a.nb, muc = (float)muc_d;
   const float p0[4] = {ph.x, ph.y, ph.z, ph.w};
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (epi) {
@@ -916,7 +939,7 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
       const int c = c4 + e;
       const float phh = red_get(red, 0, r, c) + red_get(red, 1, r, c);
       const float t = red_get(red, 2, r, c) + red_get(red, 3, r, c);
-      v[e] = p0[e] - eta * a.theta * phh + eta * (t * inv_b + muc * sm.p2.cmu[c]);
+      v[e] = step_value(p0[e], a.eta, a.theta, phh, t, inv_b, muc, sm.p2.cmu[c]);
     }
   }
   TilePre pre{};  // the reference's log: ||Phi~ - Phi||^2 before the renormalisation
@@ -954,7 +977,7 @@ __device__ inline void guard_scale(unsigned long long rs[8], const unsigned long
   }
   for (int t = lane + 512; t < kp; t += 64) m = rowsum[t] > m ? rowsum[t] : m;
   const float mx = (float)(wave_max((double)m) * 2.3283064365386963e-10);
-  if (lane == 0) *cscale = mx > 2.f ? sqrtf(2.f / mx) : 1.f;
+  if (lane == 0) *cscale = guard_value(mx);
 }
 
 // G = X^T X of a Newton-Schulz iteration on upper-triangle tile `tile` (block and mirror), and
@@ -1026,12 +1049,11 @@ __device__ __forceinline__ void qpoly_tile(const QpolyArgs& a, int tile, StgdSme
   red_put(red, acc);
   __syncthreads();
   if (!epi_thread()) return;
-  const float c2 = sm.p2.cscale * sm.p2.cscale;
-  const float a1 = -1.25f * c2, a2 = 0.375f * c2 * c2;
+  const float cs = sm.p2.cscale;
   const float gg[4] = {gv.x, gv.y, gv.z, gv.w};
   float v[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = a1 * gg[e] + a2 * red_sum4(red, r, c4 + e);
+  for (int e = 0; e < 4; ++e) v[e] = qpoly_value(cs, gg[e], red_sum4(red, r, c4 + e));
   put4<SPLIT>(a.q, a.q16, nel, (i0 + r) * kp + j0 + c4, v);
 }
 
@@ -1064,12 +1086,11 @@ __device__ __forceinline__ void update_tile(const UpdateArgs& a, int tile, StgdS
   red_put(red, acc);
   __syncthreads();
   const float cs = sm.p2.cscale;
-  const float c1 = (quintic ? 1.875f : 1.5f) * cs, c3 = quintic ? cs : -0.5f * cs * cs * cs;
   const float x[4] = {xv.x, xv.y, xv.z, xv.w};
   float v[4] = {0.f, 0.f, 0.f, 0.f};
   if (epi_thread())
 #pragma unroll
-    for (int e = 0; e < 4; ++e) v[e] = c1 * x[e] + c3 * red_sum4(red, r, c4 + e);
+    for (int e = 0; e < 4; ++e) v[e] = update_value(cs, quintic, x[e], red_sum4(red, r, c4 + e));
   finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, a.out, a.out16, a.outT, a.outT16, pre, a.fpart ? a.fpart + tile : nullptr,
                      a.mpart);
 }
@@ -1152,7 +1173,7 @@ __device__ inline bool stop_test(const StopArgs& a, int64_t t, double f) {
 // was set by a sibling workgroup, and workgroup 0 must still store the entry. The skipped kernels
 // write nothing, and the host reads stop_at after the run.
 template <int DMODE, int KMODE, typename TY, typename TPH, int PHASE, bool STOP>
-__global__ __launch_bounds__(kThreads) void stgd_phase_kernel(typename ArgsOf<PHASE>::type a, StopArgs s) {
+__global__ __launch_bounds__(kThreads, PHASE == PH_P1 ? 3 : 1) void stgd_phase_kernel(typename ArgsOf<PHASE>::type a, StopArgs s) {
   __shared__ StgdSmem sm;
   if constexpr (STOP && PHASE != PH_SETUP) {
     const int64_t g = s.stop->base + s.st;
@@ -1172,6 +1193,466 @@ __global__ __launch_bounds__(kThreads) void stgd_phase_kernel(typename ArgsOf<PH
     }
   }
   phase_tile<DMODE, KMODE, TY, TPH, PHASE>(a, blockIdx.x, sm, !STOP);
+}
+
+// ---- whole runs of a small instance in one workgroup ---------------------------------------------------
+// With k <= 32 every k x k matrix is one 32 x 32 block, and a step of the phase kernels is six dependent launches of
+// a few workgroups each, 25-30 us of launch and memory latency around about 1 us of work. Here one workgroup of
+// eight waves runs all steps of a launch with Phi and the matrices derived from it in LDS and four barriers per
+// step; the sums are those of the phase kernels, term by term (MFMA over the same k order, partial sums over the
+// same halves of the minibatch, the epilogues' butterflies), so Phi and the log are bit-identical. Products with
+// the zero padding beyond k are left out (they add exact zeros).
+//   waves 0..3  P_A, P_B and C_g of the minibatch's 32-row tiles (tiles w, w + 4, ..); then, each for eight rows,
+//               Phi~ from the summed products
+//   wave 4      (Phi^T Phi)^o2 and Phi H; then the Newton-Schulz iterations alone, without barriers
+//   waves 5, 6  Y_C^T C_g over the two halves of the minibatch
+//   wave 7      c_mu; the log entry of the previous step
+// The rows of Y of the next step are loaded during the Newton-Schulz iterations. One compute unit bounds the
+// minibatch: b = 512 takes about 9 us per step, beyond it (and beyond the LDS that holds C_g) the phase kernels
+// spread the work. SMALLMEAS
+constexpr int kSmallB = 512;        // largest padded minibatch
+constexpr int kSmallThreads = 512;
+
+struct SmallArgs {
+  const void *ya, *yb, *yct;        // all rows of X
+  const double *mu_a, *mu_b, *mu_c;
+  const float* phi_in;
+  float* phi_out;
+  double* frob;                     // [nsteps]
+  int64_t step0, nsteps, spe, n_x, n_pad;
+  int32_t k, kp, b, bl, ns_iters, quintic, renorm_every;
+  float c3, c1, c0, eta, theta;
+};
+
+// A 32 x 32 operand in LDS: rows along the reduction index, FP32 or a split BF16 pair. The row strides put the 16-byte
+// pieces of 16 consecutive rows on distinct banks.
+template <int MODE>
+struct SmallMat {
+  float v[32][36];
+};
+template <>
+struct SmallMat<MM_BF16X3> {
+  __bf16 hi[32][40];
+  __bf16 lo[32][40];
+};
+
+__device__ inline void small_put(SmallMat<MM_F32>& m, int r, int c, float x) { m.v[r][c] = x; }
+__device__ inline void small_put(SmallMat<MM_BF16X3>& m, int r, int c, float x) {
+#pragma clang fp contract(off)  // lo is of the rounded x, also where x is a product
+  const __bf16 hi = (__bf16)x;
+  m.hi[r][c] = hi;
+  m.lo[r][c] = (__bf16)(x - (float)hi);
+}
+__device__ inline void small_put4(SmallMat<MM_F32>& m, int r, int c, const float x[4]) {
+  *reinterpret_cast<float4*>(&m.v[r][c]) = make_float4(x[0], x[1], x[2], x[3]);
+}
+__device__ inline void small_put4(SmallMat<MM_BF16X3>& m, int r, int c, const float x[4]) {
+#pragma clang fp contract(off)
+  bf16x4 hi, lo;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    hi[e] = (__bf16)x[e];
+    lo[e] = (__bf16)(x[e] - (float)hi[e]);
+  }
+  *reinterpret_cast<bf16x4*>(&m.hi[r][c]) = hi;
+  *reinterpret_cast<bf16x4*>(&m.lo[r][c]) = lo;
+}
+
+// A product of an operand with itself, from accumulator layout, as an operand of its rows. In FP32 it is symmetric to
+// the bit, so a lane stores its column as a row, four values at a time; the split form takes hi.lo before lo.hi
+// and is not.
+template <int MODE>
+__device__ inline void small_put_sym(SmallMat<MODE>& m, const float v[16]) {
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (MODE == MM_F32) {
+      small_put4(m, c, 8 * q + 4 * h, v + 4 * q);
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) small_put(m, 8 * q + 4 * h + e, c, v[4 * q + e]);
+    }
+  }
+}
+
+// A B^T over the first k columns of two operands; +0 added as the phase kernels' sums over empty parts do.
+__device__ inline floatx16 small_mm(const SmallMat<MM_F32>& A, const SmallMat<MM_F32>& B, int k) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  floatx16 acc = {};
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (8 * c < k) {
+      const floatx4 x = *reinterpret_cast<const floatx4*>(&A.v[r][8 * c + 4 * h]);
+      const floatx4 y = *reinterpret_cast<const floatx4*>(&B.v[r][8 * c + 4 * h]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+    }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] += 0.f;
+  return acc;
+}
+__device__ inline floatx16 small_mm(const SmallMat<MM_BF16X3>& A, const SmallMat<MM_BF16X3>& B, int k) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  floatx16 acc = {};
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (16 * c < k) {
+      const bf16x8 xh = *reinterpret_cast<const bf16x8*>(&A.hi[r][16 * c + 8 * h]);
+      const bf16x8 xl = *reinterpret_cast<const bf16x8*>(&A.lo[r][16 * c + 8 * h]);
+      const bf16x8 yh = *reinterpret_cast<const bf16x8*>(&B.hi[r][16 * c + 8 * h]);
+      const bf16x8 yl = *reinterpret_cast<const bf16x8*>(&B.lo[r][16 * c + 8 * h]);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, yh, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, yl, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xl, yh, acc, 0, 0, 0);
+    }
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] += 0.f;
+  return acc;
+}
+
+// acc += (a block of 32 data rows in MFMA layout) Phi over the first k columns.
+__device__ inline void small_data_mm(floatx16& acc, const u32x4 a[4], const SmallMat<MM_F32>& B, int k) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (8 * c < k) {
+      const floatx4 x = as_f32(a[c]), y = *reinterpret_cast<const floatx4*>(&B.v[r][8 * c + 4 * h]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+    }
+}
+__device__ inline void small_data_mm(floatx16& acc, const u32x4 a[4], const SmallMat<MM_BF16X3>& B, int k) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (16 * c < k)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(a[c]), *reinterpret_cast<const bf16x8*>(&B.hi[r][16 * c + 8 * h]), acc, 0, 0, 0);
+}
+
+// acc += (a block of Y_C^T in MFMA layout) C_g over the group's first n columns x (rows of the minibatch; C_g is zero
+// beyond them); cg points at the group's first column of C_g^T, row stride ld.
+__device__ inline void small_cg_mm(floatx16& acc, const u32x4 a[4], const float* cg, int ld, int n) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (8 * c < n) {
+      const floatx4 x = as_f32(a[c]), y = *reinterpret_cast<const floatx4*>(cg + r * ld + 8 * c + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+    }
+}
+__device__ inline void small_cg_mm(floatx16& acc, const u32x4 a[4], const __bf16* cg, int ld, int n) {
+  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (16 * c < n)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(a[c]), *reinterpret_cast<const bf16x8*>(cg + r * ld + 16 * c + 8 * h), acc, 0, 0, 0);
+}
+
+template <int MODE>
+struct SmallShm {
+  SmallMat<MODE> phi, phiT, H, x, xT, g, q;
+  float phif[2][32][36];     // Phi in FP32, this step's and the next
+  float xf[32][36];          // the Newton-Schulz iterate in FP32
+  float slot[3][16][64];     // Phi H and the halves of Y_C^T C_g, in accumulator layout
+  float cs[kSmallB / 32][32];
+  float mu[2][32];           // mu_A, mu_B
+  float mv[2][32];           // m_A, m_B
+  float cmu[32];
+  u32x4 stage[8][256];       // per-wave transpose buffers
+  typedef typename std::conditional<MODE == MM_F32, float, __bf16>::type T;
+  alignas(16) T cgt[1];      // [32][b + 16 bytes]
+};
+
+template <int MODE>
+static size_t small_shm_bytes(int b) {
+  typedef typename SmallShm<MODE>::T T;
+  return sizeof(SmallShm<MODE>) + sizeof(T) * 32 * (size_t)(b + 16 / sizeof(T));
+}
+
+// The new Phi as the wave that holds it in accumulator layout (v[i] = element (8 (i / 4) + 4 h + i % 4, lane % 32)):
+// its operands, FP32 copy and the sums m_s = mu_s^T Phi (rows in pairs, fours and eights, then the four groups of
+// eight, as finish_tile takes them).
+template <int MODE>
+__device__ inline void small_new_phi(SmallShm<MODE>& S, int buf, const float v[16]) {
+  const int lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  float ma[4], mb[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float* x = v + 4 * q;
+    small_put4(S.phiT, c, 8 * q + 4 * h, x);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      small_put(S.phi, 8 * q + 4 * h + e, c, x[e]);
+      S.phif[buf][8 * q + 4 * h + e][c] = x[e];
+    }
+    const float* u = &S.mu[0][8 * q + 4 * h];
+    const float* w = &S.mu[1][8 * q + 4 * h];
+    float sa, sb;
+    {
+#pragma clang fp contract(off)
+      sa = fmaf(u[0], x[0], u[1] * x[1]) + fmaf(u[2], x[2], u[3] * x[3]);
+      sb = fmaf(w[0], x[0], w[1] * x[1]) + fmaf(w[2], x[2], w[3] * x[3]);
+    }
+    ma[q] = swap_add32(sa, sa);
+    mb[q] = swap_add32(sb, sb);
+  }
+  if (h == 0) {
+    S.mv[0][c] = (ma[0] + ma[1]) + (ma[2] + ma[3]) + 0.f;
+    S.mv[1][c] = (mb[0] + mb[1]) + (mb[2] + mb[3]) + 0.f;
+  }
+}
+
+template <int MODE, typename TY>
+__global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs a) {
+  extern __shared__ __attribute__((aligned(16))) unsigned char small_raw[];
+  SmallShm<MODE>& S = *reinterpret_cast<SmallShm<MODE>*>(small_raw);
+  typedef typename SmallShm<MODE>::T T;
+  constexpr int G = MODE == MM_F32 ? 32 : 64;  // minibatch rows of one Y_C^T group
+  constexpr int PF = 4;                        // groups in flight per wave
+  const int w = wave_id(), lane = threadIdx.x & 63, c = lane & 31, h = lane >> 5;
+  const int kp = a.kp, b = a.b, k = a.k, nt = b / 32, ldc = b + 16 / (int)sizeof(T);
+  const TY* ya = static_cast<const TY*>(a.ya);
+  const TY* yb = static_cast<const TY*>(a.yb);
+  const TY* yct = static_cast<const TY*>(a.yct);
+  u32x4* stage = S.stage[w];
+  T* cgt = S.cgt;
+
+  auto rows_of = [&](int64_t st, int64_t& row0, int& nb) {
+    row0 = ((a.step0 + st) % a.spe) * a.bl;
+    nb = (int)min((int64_t)a.bl, a.n_x - row0);
+  };
+  u32x4 pre[PF][4];                            // rows ahead: two tiles of Y_A, Y_B (waves 0..3), PF groups of Y_C^T
+  u32x4 (&ra)[4] = pre[0], (&rb)[4] = pre[1];
+  const int part = w - 5, ng = b / G;          // waves 5, 6: groups [g0, g1)
+  const int g0 = w >= 5 ? ng * part / 2 : 0, g1 = w >= 5 ? ng * (part + 1) / 2 : 0;
+  auto load_tile = [&](int64_t row0, int tile) {
+    stage_load<true>(ra, ya + (row0 + 32 * tile) * kp, kp);
+    stage_load<true>(rb, yb + (row0 + 32 * tile) * kp, kp);
+  };
+  auto load_group = [&](u32x4 (&y)[4], int64_t row0, int g) {
+    const TY* p = yct + row0 + (int64_t)g * G;
+    if (row0 % (16 / (int64_t)sizeof(TY)) == 0) stage_load<true>(y, p, a.n_pad);
+    else stage_load<false>(y, p, a.n_pad);
+  };
+  auto prefetch = [&](int64_t st) {
+    if (st >= a.nsteps) return;
+    int64_t row0;
+    int nb;
+    rows_of(st, row0, nb);
+    if (w < 4) {
+      if (w < nt) load_tile(row0, w);
+    } else if (w == 5 || w == 6) {
+#pragma unroll
+      for (int u = 0; u < PF; ++u)
+        if (g0 + u < g1) load_group(pre[u], row0, g0 + u);
+    }
+  };
+
+  // log entry of step st: Phi in buffer `now` against the other, summed as the four waves of finish_tile do (rows 8 q ..,
+  // four columns per lane)
+  auto log_entry = [&](int64_t st, int now) {
+    double f[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int r = 8 * q + (lane >> 3), c4 = 4 * (lane & 7);
+      double d = 0.0;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const double dd = (double)S.phif[now][r][c4 + e] - (double)S.phif[now ^ 1][r][c4 + e];
+        d = fma(dd, dd, d);
+      }
+      f[q] = wave_sum(d);
+    }
+    if (lane == 0) a.frob[st] = (f[0] + f[1]) + (f[2] + f[3]);
+  };
+
+  float uc[4];                                 // waves 0..3: mu_C of their rows
+  if (w < 4)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) uc[e] = (float)a.mu_c[8 * w + 4 * h + e];
+  if (w == 4) {
+    S.mu[h][c] = (float)(h ? a.mu_b[c] : a.mu_a[c]);
+    asm volatile("" ::: "memory");
+    float v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = a.phi_in[(8 * (i >> 2) + 4 * h + (i & 3)) * kp + c];
+    small_new_phi<MODE>(S, 0, v);
+  }
+  prefetch(0);
+  __syncthreads();
+
+  int cur = 0;
+  for (int64_t st = 0; st < a.nsteps; ++st) {
+    int64_t row0;
+    int nb;
+    rows_of(st, row0, nb);
+    // P_A, P_B, C_g; (Phi^T Phi)^o2; the previous step's log entry
+    if (w < 4) {
+      const float mA = S.mv[0][c], mB = S.mv[1][c];
+      for (int tile = w; tile < nt; tile += 4) {
+        u32x4 xa[4], xb[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          xa[i] = ra[i];
+          xb[i] = rb[i];
+        }
+        if (tile + 4 < nt) load_tile(row0, tile + 4);
+        stage_swap(xa, stage);
+        stage_swap(xb, stage);
+        floatx16 pa = {}, pb = {};
+        small_data_mm(pa, xa, S.phiT, k);
+        small_data_mm(pb, xb, S.phiT, k);
+        float t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float cg[4], cs = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const int x = 32 * tile + 8 * q + 4 * h + e;
+            const float p = pa[4 * q + e] + 0.f, r = pb[4 * q + e] + 0.f;
+            const bool valid = x < nb;
+            const float ab = p * r;
+            {
+#pragma clang fp contract(off)
+              cs += valid ? ab : 0.f;
+            }
+            cg[e] = valid ? cg_value(a.c3, a.c1, p, r, ab, mA, mB) : 0.f;
+          }
+          store4(cgt + c * ldc + 32 * tile + 8 * q + 4 * h, cg);
+          t[q] = swap_add32(cs, cs);
+        }
+        if (h == 0) S.cs[tile][c] = (t[0] + t[1]) + (t[2] + t[3]);
+      }
+    } else if (w == 4) {
+      const floatx16 g = small_mm(S.phiT, S.phiT, k);
+      float v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = g[i] * g[i];
+      small_put_sym<MODE>(S.H, v);
+    } else if (w == 7 && st > 0) {
+      log_entry(st - 1, cur);
+    }
+    __syncthreads();
+    // Phi H, the halves of Y_C^T C_g, c_mu
+    if (w == 4) {
+      const floatx16 v = small_mm(S.phi, S.H, k);
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S.slot[0][i][lane] = v[i];
+    } else if (w == 5 || w == 6) {
+      floatx16 acc = {};
+      for (int g = g0; g < g1; g += PF) {
+#pragma unroll
+        for (int u = 0; u < PF; ++u) {
+          if (g + u < g1) {
+            stage_swap(pre[u], stage);
+            small_cg_mm(acc, pre[u], cgt + (g + u) * G, ldc, nb - (g + u) * G);
+            if (g + u + PF < g1) load_group(pre[u], row0, g + u + PF);
+          }
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < 16; ++i) S.slot[w - 4][i][lane] = acc[i];
+    } else if (w == 7) {
+      float m[8];
+#pragma unroll
+      for (int q = 0; q < 8; ++q) {
+        const float v0 = q < nt ? S.cs[q][c] : 0.f, v1 = q + 8 < nt ? S.cs[q + 8][c] : 0.f;
+        m[q] = v0 + v1;
+      }
+      const float ssum = ((m[0] + m[1]) + (m[2] + m[3])) + ((m[4] + m[5]) + (m[6] + m[7]));
+      if (h == 0) S.cmu[c] = cmu_value(a.c0, a.c1, S.mv[0][c], S.mv[1][c], ssum, nb);
+    }
+    __syncthreads();
+    // Phi~
+    if (w < 4) {
+      const float inv_b = 1.f / (float)nb, cmu = S.cmu[c];
+      float v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int r = 8 * w + 4 * h + e;
+        const float phh = S.slot[0][4 * w + e][lane], t = S.slot[1][4 * w + e][lane] + S.slot[2][4 * w + e][lane];
+        v[e] = step_value(S.phif[cur][r][c], a.eta, a.theta, phh, t, inv_b, uc[e], cmu);
+        small_put(S.x, r, c, v[e]);
+        S.xf[r][c] = v[e];
+      }
+      small_put4(S.xT, c, 8 * w + 4 * h, v);
+    }
+    __syncthreads();
+    // the renormalisation (wave 4) under the next step's loads
+    prefetch(st + 1);
+    if (w == 4) {
+      float x[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) x[i] = S.xf[8 * (i >> 2) + 4 * h + (i & 3)][c];
+      const int its = a.renorm_every > 0 && (a.step0 + st + 1) % a.renorm_every == 0 ? a.ns_iters : 0;
+      for (int it = 0; it < its; ++it) {
+        const floatx16 g = small_mm(S.xT, S.xT, k);
+        float gv[16], rs;  // rs: a row sum of |G| (every row on some lane), four columns at a time
+#pragma unroll
+        for (int i = 0; i < 16; ++i) gv[i] = g[i];
+        small_put_sym<MODE>(S.g, gv);
+        if constexpr (MODE == MM_F32) {  // lane c's column is row c
+          float t[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            float s = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) s += fabsf(gv[4 * q + e]);
+            t[q] = swap_add32(s, s);
+          }
+          rs = (t[0] + t[1]) + (t[2] + t[3]);
+        } else {                         // through LDS: lane 2 r + i takes half a row
+#pragma unroll
+          for (int i = 0; i < 16; ++i) S.xf[8 * (i >> 2) + 4 * h + (i & 3)][c] = gv[i];
+          asm volatile("" ::: "memory");
+          float t[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const float4 x = *reinterpret_cast<const float4*>(&S.xf[lane >> 1][16 * (lane & 1) + 4 * q]);
+            t[q] = ((fabsf(x.x) + fabsf(x.y)) + fabsf(x.z)) + fabsf(x.w);
+          }
+          rs = (t[0] + t[1]) + (t[2] + t[3]);
+          rs += dpp_mov<kDppXor1>(rs);
+        }
+        const float cs = guard_value((float)(wave_max((double)fix32(rs)) * 2.3283064365386963e-10));
+        asm volatile("" ::: "memory");
+        floatx16 y;
+        if (a.quintic) {
+          const floatx16 gg = small_mm(S.g, S.g, k);
+#pragma unroll
+          for (int i = 0; i < 16; ++i) gv[i] = qpoly_value(cs, gv[i], gg[i]);
+          small_put_sym<MODE>(S.q, gv);
+          asm volatile("" ::: "memory");
+          y = small_mm(S.x, S.q, k);
+        } else {
+          y = small_mm(S.x, S.g, k);
+        }
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = update_value(cs, a.quintic, x[i], y[i]);
+        if (it + 1 < its) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            small_put4(S.xT, c, 8 * q + 4 * h, x + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) small_put(S.x, 8 * q + 4 * h + e, c, x[4 * q + e]);
+          }
+          asm volatile("" ::: "memory");
+        }
+      }
+      small_new_phi<MODE>(S, cur ^ 1, x);
+    }
+    cur ^= 1;
+    __syncthreads();
+  }
+  if (w == 7) log_entry(a.nsteps - 1, cur);
+  if (w < 4)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 8 * w + 4 * h + e;
+      a.phi_out[r * kp + c] = S.phif[cur][r][c];
+    }
 }
 
 // ---- resolving the arguments (host) ------------------------------------------------------------------
@@ -1422,10 +1903,62 @@ static bool step_renorms(int64_t gstep, int32_t renorm_every, int32_t ns_iters) 
   return renorm_every > 0 && ((gstep + 1) % renorm_every == 0) && ns_iters > 0;
 }
 
+// Whole runs of instances that fit one workgroup (see stgd_small_kernel); launches of at most kSmallSteps steps.
+constexpr int64_t kSmallSteps = 4096;
+
+static bool small_run(const StgdArgs& a, const StgdTiming* timing, const StgdRenorm& renorm) {
+  return a.k <= 32 && a.kp == 64 && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre && !timing && !renorm;
+}
+
+template <int MODE, typename TY>
+static int run_small(hipStream_t s, const StgdArgs& args, const void* YA, const void* YB, const void* YCt, int64_t step0,
+                     int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree, const StgdBuffers& B, int& cur,
+                     double* frob_log) {
+  const void* fn = reinterpret_cast<const void*>(stgd_small_kernel<MODE, TY>);
+  const size_t shm = small_shm_bytes<MODE>(args.b);
+  MMSB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_shm_bytes<MODE>(kSmallB)));
+  for (int64_t st = 0; st < nsteps; st += kSmallSteps) {
+    const int64_t n = std::min<int64_t>(kSmallSteps, nsteps - st);
+    SmallArgs a;
+    a.ya = YA;
+    a.yb = YB;
+    a.yct = YCt;
+    a.mu_a = args.mu_a;
+    a.mu_b = args.mu_b;
+    a.mu_c = args.mu_c;
+    a.phi_in = B.phi[cur];
+    a.phi_out = B.phi[cur ^ (int)(n & 1)];
+    a.frob = frob_log + st;
+    a.step0 = step0 + st;
+    a.nsteps = n;
+    a.spe = ceil_div(args.n_x, args.bl);
+    a.n_x = args.n_x;
+    a.n_pad = args.n_pad;
+    a.k = args.k;
+    a.kp = args.kp;
+    a.b = args.b;
+    a.bl = args.bl;
+    a.ns_iters = ns_iters;
+    a.quintic = ns_degree == 5;
+    a.renorm_every = renorm_every;
+    a.c3 = args.c3;
+    a.c1 = args.c1;
+    a.c0 = args.c0;
+    a.eta = args.eta;
+    a.theta = args.theta;
+    hipLaunchKernelGGL((stgd_small_kernel<MODE, TY>), dim3(1), dim3(kSmallThreads), shm, s, a);
+    MMSB_LAUNCH_CHECK();
+    cur ^= (int)(n & 1);
+  }
+  return MMSB_OK;
+}
+
 template <int DMODE, int KMODE, typename TY, typename TPH>
 static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const void* YB, const void* YCt, int64_t step0,
                      int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree, const StgdBuffers& B,
                      int& cur, double* frob_log, StgdTiming* timing, const StgdFill& fill, const StgdRenorm& renorm) {
+  if (small_run(args, timing, renorm))
+    return run_small<KMODE, TY>(s, args, YA, YB, YCt, step0, nsteps, renorm_every, ns_iters, ns_degree, B, cur, frob_log);
   const int kp = args.kp;
   const int64_t spe = ceil_div(args.n_x, args.bl);
   const StepPlan P{args, B, YA, YB, YCt, ns_iters, ns_degree, KMODE == MM_BF16X3};
