@@ -129,6 +129,7 @@ struct mmsb_ctx {
   bool have_phi = false;
   // stop request (forceExit_flag, stpm.c:61,754): set from any thread, honoured between epochs
   std::atomic<int> stop_req{0};
+  std::atomic<StgdSmallCtl*> small_ctl{nullptr};  // pinned; its stop follows stop_req during a one-workgroup run
   // eigen / post
   double *lam = nullptr, *lamp = nullptr, *ahat = nullptr, *phil = nullptr, *LBU = nullptr;
   float *Upost = nullptr, *ZBtU = nullptr;
@@ -828,6 +829,28 @@ static int run_stgd_steps(mmsb_ctx* c, int64_t nsteps, int32_t precision, StgdTi
   const bool renorm_aligned = c->cfg.renorm_every <= 1 || spe % c->cfg.renorm_every == 0;
   if (rule) TRY(stgd_set_i64(c->s, &c->stopctl->stop_at, INT64_MAX));
   int64_t done = 0;
+  if (!timing && !qr && stgd_small_fits(a)) {  // the kernel itself looks for a stop request at its epochs' ends
+    StgdSmallCtl* ctl = c->small_ctl.load();
+    if (!ctl) {
+      HCHK(hipHostMalloc(reinterpret_cast<void**>(&ctl), sizeof(*ctl), hipHostMallocDefault));
+      ctl->stop = 0;
+      c->small_ctl.store(ctl);
+    }
+    // a request before this line has set stop_req, a later one sets ctl->stop itself
+    __atomic_store_n(&ctl->stop, 0, __ATOMIC_SEQ_CST);
+    if (c->stop_req.load()) __atomic_store_n(&ctl->stop, 1, __ATOMIC_SEQ_CST);
+    while (done < nsteps) {
+      const int64_t step0 = c->steps_done + done, ns = std::min<int64_t>(kSmallSteps, nsteps - done);
+      TRY(stgd_run_small(c->s, precision, a, ya, yb, yc, step0, ns, c->cfg.renorm_every, c->cfg.ns_iters, c->cfg.ns_degree,
+                         bufs, c->cur, c->frob + step0, ctl));
+      HCHK(hipStreamSynchronize(c->s));
+      c->cur ^= (int)(ctl->ran & 1);
+      done += ctl->ran;
+      if (ctl->ran < ns || (done < nsteps && (step0 + ns) % spe == 0 && c->stop_req.load())) break;
+    }
+    c->steps_done += done;
+    return MMSB_OK;
+  }
   while (done < nsteps) {
     const int64_t step0 = c->steps_done + done;
     const int cur0 = c->cur;
@@ -1469,6 +1492,7 @@ extern "C" void mmsb_destroy(mmsb_ctx* c) {
       for (hipGraphExec_t& g : row)
         if (g) (void)hipGraphExecDestroy(g);
   for (void* p : c->allocs) (void)hipFree(p);
+  if (StgdSmallCtl* ctl = c->small_ctl.load()) (void)hipHostFree(ctl);
   if (c->s) (void)hipStreamDestroy(c->s);
   delete c;
   if (g_live_contexts.fetch_sub(1) == 1) release_process_resources();
@@ -1586,6 +1610,11 @@ extern "C" int mmsb_set_yvectors(mmsb_ctx* c, int64_t n_x, int32_t k, const doub
   return MMSB_OK;
 }
 
+static void request_stop(mmsb_ctx* c) {
+  c->stop_req.store(1);
+  if (StgdSmallCtl* ctl = c->small_ctl.load()) __atomic_store_n(&ctl->stop, 1, __ATOMIC_SEQ_CST);
+}
+
 extern "C" int mmsb_stgd_timed(mmsb_ctx* c, int64_t steps, int32_t precision, double* phase_ms) {
   clear_error();
   MMSB_CHECK_ARG(c && phase_ms, "stgd_timed: null argument");
@@ -1638,17 +1667,23 @@ extern "C" int mmsb_stgd(mmsb_ctx* c, int64_t steps, int32_t precision) {
     const stpm_config& cf = c->cfg;
     const int64_t spe = (c->n[0] + c->bl - 1) / c->bl;
     const bool rule = cf.sgd_iter_min > 0 || cf.sgd_iter_max > 0;
-    for (int32_t e = 0; e < cf.epochs; ++e) {
-      const bool low = precision == MMSB_PREC_BF16 && e < cf.epochs - cf.polish_epochs;
+    // epochs of one precision are one call where that call watches for the request by itself
+    const bool joined = !rule && c->steps_done % spe == 0 && cf.renorm_mode != MMSB_RENORM_QR && stgd_small_fits(stgd_args(c));
+    int32_t span = 1;
+    for (int32_t e = 0; e < cf.epochs; e += span) {
+      const int32_t n_low = precision == MMSB_PREC_BF16 ? std::min(cf.epochs, std::max(0, cf.epochs - cf.polish_epochs)) : 0;
+      const bool low = e < n_low;
       bool stopped = false;
-      TRY(run_stgd_steps(c, spe, low ? MMSB_PREC_BF16 : MMSB_PREC_FP32, nullptr, rule, &stopped));
+      if (joined) span = (int32_t)std::min<int64_t>((low ? n_low : cf.epochs) - e, std::max<int64_t>(1, 16 * kSmallSteps / spe));
+      const int64_t end = c->steps_done + span * spe;
+      TRY(run_stgd_steps(c, span * spe, low ? MMSB_PREC_BF16 : MMSB_PREC_FP32, nullptr, rule, &stopped));
       if (stopped) {
         c->log("STGD loop ended after step %lld\n", (long long)c->steps_done);
         break;
       }
-      if (e + 1 < cf.epochs) {
+      if (e + span < cf.epochs || c->steps_done < end) {
         HCHK(hipStreamSynchronize(c->s));
-        if (c->stop_req.load()) {
+        if (c->stop_req.load() || c->steps_done < end) {
           c->log("Exiting STPM loop now\n");
           break;
         }
@@ -1664,7 +1699,7 @@ extern "C" int mmsb_stgd(mmsb_ctx* c, int64_t steps, int32_t precision) {
 extern "C" int mmsb_request_stop(mmsb_ctx* c) {
   clear_error();
   MMSB_CHECK_ARG(c, "request_stop: null context");
-  c->stop_req.store(1);
+  request_stop(c);
   return MMSB_OK;
 }
 
@@ -2055,7 +2090,7 @@ extern "C" int post_proc(void) {
 
 extern "C" void stpm_force_exit(void) {
   mmsb_ctx* c = g_ctx;
-  if (c) c->stop_req.store(1);
+  if (c) request_stop(c);
 }
 
 extern "C" void mmsb_release(void) {

@@ -99,6 +99,20 @@ int stgd_run(hipStream_t s, int32_t precision, const StgdArgs& args, const void*
              int64_t step0, int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree,
              const StgdBuffers& bufs, int& cur, double* frob_log, StgdTiming* timing = nullptr,
              const StgdFill& fill = StgdFill(), const StgdRenorm& renorm = StgdRenorm());
+
+// Runs of an instance that fits one workgroup (k <= 32, minibatches of at most 512 rows, no end test, Newton-Schulz
+// renormalisation): one launch takes all nsteps steps. At the end of each epoch but the last the kernel reads
+// ctl->stop and ends there when it is set; ctl->ran is the number of steps taken, and Phi is in bufs.phi[cur] after an
+// even number, else in bufs.phi[cur ^ 1]. ctl lies in pinned host memory.
+struct StgdSmallCtl {
+  int32_t stop;
+  int64_t ran;
+};
+constexpr int64_t kSmallSteps = 4096;  // most steps of one launch (30-40 ms)
+bool stgd_small_fits(const StgdArgs& args);
+int stgd_run_small(hipStream_t s, int32_t precision, const StgdArgs& args, const void* YA, const void* YB, const void* YCt,
+                   int64_t step0, int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree,
+                   const StgdBuffers& bufs, int cur, double* frob_log, StgdSmallCtl* ctl);
 // Sets *p = v on stream s (one thread; capturable, unlike a memset node).
 int stgd_set_i64(hipStream_t s, int64_t* p, int64_t v);
 

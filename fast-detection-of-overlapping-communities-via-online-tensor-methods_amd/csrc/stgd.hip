@@ -1216,9 +1216,9 @@ constexpr int kSmallThreads = 512;
 struct SmallArgs {
   const void *ya, *yb, *yct;        // all rows of X
   const double *mu_a, *mu_b, *mu_c;
-  const float* phi_in;
-  float* phi_out;
+  float *phi0, *phi1;               // Phi on entry in phi0; on exit there after an even number of steps, else in phi1
   double* frob;                     // [nsteps]
+  StgdSmallCtl* ctl;
   int64_t step0, nsteps, spe, n_x, n_pad;
   int32_t k, kp, b, bl, ns_iters, quintic, renorm_every;
   float c3, c1, c0, eta, theta;
@@ -1275,91 +1275,128 @@ __device__ inline void small_put_sym(SmallMat<MODE>& m, const float v[16]) {
   }
 }
 
+// The fragments of a 32 x 32 operand in MFMA layout: all LDS reads go out before the products that use them.
+template <int MODE>
+struct SmallFrag;
+template <>
+struct SmallFrag<MM_F32> {
+  floatx4 v[4];
+  __device__ inline void load(const SmallMat<MM_F32>& m) {
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) v[c] = *reinterpret_cast<const floatx4*>(&m.v[r][8 * c + 4 * h]);
+  }
+};
+template <>
+struct SmallFrag<MM_BF16X3> {
+  bf16x8 hi[2], lo[2];
+  __device__ inline void load(const SmallMat<MM_BF16X3>& m) {
+    const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      hi[c] = *reinterpret_cast<const bf16x8*>(&m.hi[r][16 * c + 8 * h]);
+      lo[c] = *reinterpret_cast<const bf16x8*>(&m.lo[r][16 * c + 8 * h]);
+    }
+  }
+};
+
 // A B^T over the first k columns of two operands; +0 added as the phase kernels' sums over empty parts do.
-__device__ inline floatx16 small_mm(const SmallMat<MM_F32>& A, const SmallMat<MM_F32>& B, int k) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+__device__ inline floatx16 small_mm(const SmallFrag<MM_F32>& A, const SmallFrag<MM_F32>& B, int k) {
   floatx16 acc = {};
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     if (8 * c < k) {
-      const floatx4 x = *reinterpret_cast<const floatx4*>(&A.v[r][8 * c + 4 * h]);
-      const floatx4 y = *reinterpret_cast<const floatx4*>(&B.v[r][8 * c + 4 * h]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(A.v[c][e], B.v[c][e], acc, 0, 0, 0);
     }
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] += 0.f;
   return acc;
 }
-__device__ inline floatx16 small_mm(const SmallMat<MM_BF16X3>& A, const SmallMat<MM_BF16X3>& B, int k) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+__device__ inline floatx16 small_mm(const SmallFrag<MM_BF16X3>& A, const SmallFrag<MM_BF16X3>& B, int k) {
   floatx16 acc = {};
 #pragma unroll
   for (int c = 0; c < 2; ++c)
     if (16 * c < k) {
-      const bf16x8 xh = *reinterpret_cast<const bf16x8*>(&A.hi[r][16 * c + 8 * h]);
-      const bf16x8 xl = *reinterpret_cast<const bf16x8*>(&A.lo[r][16 * c + 8 * h]);
-      const bf16x8 yh = *reinterpret_cast<const bf16x8*>(&B.hi[r][16 * c + 8 * h]);
-      const bf16x8 yl = *reinterpret_cast<const bf16x8*>(&B.lo[r][16 * c + 8 * h]);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, yh, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xh, yl, acc, 0, 0, 0);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xl, yh, acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.hi[c], B.hi[c], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.hi[c], B.lo[c], acc, 0, 0, 0);
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A.lo[c], B.hi[c], acc, 0, 0, 0);
     }
 #pragma unroll
   for (int i = 0; i < 16; ++i) acc[i] += 0.f;
   return acc;
 }
 
-// acc += (a block of 32 data rows in MFMA layout) Phi over the first k columns.
-__device__ inline void small_data_mm(floatx16& acc, const u32x4 a[4], const SmallMat<MM_F32>& B, int k) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+// pa += (a block of 32 data rows in MFMA layout) Phi and pb likewise, over the first k columns.
+__device__ inline void small_data_mm(floatx16& pa, floatx16& pb, const u32x4 xa[4], const u32x4 xb[4],
+                                     const SmallFrag<MM_F32>& B, int k) {
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     if (8 * c < k) {
-      const floatx4 x = as_f32(a[c]), y = *reinterpret_cast<const floatx4*>(&B.v[r][8 * c + 4 * h]);
+      const floatx4 x = as_f32(xa[c]), z = as_f32(xb[c]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) {
+        pa = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], B.v[c][e], pa, 0, 0, 0);
+        pb = __builtin_amdgcn_mfma_f32_32x32x2f32(z[e], B.v[c][e], pb, 0, 0, 0);
+      }
     }
 }
-__device__ inline void small_data_mm(floatx16& acc, const u32x4 a[4], const SmallMat<MM_BF16X3>& B, int k) {
-  const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+__device__ inline void small_data_mm(floatx16& pa, floatx16& pb, const u32x4 xa[4], const u32x4 xb[4],
+                                     const SmallFrag<MM_BF16X3>& B, int k) {
 #pragma unroll
   for (int c = 0; c < 2; ++c)
-    if (16 * c < k)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(a[c]), *reinterpret_cast<const bf16x8*>(&B.hi[r][16 * c + 8 * h]), acc, 0, 0, 0);
+    if (16 * c < k) {
+      pa = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(xa[c]), B.hi[c], pa, 0, 0, 0);
+      pb = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(xb[c]), B.hi[c], pb, 0, 0, 0);
+    }
 }
 
 // acc += (a block of Y_C^T in MFMA layout) C_g over the group's first n columns x (rows of the minibatch; C_g is zero
 // beyond them); cg points at the group's first column of C_g^T, row stride ld.
 __device__ inline void small_cg_mm(floatx16& acc, const u32x4 a[4], const float* cg, int ld, int n) {
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  floatx4 y[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) y[c] = *reinterpret_cast<const floatx4*>(cg + r * ld + 8 * c + 4 * h);
 #pragma unroll
   for (int c = 0; c < 4; ++c)
     if (8 * c < n) {
-      const floatx4 x = as_f32(a[c]), y = *reinterpret_cast<const floatx4*>(cg + r * ld + 8 * c + 4 * h);
+      const floatx4 x = as_f32(a[c]);
 #pragma unroll
-      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[e], acc, 0, 0, 0);
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(x[e], y[c][e], acc, 0, 0, 0);
     }
 }
 __device__ inline void small_cg_mm(floatx16& acc, const u32x4 a[4], const __bf16* cg, int ld, int n) {
   const int lane = threadIdx.x & 63, r = lane & 31, h = lane >> 5;
+  bf16x8 y[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) y[c] = *reinterpret_cast<const bf16x8*>(cg + r * ld + 16 * c + 8 * h);
 #pragma unroll
   for (int c = 0; c < 4; ++c)
-    if (16 * c < n)
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(a[c]), *reinterpret_cast<const bf16x8*>(cg + r * ld + 16 * c + 8 * h), acc, 0, 0, 0);
+    if (16 * c < n) acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16(a[c]), y[c], acc, 0, 0, 0);
 }
 
 template <int MODE>
 struct SmallShm {
-  SmallMat<MODE> phi, phiT, H, x, xT, g, q;
+  SmallMat<MODE> phiT, H, xT, g, q;
+  SmallMat<MODE> phis, xs;   // split runs: Phi and the Newton-Schulz iterate as operands (FP32 runs use the copies below)
   float phif[2][32][36];     // Phi in FP32, this step's and the next
   float xf[32][36];          // the Newton-Schulz iterate in FP32
+  __device__ inline const SmallMat<MODE>& phi_op(int cur) const {
+    if constexpr (MODE == MM_F32) return *reinterpret_cast<const SmallMat<MODE>*>(&phif[cur]);
+    else return phis;
+  }
+  __device__ inline const SmallMat<MODE>& x_op() const {
+    if constexpr (MODE == MM_F32) return *reinterpret_cast<const SmallMat<MODE>*>(&xf);
+    else return xs;
+  }
   float slot[3][16][64];     // Phi H and the halves of Y_C^T C_g, in accumulator layout
   float cs[kSmallB / 32][32];
-  float mu[2][32];           // mu_A, mu_B
+  alignas(16) float mu[2][32];  // mu_A, mu_B
   float mv[2][32];           // m_A, m_B
   float cmu[32];
-  u32x4 stage[8][256];       // per-wave transpose buffers
+  int stop;
+  alignas(16) u32x4 stage[8][256];       // per-wave transpose buffers
   typedef typename std::conditional<MODE == MM_F32, float, __bf16>::type T;
   alignas(16) T cgt[1];      // [32][b + 16 bytes]
 };
@@ -1383,11 +1420,11 @@ __device__ inline void small_new_phi(SmallShm<MODE>& S, int buf, const float v[1
     small_put4(S.phiT, c, 8 * q + 4 * h, x);
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      small_put(S.phi, 8 * q + 4 * h + e, c, x[e]);
+      if constexpr (MODE != MM_F32) small_put(S.phis, 8 * q + 4 * h + e, c, x[e]);
       S.phif[buf][8 * q + 4 * h + e][c] = x[e];
     }
-    const float* u = &S.mu[0][8 * q + 4 * h];
-    const float* w = &S.mu[1][8 * q + 4 * h];
+    const floatx4 u = *reinterpret_cast<const floatx4*>(&S.mu[0][8 * q + 4 * h]);
+    const floatx4 w = *reinterpret_cast<const floatx4*>(&S.mu[1][8 * q + 4 * h]);
     float sa, sb;
     {
 #pragma clang fp contract(off)
@@ -1418,10 +1455,8 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
   u32x4* stage = S.stage[w];
   T* cgt = S.cgt;
 
-  auto rows_of = [&](int64_t st, int64_t& row0, int& nb) {
-    row0 = ((a.step0 + st) % a.spe) * a.bl;
-    nb = (int)min((int64_t)a.bl, a.n_x - row0);
-  };
+  int64_t pos = a.step0 % a.spe;               // place of the step in its epoch and in its renormalisation period
+  int rn = a.renorm_every > 0 ? (int)(a.step0 % a.renorm_every) : 0;
   u32x4 pre[PF][4];                            // rows ahead: two tiles of Y_A, Y_B (waves 0..3), PF groups of Y_C^T
   u32x4 (&ra)[4] = pre[0], (&rb)[4] = pre[1];
   const int part = w - 5, ng = b / G;          // waves 5, 6: groups [g0, g1)
@@ -1435,11 +1470,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
     if (row0 % (16 / (int64_t)sizeof(TY)) == 0) stage_load<true>(y, p, a.n_pad);
     else stage_load<false>(y, p, a.n_pad);
   };
-  auto prefetch = [&](int64_t st) {
-    if (st >= a.nsteps) return;
-    int64_t row0;
-    int nb;
-    rows_of(st, row0, nb);
+  auto prefetch = [&](int64_t row0) {
     if (w < 4) {
       if (w < nt) load_tile(row0, w);
     } else if (w == 5 || w == 6) {
@@ -1476,20 +1507,28 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
     asm volatile("" ::: "memory");
     float v[16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = a.phi_in[(8 * (i >> 2) + 4 * h + (i & 3)) * kp + c];
+    for (int i = 0; i < 16; ++i) v[i] = a.phi0[(8 * (i >> 2) + 4 * h + (i & 3)) * kp + c];
     small_new_phi<MODE>(S, 0, v);
   }
-  prefetch(0);
+  prefetch(pos * a.bl);
   __syncthreads();
 
   int cur = 0;
-  for (int64_t st = 0; st < a.nsteps; ++st) {
-    int64_t row0;
-    int nb;
-    rows_of(st, row0, nb);
+  int64_t st = 0;
+  while (true) {
+    const int64_t row0 = pos * a.bl;
+    const int nb = (int)min((int64_t)a.bl, a.n_x - row0);
+    if (++pos == a.spe) pos = 0;
+    const bool renorm = a.renorm_every > 0 && ++rn == a.renorm_every;
+    if (renorm) rn = 0;
+    const bool poll = pos == 0 && st + 1 < a.nsteps;  // an epoch ends here with more to come
+    int stop = 0;
+    if (poll && w == 7) stop = __hip_atomic_load(&a.ctl->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     // P_A, P_B, C_g; (Phi^T Phi)^o2; the previous step's log entry
     if (w < 4) {
       const float mA = S.mv[0][c], mB = S.mv[1][c];
+      SmallFrag<MODE> phi;
+      phi.load(S.phiT);
       for (int tile = w; tile < nt; tile += 4) {
         u32x4 xa[4], xb[4];
 #pragma unroll
@@ -1501,8 +1540,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
         stage_swap(xa, stage);
         stage_swap(xb, stage);
         floatx16 pa = {}, pb = {};
-        small_data_mm(pa, xa, S.phiT, k);
-        small_data_mm(pb, xb, S.phiT, k);
+        small_data_mm(pa, pb, xa, xb, phi, k);
         float t[4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -1525,18 +1563,27 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
         if (h == 0) S.cs[tile][c] = (t[0] + t[1]) + (t[2] + t[3]);
       }
     } else if (w == 4) {
-      const floatx16 g = small_mm(S.phiT, S.phiT, k);
+      SmallFrag<MODE> phi;
+      phi.load(S.phiT);
+      const floatx16 g = small_mm(phi, phi, k);
       float v[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) v[i] = g[i] * g[i];
       small_put_sym<MODE>(S.H, v);
-    } else if (w == 7 && st > 0) {
+    } else if (w == 5 || w == 6) {  // Y_C^T into MFMA layout ahead of C_g
+#pragma unroll
+      for (int u = 0; u < PF; ++u)
+        if (g0 + u < g1) stage_swap(pre[u], stage);
+    } else if (st > 0) {
       log_entry(st - 1, cur);
     }
     __syncthreads();
     // Phi H, the halves of Y_C^T C_g, c_mu
     if (w == 4) {
-      const floatx16 v = small_mm(S.phi, S.H, k);
+      SmallFrag<MODE> phi, hh;
+      phi.load(S.phi_op(cur));
+      hh.load(S.H);
+      const floatx16 v = small_mm(phi, hh, k);
 #pragma unroll
       for (int i = 0; i < 16; ++i) S.slot[0][i][lane] = v[i];
     } else if (w == 5 || w == 6) {
@@ -1545,7 +1592,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
 #pragma unroll
         for (int u = 0; u < PF; ++u) {
           if (g + u < g1) {
-            stage_swap(pre[u], stage);
+            if (g > g0) stage_swap(pre[u], stage);
             small_cg_mm(acc, pre[u], cgt + (g + u) * G, ldc, nb - (g + u) * G);
             if (g + u + PF < g1) load_group(pre[u], row0, g + u + PF);
           }
@@ -1573,21 +1620,25 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
         const int r = 8 * w + 4 * h + e;
         const float phh = S.slot[0][4 * w + e][lane], t = S.slot[1][4 * w + e][lane] + S.slot[2][4 * w + e][lane];
         v[e] = step_value(S.phif[cur][r][c], a.eta, a.theta, phh, t, inv_b, uc[e], cmu);
-        small_put(S.x, r, c, v[e]);
+        if constexpr (MODE != MM_F32) small_put(S.xs, r, c, v[e]);
         S.xf[r][c] = v[e];
       }
       small_put4(S.xT, c, 8 * w + 4 * h, v);
     }
     __syncthreads();
     // the renormalisation (wave 4) under the next step's loads
-    prefetch(st + 1);
+    if (st + 1 < a.nsteps) prefetch(pos * a.bl);
+    if (poll && w == 7 && lane == 0) S.stop = stop;
     if (w == 4) {
       float x[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) x[i] = S.xf[8 * (i >> 2) + 4 * h + (i & 3)][c];
-      const int its = a.renorm_every > 0 && (a.step0 + st + 1) % a.renorm_every == 0 ? a.ns_iters : 0;
+      const int its = renorm ? a.ns_iters : 0;
       for (int it = 0; it < its; ++it) {
-        const floatx16 g = small_mm(S.xT, S.xT, k);
+        SmallFrag<MODE> fa, fb;
+        fa.load(S.xT);
+        const floatx16 g = small_mm(fa, fa, k);
+        fa.load(S.x_op());
         float gv[16], rs;  // rs: a row sum of |G| (every row on some lane), four columns at a time
 #pragma unroll
         for (int i = 0; i < 16; ++i) gv[i] = g[i];
@@ -1615,19 +1666,19 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
           rs = (t[0] + t[1]) + (t[2] + t[3]);
           rs += dpp_mov<kDppXor1>(rs);
         }
-        const float cs = guard_value((float)(wave_max((double)fix32(rs)) * 2.3283064365386963e-10));
+        // the largest row sum, clamped as fix32 does; above 2, where the guard acts, its fixed point is exact
+        const float cs = guard_value(wave_max(fminf(rs, 1073741824.f)));
         asm volatile("" ::: "memory");
-        floatx16 y;
+        fb.load(S.g);
         if (a.quintic) {
-          const floatx16 gg = small_mm(S.g, S.g, k);
+          const floatx16 gg = small_mm(fb, fb, k);
 #pragma unroll
           for (int i = 0; i < 16; ++i) gv[i] = qpoly_value(cs, gv[i], gg[i]);
           small_put_sym<MODE>(S.q, gv);
           asm volatile("" ::: "memory");
-          y = small_mm(S.x, S.q, k);
-        } else {
-          y = small_mm(S.x, S.g, k);
+          fb.load(S.q);
         }
+        const floatx16 y = small_mm(fa, fb, k);
         asm volatile("" ::: "memory");
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = update_value(cs, a.quintic, x[i], y[i]);
@@ -1636,7 +1687,10 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
           for (int q = 0; q < 4; ++q) {
             small_put4(S.xT, c, 8 * q + 4 * h, x + 4 * q);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) small_put(S.x, 8 * q + 4 * h + e, c, x[4 * q + e]);
+            for (int e = 0; e < 4; ++e) {
+              if constexpr (MODE != MM_F32) small_put(S.xs, 8 * q + 4 * h + e, c, x[4 * q + e]);
+              else S.xf[8 * q + 4 * h + e][c] = x[4 * q + e];
+            }
           }
           asm volatile("" ::: "memory");
         }
@@ -1644,14 +1698,20 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
       small_new_phi<MODE>(S, cur ^ 1, x);
     }
     cur ^= 1;
+    ++st;
     __syncthreads();
+    if (st == a.nsteps || (poll && S.stop)) break;
   }
-  if (w == 7) log_entry(a.nsteps - 1, cur);
+  if (w == 7) {
+    log_entry(st - 1, cur);
+    if (lane == 0) a.ctl->ran = st;
+  }
+  float* phi_out = cur ? a.phi1 : a.phi0;
   if (w < 4)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int r = 8 * w + 4 * h + e;
-      a.phi_out[r * kp + c] = S.phif[cur][r][c];
+      phi_out[r * kp + c] = S.phif[cur][r][c];
     }
 }
 
@@ -1903,62 +1963,65 @@ static bool step_renorms(int64_t gstep, int32_t renorm_every, int32_t ns_iters) 
   return renorm_every > 0 && ((gstep + 1) % renorm_every == 0) && ns_iters > 0;
 }
 
-// Whole runs of instances that fit one workgroup (see stgd_small_kernel); launches of at most kSmallSteps steps.
-constexpr int64_t kSmallSteps = 4096;
-
-static bool small_run(const StgdArgs& a, const StgdTiming* timing, const StgdRenorm& renorm) {
-  return a.k <= 32 && a.kp == 64 && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre && !timing && !renorm;
+bool stgd_small_fits(const StgdArgs& a) {
+  return a.k <= 32 && a.kp == 64 && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
 }
 
 template <int MODE, typename TY>
 static int run_small(hipStream_t s, const StgdArgs& args, const void* YA, const void* YB, const void* YCt, int64_t step0,
-                     int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree, const StgdBuffers& B, int& cur,
-                     double* frob_log) {
+                     int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree, const StgdBuffers& B, int cur,
+                     double* frob_log, StgdSmallCtl* ctl) {
   const void* fn = reinterpret_cast<const void*>(stgd_small_kernel<MODE, TY>);
   const size_t shm = small_shm_bytes<MODE>(args.b);
   MMSB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_shm_bytes<MODE>(kSmallB)));
-  for (int64_t st = 0; st < nsteps; st += kSmallSteps) {
-    const int64_t n = std::min<int64_t>(kSmallSteps, nsteps - st);
-    SmallArgs a;
-    a.ya = YA;
-    a.yb = YB;
-    a.yct = YCt;
-    a.mu_a = args.mu_a;
-    a.mu_b = args.mu_b;
-    a.mu_c = args.mu_c;
-    a.phi_in = B.phi[cur];
-    a.phi_out = B.phi[cur ^ (int)(n & 1)];
-    a.frob = frob_log + st;
-    a.step0 = step0 + st;
-    a.nsteps = n;
-    a.spe = ceil_div(args.n_x, args.bl);
-    a.n_x = args.n_x;
-    a.n_pad = args.n_pad;
-    a.k = args.k;
-    a.kp = args.kp;
-    a.b = args.b;
-    a.bl = args.bl;
-    a.ns_iters = ns_iters;
-    a.quintic = ns_degree == 5;
-    a.renorm_every = renorm_every;
-    a.c3 = args.c3;
-    a.c1 = args.c1;
-    a.c0 = args.c0;
-    a.eta = args.eta;
-    a.theta = args.theta;
-    hipLaunchKernelGGL((stgd_small_kernel<MODE, TY>), dim3(1), dim3(kSmallThreads), shm, s, a);
-    MMSB_LAUNCH_CHECK();
-    cur ^= (int)(n & 1);
-  }
+  SmallArgs a;
+  a.ya = YA;
+  a.yb = YB;
+  a.yct = YCt;
+  a.mu_a = args.mu_a;
+  a.mu_b = args.mu_b;
+  a.mu_c = args.mu_c;
+  a.phi0 = B.phi[cur];
+  a.phi1 = B.phi[cur ^ 1];
+  a.frob = frob_log;
+  a.ctl = ctl;
+  a.step0 = step0;
+  a.nsteps = nsteps;
+  a.spe = ceil_div(args.n_x, args.bl);
+  a.n_x = args.n_x;
+  a.n_pad = args.n_pad;
+  a.k = args.k;
+  a.kp = args.kp;
+  a.b = args.b;
+  a.bl = args.bl;
+  a.ns_iters = ns_iters;
+  a.quintic = ns_degree == 5;
+  a.renorm_every = renorm_every;
+  a.c3 = args.c3;
+  a.c1 = args.c1;
+  a.c0 = args.c0;
+  a.eta = args.eta;
+  a.theta = args.theta;
+  hipLaunchKernelGGL((stgd_small_kernel<MODE, TY>), dim3(1), dim3(kSmallThreads), shm, s, a);
+  MMSB_LAUNCH_CHECK();
   return MMSB_OK;
+}
+
+int stgd_run_small(hipStream_t s, int32_t precision, const StgdArgs& args, const void* YA, const void* YB, const void* YCt,
+                   int64_t step0, int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree,
+                   const StgdBuffers& bufs, int cur, double* frob_log, StgdSmallCtl* ctl) {
+  MMSB_CHECK_ARG(stgd_small_fits(args) && nsteps > 0, "stgd_run_small: instance too large");
+  if (precision == MMSB_PREC_BF16)
+    return run_small<MM_BF16X3, __bf16>(s, args, YA, YB, YCt, step0, nsteps, renorm_every, ns_iters, ns_degree, bufs, cur,
+                                        frob_log, ctl);
+  return run_small<MM_F32, float>(s, args, YA, YB, YCt, step0, nsteps, renorm_every, ns_iters, ns_degree, bufs, cur, frob_log,
+                                  ctl);
 }
 
 template <int DMODE, int KMODE, typename TY, typename TPH>
 static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const void* YB, const void* YCt, int64_t step0,
                      int64_t nsteps, int32_t renorm_every, int32_t ns_iters, int32_t ns_degree, const StgdBuffers& B,
                      int& cur, double* frob_log, StgdTiming* timing, const StgdFill& fill, const StgdRenorm& renorm) {
-  if (small_run(args, timing, renorm))
-    return run_small<KMODE, TY>(s, args, YA, YB, YCt, step0, nsteps, renorm_every, ns_iters, ns_degree, B, cur, frob_log);
   const int kp = args.kp;
   const int64_t spe = ceil_div(args.n_x, args.bl);
   const StepPlan P{args, B, YA, YB, YCt, ns_iters, ns_degree, KMODE == MM_BF16X3};

@@ -90,6 +90,18 @@ __device__ inline double wave_max(double v) {
   return fmax(fmax(read_lane(v, 0), read_lane(v, 16)), fmax(read_lane(v, 32), read_lane(v, 48)));
 }
 
+__device__ inline float read_lane(float v, int lane) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
+}
+
+__device__ inline float wave_max(float v) {
+  v = fmaxf(v, dpp_mov<kDppRor8>(v));
+  v = fmaxf(v, dpp_mov<kDppRor4>(v));
+  v = fmaxf(v, dpp_mov<kDppXor2>(v));
+  v = fmaxf(v, dpp_mov<kDppXor1>(v));
+  return fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
+}
+
 // Sums over the lanes of a quad, and of a group of eight (offsets 1, 2, 4).
 __device__ inline float quad_sum(float v) {
 #pragma clang fp contract(off)

@@ -60,3 +60,19 @@ def test_small_run_with_the_guard_acting(mmsb, prec):
 
 def test_small_run_longer_than_a_launch(mmsb):
     same(mmsb, 4099, 5, 1, "fp32", (4099, 4100), learn_rate=1e-4)
+
+
+@pytest.mark.parametrize("first", [0, 3])
+def test_joined_epochs_equal_single_ones(mmsb, first):
+    """Mixed-precision epochs (the last one in FP32) as one call, from an epoch boundary and from inside an epoch."""
+    n, k, b = 500, 10, 64
+    p, q = (pipeline(mmsb, n, k, b, 5, False, epochs=6, polish_epochs=2, learn_rate=2e-3, sgd_iter_min=0, sgd_iter_max=0)
+            for _ in range(2))
+    p.stgd(first, "bf16")
+    p.stgd(-1, "bf16")
+    q.stgd_timed(first, "bf16")
+    for e in range(6):
+        q.stgd_timed(8, "bf16" if e < 4 else "fp32")
+    assert np.array_equal(p.get("phi"), q.get("phi")) and np.array_equal(p.get("frob"), q.get("frob"))
+    p.close()
+    q.close()
