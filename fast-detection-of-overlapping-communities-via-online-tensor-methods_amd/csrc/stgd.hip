@@ -228,21 +228,73 @@ struct Frag<MM_BF16X3> {
   }
 };
 
-// Ring depth per mode (fragment registers: 32 VGPRs per set for FP32 and BF16, 64 for split BF16).
-// Two sets keep 8 (FP32, BF16) or 16 (split BF16) loads per wave in flight ahead of the MFMAs.
-#ifndef MMSB_RING_F32
-#define MMSB_RING_F32 2
-#endif
-#ifndef MMSB_RING_BF16
-#define MMSB_RING_BF16 2
-#endif
-#ifndef MMSB_RING_BF16X3
-#define MMSB_RING_BF16X3 2
-#endif
-static_assert(MMSB_RING_F32 >= 2 && MMSB_RING_BF16 >= 2 && MMSB_RING_BF16X3 >= 2, "ring depth must be at least 2");
-template <int MODE>
-constexpr int ring_depth() {
-  return MODE == MM_BF16X3 ? MMSB_RING_BF16X3 : (MODE == MM_BF16 ? MMSB_RING_BF16 : MMSB_RING_F32);
+// use(f[..]) of the groups at k = 0, G, .. (< kl) in order, each after load(f[..], k), with the loads ahead of the uses: with
+// D = 4 sets and a multiple of four groups the next three groups are in flight, else the next one. No load is under a condition of
+// its own: where paths with and without a load meet, the compiler waits for all loads in flight (it counts the newest
+// ones it is sure of), and a ring of guarded loads then costs one memory latency per group, 0.5 us (P2 of an FP32 step
+// at k = 100, b = 1024: 14.5 us with guards, 10.9 without; BF16 at k = 500: 6.1 and 5.5, Newton-Schulz 22 and 20.5). COMPACT keeps the
+// guards for fewer registers (the body twice instead of five times): for reductions of one or two groups, where all
+// loads go out first anyway.
+template <int G, bool COMPACT = false, int D, typename F, typename L, typename M>
+__device__ __forceinline__ void pipelined(F (&f)[D], int64_t kl, L load, M mma) {
+  static_assert(D == 2 || D == 4, "two or four sets");
+  if (kl <= 0) return;
+  auto use = [&](F& x) {
+    x.swap();
+    mma(x);
+  };
+  if constexpr (COMPACT) {
+    load(f[0], (int64_t)0);
+    for (int64_t k = 0; k < kl; k += 2 * G) {
+#pragma unroll
+      for (int d = 0; d < 2; ++d) {
+        const int64_t kk = k + d * G;
+        if (kk < kl) {
+          const int64_t kn = kk + G;
+          if (kn < kl) load(f[1 - d], kn);
+          use(f[d]);
+        }
+      }
+    }
+    return;
+  }
+  const int n = (int)(kl / G);  // 32-bit offsets: fewer registers
+  if constexpr (D == 4) {
+    if (n % 4 == 0) {
+#pragma unroll
+      for (int d = 0; d < 4; ++d) load(f[d], d * G);
+      f[0].swap();  // each group goes through LDS under the MFMAs of the one before
+      for (int g = 4; g < n; g += 4) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) {
+          f[(d + 1) % 4].swap();
+          mma(f[d]);
+          load(f[d], (g + d) * G);
+        }
+      }
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        if (d < 3) f[d + 1].swap();
+        mma(f[d]);
+      }
+      return;
+    }
+  }
+  load(f[0], 0);
+  int g = 0;
+  for (; g + 2 < n; g += 2) {
+    load(f[1], (g + 1) * G);
+    use(f[0]);
+    load(f[0], (g + 2) * G);
+    use(f[1]);
+  }
+  if (g + 1 < n) {
+    load(f[1], (g + 1) * G);
+    use(f[0]);
+    use(f[1]);
+  } else {
+    use(f[0]);
+  }
 }
 
 // The part of a reduction of length K (a multiple of the group) that wave `idx` of `parts` owns.
@@ -256,35 +308,20 @@ __device__ inline void kslice(int64_t K, int parts, int idx, int64_t& k0, int64_
 }
 
 // acc += A[r0 + 0..32, k0 .. k0+kl) * B[c0 + 0..32, k0 .. k0+kl)^T for the calling wave.
-// kl is a multiple of kgroup<MODE>(); AAL says whether A's rows are 16-byte aligned at k0.
-// Fragment set d of the ring is loaded D - 1 groups before its MFMAs; the ring index is a
-// compile-time constant after unrolling, so the sets stay in registers.
-template <int MODE, bool AAL, typename TA, typename TB>
+// kl is a multiple of kgroup<MODE>(); AAL says whether A's rows are 16-byte aligned at k0; D fragment sets (32 VGPRs
+// each for FP32 and BF16, 64 for split BF16).
+template <int MODE, bool AAL, int D = 2, bool COMPACT = false, typename TA, typename TB>
 __device__ inline void wave_mm(floatx16& acc, const Opnd<TA>& A, const Opnd<TB>& B, int64_t r0, int64_t c0, int64_t k0,
                                int64_t kl) {
-  if (kl <= 0) return;
   constexpr int G = kgroup<MODE>();
-  constexpr int D = ring_depth<MODE>();
   const TA* a = A.hi + r0 * A.ld + k0;
   const TA* al = A.lo + r0 * A.ld + k0;
   const TB* b = B.hi + c0 * B.ld + k0;
   const TB* bl = B.lo + c0 * B.ld + k0;
   Frag<MODE> f[D];
-#pragma unroll
-  for (int d = 0; d < D - 1; ++d)
-    if (d * G < kl) f[d].template load<AAL>(a + d * G, al + d * G, A.ld, b + d * G, bl + d * G, B.ld);
-  for (int64_t g = 0; g < kl; g += D * G) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int64_t kk = g + d * G;
-      if (kk < kl) {
-        const int64_t kn = kk + (D - 1) * G;
-        if (kn < kl) f[(d + D - 1) % D].template load<AAL>(a + kn, al + kn, A.ld, b + kn, bl + kn, B.ld);
-        f[d].swap();
-        f[d].mma(acc);
-      }
-    }
-  }
+  pipelined<G, COMPACT>(
+      f, kl, [&](Frag<MODE>& x, auto k) { x.template load<AAL>(a + k, al + k, A.ld, b + k, bl + k, B.ld); },
+      [&](Frag<MODE>& x) { x.mma(acc); });
 }
 
 // Two products that share their column operand, acc_a += A1 B^T and acc_b += A2 B^T, for one wave
@@ -322,29 +359,17 @@ struct FragPair {
   }
 };
 
-template <int MODE>
+template <int MODE, bool COMPACT = false>
 __device__ inline void wave_mm_pair(floatx16& acc_a, floatx16& acc_b, const op_t<MODE>* A1, const op_t<MODE>* A2, int64_t lda,
                                     const op_t<MODE>* B, int64_t ldb, int64_t r0, int64_t c0, int64_t k0, int64_t kl) {
-  if (kl <= 0) return;
   constexpr int G = kgroup<MODE>();
-  constexpr int D = 2;
-  const op_t<MODE>* a1 = A1 + r0 * lda + k0;
-  const op_t<MODE>* a2 = A2 + r0 * lda + k0;
+  const op_t<MODE>* p1 = A1 + r0 * lda + k0;
+  const op_t<MODE>* p2 = A2 + r0 * lda + k0;
   const op_t<MODE>* b = B + c0 * ldb + k0;
-  FragPair<MODE> f[D];
-  f[0].load(a1, a2, lda, b, ldb);
-  for (int64_t g = 0; g < kl; g += D * G) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int64_t kk = g + d * G;
-      if (kk < kl) {
-        const int64_t kn = kk + (D - 1) * G;
-        if (kn < kl) f[(d + D - 1) % D].load(a1 + kn, a2 + kn, lda, b + kn, ldb);
-        f[d].swap();
-        f[d].mma(acc_a, acc_b);
-      }
-    }
-  }
+  FragPair<MODE> f[2];
+  pipelined<G, COMPACT>(
+      f, kl, [&](FragPair<MODE>& x, auto k) { x.load(p1 + k, p2 + k, lda, b + k, ldb); },
+      [&](FragPair<MODE>& x) { x.mma(acc_a, acc_b); });
 }
 
 __device__ inline bool epi_thread() { return threadIdx.x < 256; }
@@ -555,7 +580,8 @@ __device__ inline void store4(T* p, const float v[4]) {
 // serve the per-phase launches of one instance (stgd_phase_kernel, blockIdx.x = tile) and the
 // persistent launch over many instances (stgd_batch_kernel, tiles from a work queue).
 enum StgdPhase { PH_SETUP = 0, PH_P1 = 1, PH_P2 = 2, PH_GRAM = 3, PH_UPDATE = 4, PH_COPY = 5, PH_QPOLY = 6, PH_QRFIN = 7,
-                 PH_FROB = 8 };
+                 PH_FROB = 8,
+                 PH_P2S = 9 };  // P2 spread wider, for one instance's launches (see p2_spread)
 
 // What one phase of one step reads and writes, resolved on the host: every pointer is the one to use (the Phi
 // ping-pong, the Newton-Schulz scratch of the iteration, the minibatch's first row), so that a kernel fetches
@@ -653,7 +679,7 @@ union PhaseArgs {
 template <int PHASE>
 __host__ __device__ inline const auto& phase_args(const PhaseArgs& a) {
   if constexpr (PHASE == PH_P1) return a.p1;
-  else if constexpr (PHASE == PH_P2) return a.p2;
+  else if constexpr (PHASE == PH_P2 || PHASE == PH_P2S) return a.p2;
   else if constexpr (PHASE == PH_GRAM) return a.gram;
   else if constexpr (PHASE == PH_QPOLY) return a.qpoly;
   else if constexpr (PHASE == PH_UPDATE) return a.update;
@@ -664,6 +690,7 @@ template <int PHASE>
 struct ArgsOf { using type = CopyArgs; };
 template <> struct ArgsOf<PH_P1> { using type = P1Args; };
 template <> struct ArgsOf<PH_P2> { using type = P2Args; };
+template <> struct ArgsOf<PH_P2S> { using type = P2Args; };
 template <> struct ArgsOf<PH_GRAM> { using type = GramArgs; };
 template <> struct ArgsOf<PH_QPOLY> { using type = QpolyArgs; };
 template <> struct ArgsOf<PH_UPDATE> { using type = UpdateArgs; };
@@ -791,6 +818,9 @@ __device__ inline float cspart_reduce(const PartSum& ps, const float* cs_part, i
 template <int DMODE, int KMODE, typename TY, typename TPH>
 __device__ __forceinline__ void p1_tile(const P1Args& a, int tile, StgdSmem& sm, bool log) {
   constexpr bool SPLIT = KMODE == MM_BF16X3;
+  // three workgroups per compute unit need at most 168 registers: at k = 500, b = 1024 (2048) P1 takes 7.5 (10.6) us,
+  // 8.6 (11.3) with the five bodies and their spills, 7.5 (11.2) with two workgroups
+  constexpr bool COMPACT = DMODE == MM_BF16;
   const int kp = a.kp;
   const int ntk = kp / 32;
   const int64_t nel = (int64_t)kp * kp;
@@ -807,7 +837,7 @@ __device__ __forceinline__ void p1_tile(const P1Args& a, int tile, StgdSmem& sm,
     // every wave: P_A and P_B over its part of the k reduction, sharing the Phi^T fragments
     floatx16 acc_b = {};
     kslice<DMODE>(kp, kWaves, w, k0, kl);
-    wave_mm_pair<DMODE>(acc, acc_b, static_cast<const TY*>(a.ya), static_cast<const TY*>(a.yb), kp,
+    wave_mm_pair<DMODE, COMPACT>(acc, acc_b, static_cast<const TY*>(a.ya), static_cast<const TY*>(a.yb), kp,
                         pick<DMODE>(a.phiT, nel, kp).hi, kp, x0, j0, k0, kl);
     if (epi_thread()) {
       const float m = mpart_reduce(ps, a.mpart, kp, ntk, j0);
@@ -853,7 +883,7 @@ __device__ __forceinline__ void p1_tile(const P1Args& a, int tile, StgdSmem& sm,
     const int64_t i0 = (int64_t)ti * 32, j0 = (int64_t)tj * 32;
     const Opnd<op_t<KMODE>> phiT_k = pick<KMODE>(a.phiT, nel, kp);
     kslice<KMODE>(kp, kWaves, w, k0, kl);
-    wave_mm<KMODE, true>(acc, phiT_k, phiT_k, i0, j0, k0, kl);  // G = Phi^T Phi
+    wave_mm<KMODE, true, 2, COMPACT>(acc, phiT_k, phiT_k, i0, j0, k0, kl);  // G = Phi^T Phi
     if (log) {
       const double f = wave_sum(fs);
       if (threadIdx.x == 0) *a.frob_prev = f;
@@ -916,9 +946,9 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
     const Opnd<TY> yc = opnd<TY>(static_cast<const TY*>(a.yct), nullptr, a.n_pad);
     const Opnd<TPH> cg = opnd<TPH>(static_cast<const TPH*>(a.cgt), nullptr, a.b);
     if (a.aligned)
-      wave_mm<DMODE, true>(acc, yc, cg, i0, j0, k0, kl);
+      wave_mm<DMODE, true, 4>(acc, yc, cg, i0, j0, k0, kl);
     else
-      wave_mm<DMODE, false>(acc, yc, cg, i0, j0, k0, kl);
+      wave_mm<DMODE, false, 4>(acc, yc, cg, i0, j0, k0, kl);
   }
   if (epi) {
     const int c = threadIdx.x >> 3;
@@ -946,6 +976,117 @@ __device__ __forceinline__ void p2_tile(const P2Args& a, int tile, StgdSmem& sm)
 #pragma unroll
   for (int e = 0; e < 4; ++e) pre.pv[e] = p0[e];
   finish_tile<SPLIT>(sm.p2.S, kp, ti, i0, j0, v, a.out, a.out16, a.outT, a.outT16, pre, a.fpart ? a.fpart + tile : nullptr, nullptr);
+}
+
+// A block of 16 rows x 128 bytes of an FP32 operand: loaded and put into the layout of the 16 x 16 x 4 MFMA through the
+// wave's buffer, in the k order of the 32-row blocks (8 c + e, 8 c + 4 + e for e = 0 .. 3). Both MFMA shapes add one
+// product after the other in k order, so the 16-row blocks give the 32-row blocks' bits.
+template <bool AL>
+__device__ inline void quad_load(u32x4 v[2], const float* row0, int64_t ld) {
+  const uint32_t lane = threadIdx.x & 63;
+  const uint32_t off = ((lane >> 3) * (uint32_t)ld + (lane & 7) * 4) * 4;
+  const char* base = reinterpret_cast<const char*>(row0);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) v[c] = ld16<AL>(reinterpret_cast<const float*>(base + 32 * c * ld + off));
+}
+
+struct QuadFrag {
+  u32x4 a[2], b[2];
+  __device__ inline void swap() {
+    u32x4* buf = wave_stage();  // A's rows, then B's
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int row = (lane >> 3) + 8 * c, at = row * 8 + ((lane & 7) ^ ((row >> 1) & 7));
+      buf[at] = a[c];
+      buf[128 + at] = b[c];
+    }
+    asm volatile("" ::: "memory");
+    const uint32_t* p = reinterpret_cast<const uint32_t*>(buf) + (g >> 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const int at = 4 * (r * 8 + ((2 * c + (g & 1)) ^ ((r >> 1) & 7)));
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        a[c >> 1][2 * (c & 1) + e] = p[at + 2 * e];
+        b[c >> 1][2 * (c & 1) + e] = p[512 + at + 2 * e];
+      }
+    }
+    asm volatile("" ::: "memory");
+  }
+  __device__ inline void mma(floatx4& acc) const {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const floatx4 x = as_f32(a[c]), y = as_f32(b[c]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(x[e], y[e], acc, 0, 0, 0);
+    }
+  }
+};
+
+// wave_mm of one 16 x 16 block in FP32.
+template <bool AAL>
+__device__ inline void quad_mm(floatx4& acc, const float* a, int64_t lda, const float* b, int64_t ldb, int64_t kl) {
+  QuadFrag f[4];
+  pipelined<32>(
+      f, kl,
+      [&](QuadFrag& x, auto k) {
+        quad_load<AAL>(x.a, a + k, lda);
+        quad_load<true>(x.b, b + k, ldb);
+      },
+      [&](QuadFrag& x) { x.mma(acc); });
+}
+
+// P2 of an FP32 step in 16 x 16 tiles, four times the workgroups: of a 32 x 32 tile the two waves that take Y_C^T C_g
+// pass MFMAs in a row for 6.8 us at b = 1024 while most compute units have no tile (16 tiles at k = 100). P2 at k = 100,
+// b = 1024 (2048): 4.3 (8.1) us against 10.9 (20.5).
+__device__ __forceinline__ void p2_quad_tile(const P2Args& a, int tile, StgdSmem& sm) {
+  static_assert(kWaves == 4, "two waves for each of the two products");
+  const int kp = a.kp, nq = kp / 16;
+  const int w = wave_id(), lane = threadIdx.x & 63;
+  const int64_t i0 = (int64_t)(tile / nq) * 16, j0 = (int64_t)(tile % nq) * 16;
+  const int r = threadIdx.x >> 4, c = threadIdx.x & 15, pc = threadIdx.x >> 3;  // pc < 16: column of c_mu
+  floatx4 acc = {};
+  int64_t k0, kl;
+  PartSum ps;
+  float mab_a = 0.f, mab_b = 0.f;
+  double muc_d = a.mu_c[i0 + r];
+  float p0 = a.phi[(i0 + r) * kp + j0 + c];
+  if (pc < 16) {
+    cspart_load(ps, a.cs_part, kp, a.b / 32, j0);
+    mab_a = a.mab[j0 + pc];
+    mab_b = a.mab[kp + j0 + pc];
+  }
+  if ((w & 2) == 0) {
+    kslice<MM_F32>(kp, 2, w & 1, k0, kl);
+    quad_mm<true>(acc, static_cast<const float*>(a.phi_op) + i0 * kp + k0, kp, static_cast<const float*>(a.h_op) + j0 * kp + k0,
+                  kp, kl);
+  } else {
+    kslice<MM_F32>(a.b, 2, w & 1, k0, kl);
+    const float* yc = static_cast<const float*>(a.yct) + i0 * a.n_pad + k0;
+    const float* cg = static_cast<const float*>(a.cgt) + j0 * a.b + k0;
+    if (a.aligned) quad_mm<true>(acc, yc, a.n_pad, cg, a.b, kl);
+    else quad_mm<false>(acc, yc, a.n_pad, cg, a.b, kl);
+  }
+  if (pc < 16) {
+    const float ssum = cspart_reduce(ps, a.cs_part, kp, a.b / 32, j0);
+    if ((threadIdx.x & 7) == 0) sm.p2.cmu[pc] = cmu_value(a.c0, a.c1, mab_a, mab_b, ssum, a.nb);
+  }
+  if (tile == 0)
+    for (int t = threadIdx.x; t < kp; t += blockDim.x) a.rowsum[t] = 0ull;
+  float (*red)[4][66] = reinterpret_cast<float (*)[4][66]>(&sm.p2.red);  // acc[i] of lane l: element (4 (l / 16) + i, l % 16)
+#pragma unroll
+  for (int i = 0; i < 4; ++i) red[w][i][lane] = acc[i];
+  __syncthreads();
+  late(muc_d);
+  late(p0);
+  const int ri = r & 3, rl = 16 * (r >> 2) + c;
+  const float phh = red[0][ri][rl] + red[1][ri][rl], t = red[2][ri][rl] + red[3][ri][rl];
+  const float v = step_value(p0, a.eta, a.theta, phh, t, 1.f / (float)a.nb, (float)muc_d, sm.p2.cmu[c]);
+  a.out[(i0 + r) * kp + j0 + c] = v;
+  sm.p2.S.t[c][r] = v;
+  __syncthreads();
+  a.outT[(j0 + r) * kp + i0 + c] = sm.p2.S.t[r][c];
 }
 
 // The Newton-Schulz scale guard c = min(1, sqrt(2 / ||G||_inf)) from the row sums of |G|, computed
@@ -1131,6 +1272,7 @@ __device__ __forceinline__ void phase_tile(const typename ArgsOf<PHASE>::type& a
   constexpr bool SPLIT = KMODE == MM_BF16X3;
   if constexpr (PHASE == PH_P1) p1_tile<DMODE, KMODE, TY, TPH>(a, tile, sm, log);
   else if constexpr (PHASE == PH_P2) p2_tile<DMODE, KMODE, TY, TPH>(a, tile, sm);
+  else if constexpr (PHASE == PH_P2S) p2_quad_tile(a, tile, sm);
   else if constexpr (PHASE == PH_GRAM) gram_tile<KMODE>(a, tile, sm);
   else if constexpr (PHASE == PH_QPOLY) qpoly_tile<KMODE>(a, tile, sm);
   else if constexpr (PHASE == PH_UPDATE) update_tile<KMODE>(a, tile, sm);
@@ -1164,7 +1306,8 @@ __device__ inline bool stop_test(const StopArgs& a, int64_t t, double f) {
 // with the products taken out, UPDATE kept 6.8 of its 9.2 us at k = 500 (P1 5.6 of 10.4, P2 4.6 of 8.9, GRAM 4.0
 // of 6.3) -- argument and guard loads that came back one after another, sums through LDS shuffles ahead of the stores.
 // Arguments resolved on the host, independent loads and sums in registers after the stores took a step at k = 500 from
-// 55 to 48 us (UPDATE 9.2 -> 6.5) and at k = 100 in FP32 from 45 to 39.
+// 55 to 48 us (UPDATE 9.2 -> 6.5) and at k = 100 in FP32 from 45 to 39; loads that stay in flight past the next group's
+// MFMAs (pipelined) and P2's smaller FP32 tiles took it on to 44 and 28.
 // With the end test on (STOP), every phase of step g = base + st first checks whether the loop
 // has ended; P1 of each step but a run's first forms the previous step's log entry in every wave
 // (its kernels have finished), workgroup 0 stores it, and every workgroup applies the test to it and
@@ -1209,7 +1352,8 @@ __global__ __launch_bounds__(kThreads, PHASE == PH_P1 ? 3 : 1) void stgd_phase_k
 //   wave 7      c_mu; the log entry of the previous step
 // The rows of Y of the next step are loaded during the Newton-Schulz iterations. One compute unit bounds the
 // minibatch: b = 512 takes about 9 us per step, beyond it (and beyond the LDS that holds C_g) the phase kernels
-// spread the work. SMALLMEAS
+// spread the work. At k = 10, b = 100 it takes 6.5 us (the phase kernels 27); the whole detection of a graph of 1000
+// nodes, 200 epochs, 57 -> 20 ms.
 constexpr int kSmallB = 512;        // largest padded minibatch
 constexpr int kSmallThreads = 512;
 
@@ -1777,7 +1921,8 @@ struct StepPlan {
         p.c1 = a.c1;
         break;
       }
-      case PH_P2: {
+      case PH_P2:
+      case PH_P2S: {
         P2Args& p = out.p2;
         p.phi_op = op(B.phi[cur], B.phi16[cur]);
         p.h_op = op(B.h, B.h16);
@@ -1963,6 +2108,15 @@ static bool step_renorms(int64_t gstep, int32_t renorm_every, int32_t ns_iters) 
   return renorm_every > 0 && ((gstep + 1) % renorm_every == 0) && ns_iters > 0;
 }
 
+// Whether P2 of an FP32 instance takes 16 x 16 tiles (without the log of Phi~, which is by 32 x 32 tiles). They load
+// each operand twice as often and win while they leave the chip's load paths idle; at b = 1024, 16 x 16 against
+// 32 x 32: 8.4 and 11.2 us at kp = 320, 11.6 and 11.2 at kp = 384, 15.9 and 11.9 at kp = 512.
+constexpr int kQuadTiles = 100;  // of 32 x 32: kp <= 320
+template <int DMODE>
+static bool p2_spread(const StgdArgs& a) {
+  return DMODE == MM_F32 && !a.frob_pre && phase_tiles(PH_P2, a.kp, a.b) <= kQuadTiles;
+}
+
 bool stgd_small_fits(const StgdArgs& a) {
   return a.k <= 32 && a.kp == 64 && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
 }
@@ -2029,7 +2183,7 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
   int64_t yrow0 = 0;
   int32_t nb = 0;
   auto launch = [&](int phase, int it) -> int {
-    const dim3 grid(phase_tiles(phase, kp, args.b)), block(kThreads);
+    const dim3 grid(phase_tiles(phase, kp, args.b) * (phase == PH_P2S ? 4 : 1)), block(kThreads);
     const int64_t st = stop.st;
     const PhaseArgs a = P.resolve(phase, it, cur, yrow0, nb, frob_log + st, st > 0 ? frob_log + st - 1 : nullptr, frob_log, nsteps);
 #define MMSB_PHASE(PH)                                                                                                      \
@@ -2043,6 +2197,14 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
       MMSB_PHASE(PH_SETUP)
       MMSB_PHASE(PH_P1)
       MMSB_PHASE(PH_P2)
+      case PH_P2S:
+        if constexpr (DMODE == MM_F32) {
+          if (stop.stop)
+            hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_P2S, true>), grid, block, 0, s, a.p2, stop);
+          else
+            hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_P2S, false>), grid, block, 0, s, a.p2, stop);
+        }
+        break;
       MMSB_PHASE(PH_GRAM)
       MMSB_PHASE(PH_UPDATE)
       MMSB_PHASE(PH_QPOLY)
@@ -2065,7 +2227,7 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
     if (args.y_window) MMSB_TRY(fill(row0, nb));
     MMSB_TRY(launch(PH_P1, 0));
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[1], s));
-    MMSB_TRY(launch(PH_P2, 0));
+    MMSB_TRY(launch(p2_spread<DMODE>(args) ? PH_P2S : PH_P2, 0));
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[2], s));
     if (renorm && renorm_every > 0 && (gstep + 1) % renorm_every == 0) {
       MMSB_TRY(renorm(B.phit, B.phia));
