@@ -1,0 +1,24 @@
+// Device memory of contexts and their transient staging. Blocks given back are kept for later allocations, up to
+// kDevCacheBytes per process: a context of 29079 nodes per partition with k = 100 holds 125 blocks (450 MB), whose
+// hipMalloc and hipFree took 2.4 and 9.5 ms of a 37 ms detection when graphs are worked on one after another. The
+// cache is emptied with the last live context (release_device_cache), and by an allocation that fails.
+#pragma once
+
+#include <hip/hip_runtime_api.h>
+
+#include <cstddef>
+
+namespace mmsb {
+
+constexpr size_t kDevCacheBytes = (size_t)1 << 30;
+
+// hipMalloc on the current device. The contents are undefined.
+hipError_t dev_alloc(void** p, size_t bytes);
+// Gives back a block of dev_alloc (null: nothing). No work that uses it may be in flight on any stream: it may be
+// handed to another context, thread or stream at once.
+void dev_free(void* p);
+// Bytes kept for the current device, part of what a new allocation can use beyond hipMemGetInfo's free bytes.
+size_t dev_cached_bytes();
+void release_device_cache();
+
+}  // namespace mmsb

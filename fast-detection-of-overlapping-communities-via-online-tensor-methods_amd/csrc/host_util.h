@@ -27,6 +27,11 @@ inline int default_threads() {
   return (int)std::max(1u, std::min(h, 16u));
 }
 
+// One thread per `per` items of n: a thread takes about 15 us to start, one after another.
+inline int threads_for(int64_t n, int64_t per) {
+  return (int)std::max<int64_t>(1, std::min<int64_t>((n + per - 1) / per, default_threads()));
+}
+
 // Calls fn(lo, hi) on `threads` contiguous sub-ranges of [0, n).
 // Runs fn(chunk, lo, hi) for the min(threads, n) static chunks [n c / t, n (c + 1) / t) of [0, n),
 // one thread each. Per-thread state must be indexed by the chunk argument: recovering it from lo

@@ -33,6 +33,7 @@
 #include <vector>
 
 #include "dense.h"
+#include "devmem.h"
 #include "host_util.h"
 #include "mmsb_stpm.h"
 #include "post.h"
@@ -159,7 +160,7 @@ static int dalloc(mmsb_ctx* c, T*& p, size_t count) {
   if (p) return MMSB_OK;
   void* q = nullptr;
   const size_t bytes = std::max<size_t>(count, 1) * sizeof(T);
-  hipError_t e = hipMalloc(&q, bytes);
+  hipError_t e = dev_alloc(&q, bytes);
   if (e != hipSuccess)
     return set_error(MMSB_ERR_NOMEM, "hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
   HCHK(hipMemsetAsync(q, 0, bytes, c->s));
@@ -174,7 +175,7 @@ static void dfree(mmsb_ctx* c, T*& p) {
   (void)hipStreamSynchronize(c->s);
   auto it = std::find(c->allocs.begin(), c->allocs.end(), (void*)p);
   if (it != c->allocs.end()) c->allocs.erase(it);
-  (void)hipFree(p);
+  dev_free(p);
   p = nullptr;
 }
 
@@ -482,6 +483,7 @@ static int choose_y_window(mmsb_ctx* c, bool& window) {
   }
   size_t free_b = 0, total_b = 0;
   HCHK(hipMemGetInfo(&free_b, &total_b));
+  free_b += dev_cached_bytes();
   const double need = resident_bytes(c);
   window = need > 0.9 * (double)free_b;
   if (window && c->cfg.csr_host)
@@ -696,7 +698,7 @@ static int ensure_frob(mmsb_ctx* c, int64_t more) {
   if (c->steps_done + more <= c->frob_cap) return MMSB_OK;
   int64_t cap = std::max<int64_t>(1024, 2 * (c->steps_done + more));
   double* nf = nullptr;
-  HCHK(hipMalloc(&nf, sizeof(double) * cap));
+  HCHK(dev_alloc(reinterpret_cast<void**>(&nf), sizeof(double) * cap));
   HCHK(hipMemsetAsync(nf, 0, sizeof(double) * cap, c->s));
   if (c->frob && c->steps_done)
     HCHK(hipMemcpyAsync(nf, c->frob, sizeof(double) * c->steps_done, hipMemcpyDeviceToDevice, c->s));
@@ -704,7 +706,7 @@ static int ensure_frob(mmsb_ctx* c, int64_t more) {
     HCHK(hipStreamSynchronize(c->s));
     auto it = std::find(c->allocs.begin(), c->allocs.end(), (void*)c->frob);
     if (it != c->allocs.end()) c->allocs.erase(it);
-    HCHK(hipFree(c->frob));
+    dev_free(c->frob);
   }
   c->allocs.push_back(nf);
   c->frob = nf;
@@ -1287,7 +1289,7 @@ static int copy_raw(mmsb_ctx* c, const View& v, void* host) {
   if (v.ld == inner) return d2h(c->s, host, v.p, bytes);
   const int64_t slab = std::max<int64_t>(1, std::min<int64_t>(outer, ((int64_t)256 << 20) / std::max<int64_t>(1, inner * esz)));
   void* d = nullptr;
-  HCHK(hipMalloc(&d, std::max<size_t>((size_t)slab * inner * esz, 1)));
+  HCHK(dev_alloc(&d, std::max<size_t>((size_t)slab * inner * esz, 1)));
   int st = MMSB_OK;
   for (int64_t o = 0; o < outer && st == MMSB_OK; o += slab) {
     const int64_t m = std::min<int64_t>(slab, outer - o);
@@ -1296,7 +1298,8 @@ static int copy_raw(mmsb_ctx* c, const View& v, void* host) {
     if (e != hipSuccess) st = set_error(MMSB_ERR_HIP, "copy_out: %s", hipGetErrorString(e));
     if (st == MMSB_OK) st = d2h(c->s, static_cast<unsigned char*>(host) + (size_t)o * inner * esz, d, (size_t)m * inner * esz);
   }
-  (void)hipFree(d);
+  if (st != MMSB_OK) (void)hipStreamSynchronize(c->s);
+  dev_free(d);
   return st;
 }
 
@@ -1445,6 +1448,7 @@ static void release_process_resources() {
   release_staging();
   release_streamer();
   release_sort_scratch();
+  release_device_cache();
 }
 
 extern "C" int mmsb_create(const stpm_config* cfg, mmsb_ctx** out) {
@@ -1491,7 +1495,8 @@ extern "C" void mmsb_destroy(mmsb_ctx* c) {
     for (auto& row : plane)
       for (hipGraphExec_t& g : row)
         if (g) (void)hipGraphExecDestroy(g);
-  for (void* p : c->allocs) (void)hipFree(p);
+  if (!c->allocs.empty()) (void)hipDeviceSynchronize();  // a batch's stream may still use the blocks
+  for (void* p : c->allocs) dev_free(p);
   if (StgdSmallCtl* ctl = c->small_ctl.load()) (void)hipHostFree(ctl);
   if (c->s) (void)hipStreamDestroy(c->s);
   delete c;
@@ -1508,9 +1513,9 @@ extern "C" int mmsb_set_block(mmsb_ctx* c, int32_t which, const mmsb_csr* b) {
   MMSB_CHECK_ARG(b->nnz >= 0 && b->nnz < INT32_MAX && b->rowptr && (b->nnz == 0 || b->colidx), "set_block: bad CSR");
   MMSB_CHECK_ARG(b->rowptr[0] == 0 && b->rowptr[b->n_rows] == b->nnz, "set_block: rowptr does not match nnz");
   {  // every row pointer monotone, every column index in range (threads report the first bad index)
-    const int nt = default_threads();
+    const int nt = threads_for(b->nnz + b->n_rows, 300000);
     std::vector<int64_t> bad_row(nt, -1), bad_nz(nt, -1);
-    parallel_chunks(b->n_rows, nt, [&](int t, int64_t lo, int64_t hi) {
+    parallel_chunks(b->n_rows, threads_for(b->n_rows, 300000), [&](int t, int64_t lo, int64_t hi) {
       for (int64_t i = lo; i < hi && bad_row[t] < 0; ++i)
         if (b->rowptr[i + 1] < b->rowptr[i]) bad_row[t] = i;
     });
@@ -1795,15 +1800,16 @@ extern "C" int mmsb_power_method(mmsb_ctx* c, int32_t iters, int32_t orthogonali
   void* work = nullptr;
   auto cleanup = [&]() {
     for (void* p : {(void*)dphi, (void*)dlam, (void*)yr[0], (void*)yr[1], (void*)yr[2], work})
-      if (p) (void)hipFree(p);
+      dev_free(p);
   };
-  hipError_t e = hipMalloc(&dphi, sizeof(double) * k * k);
-  if (e == hipSuccess) e = hipMalloc(&dlam, sizeof(double) * k);
+  hipError_t e = dev_alloc(reinterpret_cast<void**>(&dphi), sizeof(double) * k * k);
+  if (e == hipSuccess) e = dev_alloc(reinterpret_cast<void**>(&dlam), sizeof(double) * k);
   for (int i = 0; i < (c->have_y ? 1 : 3); ++i)
-    if (e == hipSuccess) e = hipMalloc(&yr[i], sizeof(float) * (size_t)chunk * kp);
-  if (e == hipSuccess) e = hipMalloc(&work, power_workspace_bytes(k, c->n[0], chunk));
+    if (e == hipSuccess) e = dev_alloc(reinterpret_cast<void**>(&yr[i]), sizeof(float) * (size_t)chunk * kp);
+  if (e == hipSuccess) e = dev_alloc(&work, power_workspace_bytes(k, c->n[0], chunk));
   if (e == hipSuccess) e = hipMemcpyAsync(dphi, hd.data(), sizeof(double) * k * k, hipMemcpyHostToDevice, c->s);
   if (e != hipSuccess) {
+    (void)hipStreamSynchronize(c->s);
     cleanup();
     return set_error(MMSB_ERR_NOMEM, "power_method: %s", hipGetErrorString(e));
   }
@@ -1841,9 +1847,8 @@ extern "C" int mmsb_power_method(mmsb_ctx* c, int32_t iters, int32_t orthogonali
     if (e == hipSuccess) e = hipMemcpyAsync(lambda, dlam, sizeof(double) * k, hipMemcpyDeviceToHost, c->s);
     if (e == hipSuccess) e = hipStreamSynchronize(c->s);
     if (e != hipSuccess) st = set_error(MMSB_ERR_HIP, "power_method: %s", hipGetErrorString(e));
-  } else {
-    (void)hipStreamSynchronize(c->s);
   }
+  if (st != MMSB_OK) (void)hipStreamSynchronize(c->s);
   cleanup();
   if (st != MMSB_OK) return st;
   if (iters == 0) std::fill(lambda, lambda + k, 0.0);
@@ -1885,7 +1890,7 @@ static int yrows_host(mmsb_ctx* c, int32_t what, int64_t row0, int64_t nrows, do
   const int32_t k = c->k, kp = c->kp;
   const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(nrows, 65536));
   float* d = nullptr;
-  HCHK(hipMalloc(&d, sizeof(float) * (size_t)chunk * kp));
+  HCHK(dev_alloc(reinterpret_cast<void**>(&d), sizeof(float) * (size_t)chunk * kp));
   std::vector<float> h((size_t)chunk * kp);
   const float* R[3] = {c->W, c->MB, c->MC};
   const DevCsr& g = c->blk[i];
@@ -1901,7 +1906,8 @@ static int yrows_host(mmsb_ctx* c, int32_t what, int64_t row0, int64_t nrows, do
       for (int64_t x = 0; x < m; ++x)
         for (int32_t j = 0; j < k; ++j) host[(r + x) * k + j] = h[(size_t)x * kp + j];
   }
-  (void)hipFree(d);
+  if (st != MMSB_OK) (void)hipStreamSynchronize(c->s);
+  dev_free(d);
   return st;
 }
 }  // namespace mmsb

@@ -54,8 +54,7 @@ int ensure(Stager& st) {
 }
 
 void par_copy(void* dst, const void* src, size_t n) {
-  const int threads = n >= ((size_t)4 << 20) ? default_threads() : 1;
-  parallel_for((int64_t)n, threads, [&](int64_t lo, int64_t hi) {
+  parallel_for((int64_t)n, threads_for((int64_t)n, 1 << 20), [&](int64_t lo, int64_t hi) {
     std::memcpy(static_cast<char*>(dst) + lo, static_cast<const char*>(src) + lo, (size_t)(hi - lo));
   });
 }
