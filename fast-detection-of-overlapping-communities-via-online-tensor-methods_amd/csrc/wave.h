@@ -102,6 +102,13 @@ __device__ inline float wave_max(float v) {
   return fmaxf(fmaxf(read_lane(v, 0), read_lane(v, 16)), fmaxf(read_lane(v, 32), read_lane(v, 48)));
 }
 
+// Exchanges the upper half of a with the lower half of b.
+__device__ inline void half_swap(float& a, float& b) {
+  const auto x = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), false, false);
+  a = __builtin_bit_cast(float, (uint32_t)x[0]);
+  b = __builtin_bit_cast(float, (uint32_t)x[1]);
+}
+
 // Sums over the lanes of a quad, and of a group of eight (offsets 1, 2, 4).
 __device__ inline float quad_sum(float v) {
 #pragma clang fp contract(off)
