@@ -1353,7 +1353,7 @@ __global__ __launch_bounds__(kThreads, PHASE == PH_P1 ? 3 : 1) void stgd_phase_k
 // The rows of Y of the next step are loaded during the Newton-Schulz iterations. One compute unit bounds the
 // minibatch: b = 512 takes about 9 us per step, beyond it (and beyond the LDS that holds C_g) the phase kernels
 // spread the work. At k = 10, b = 100 it takes 6.5 us (the phase kernels 27); the whole detection of a graph of 1000
-// nodes, 200 epochs, 57 -> 20 ms.
+// nodes, 200 epochs, 57 -> 20 ms (FP32 at k <= 16 goes to stgd_small16_kernel).
 constexpr int kSmallB = 512;        // largest padded minibatch
 constexpr int kSmallThreads = 512;
 
@@ -1862,14 +1862,17 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
 // ---- the same for k <= 16 in FP32: one 16 x 16 block -----------------------------------------------------
 // Matrices live in registers in accumulator layout (lane l: rows 4 (l / 16) + i, column l % 16, i = 0 .. 3). Read as
 // "row l % 16, columns 4 (l / 16) + i" the same registers are the transposed matrix as an MFMA operand, up to the
-// exchange of half-waves that gives the k order of the 32 x 32 products (tile_frag). So wave 4 keeps Phi and Phi^T, each
+// exchange of half-waves that gives the k order of the 32 x 32 products (tile_frag). So one wave keeps Phi and Phi^T, each
 // product with a symmetric matrix is taken for both (the same products in the same order, so each stays the exact
 // transpose of the other), and a Newton-Schulz iteration is three short MFMA chains with nothing through LDS. Y_A, Y_B
-// and Y_C^T are loaded in operand layout by the same reading. A step at k = 10, b = 100 takes T16 us against 6.5 in the
-// 32-wide kernel, whose chains are four times as long and pass every matrix through LDS.
+// and Y_C^T are loaded in operand layout by the same reading. A step at k = 10, b = 100 takes 3.0 us against 6.5 in the
+// 32-wide kernel, whose chains are four times as long and pass every matrix through LDS; what is left is latency, about
+// 1000 cycles each of P_A, P_B, of Y_C^T C_g and of an iteration. Twelve waves: eight for P_A, P_B, C_g in units of 16
+// rows, one that owns Phi, two for the halves of Y_C^T C_g, one for c_mu and the log (with four, two and the owner, the
+// log ahead of the first barrier: 3.3 us).
 struct Small16Shm {
   floatx4 phi[64];           // Phi in accumulator layout
-  float phif[2][16][20];     // Phi by rows, this step's and the next
+  float phif[3][16][20];     // Phi by rows: the previous step's, this one's and the next
   floatx4 t[2][64];          // halves of Y_C^T C_g in accumulator layout
   float tr[2][16][20];       // and by rows
   float cs[kSmallB / 16][16];
@@ -1901,12 +1904,15 @@ __device__ inline floatx4 tile_mm(const floatx4& a, const floatx4& b) {
   return acc + 0.f;
 }
 
-__global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArgs a) {
+constexpr int kSmall16Threads = 768;
+
+__global__ __launch_bounds__(kSmall16Threads, 1) void stgd_small16_kernel(SmallArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char small_raw[];
   Small16Shm& S = *reinterpret_cast<Small16Shm*>(small_raw);
-  constexpr int PF = kSmallB / 64;  // groups of 32 minibatch rows of one of the waves 5, 6
+  constexpr int P1W = 8, OWNER = 8, P2A = 9, P2B = 10, AUX = 11;  // roles of the waves
+  constexpr int PF = 4;                                          // P2: groups of 32 minibatch rows loaded ahead
   const int w = wave_id(), lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
-  const int kp = a.kp, b = a.b, nt = b / 32, ldc = b + 4;
+  const int kp = a.kp, b = a.b, nt = b / 32, nu = b / 16, ldc = b + 4;
   const float* ya = static_cast<const float*>(a.ya);
   const float* yb = static_cast<const float*>(a.yb);
   const float* yct = static_cast<const float*>(a.yct);
@@ -1914,34 +1920,37 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
 
   int64_t pos = a.step0 % a.spe;
   int rn = a.renorm_every > 0 ? (int)(a.step0 % a.renorm_every) : 0;
-  const int g0 = w == 6 ? nt / 2 : 0, g1 = w == 5 ? nt / 2 : nt;  // waves 5, 6: groups [g0, g1)
-  floatx4 ra[2], rb[2];   // waves 0 .. 3: the next tile's rows of Y_A, Y_B (two halves)
-  floatx4 yc[PF][2];      // waves 5, 6: Y_C^T of the groups
-  auto load_tile = [&](int64_t row0, int tile) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t at = (row0 + 32 * tile + 16 * h + c) * kp + 4 * g;
-      ra[h] = *reinterpret_cast<const floatx4*>(ya + at);
-      rb[h] = *reinterpret_cast<const floatx4*>(yb + at);
-    }
+  const bool p2w = w == P2A || w == P2B;
+  const int g0 = w == P2B ? nt / 2 : 0, ng = nt / 2;  // P2: groups [g0, g0 + ng)
+  floatx4 ra, rb;         // P1: the next 16 rows of Y_A, Y_B
+  floatx4 yc[PF][2];      // P2: Y_C^T of the groups
+  auto load_rows = [&](int64_t row0, int u) {
+    const int64_t at = (row0 + 16 * u + c) * kp + 4 * g;
+    ra = *reinterpret_cast<const floatx4*>(ya + at);
+    rb = *reinterpret_cast<const floatx4*>(yb + at);
   };
-  auto prefetch = [&](int64_t row0) {
-    if (w < 4) {
-      if (w < nt) load_tile(row0, w);
-    } else if (w == 5 || w == 6) {
-      const bool aligned = row0 % 4 == 0;
+  auto load_groups = [&](int64_t row0, int u0) {  // groups u0 .. u0 + PF - 1 of this wave
+    const float* p = yct + c * a.n_pad + row0 + 32 * (g0 + u0) + 4 * g;
+    auto load = [&](auto aligned) {
 #pragma unroll
       for (int u = 0; u < PF; ++u)
-        if (g0 + u < g1)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            const float* p = yct + c * a.n_pad + row0 + 32 * (g0 + u) + 16 * h + 4 * g;
-            yc[u][h] = __builtin_bit_cast(floatx4, aligned ? ld16<true>(p) : ld16<false>(p));
-          }
+        if (u0 + u < ng) {
+          yc[u][0] = __builtin_bit_cast(floatx4, ld16<decltype(aligned)::value>(p + 32 * u));
+          yc[u][1] = __builtin_bit_cast(floatx4, ld16<decltype(aligned)::value>(p + 32 * u + 16));
+        }
+    };
+    if (row0 % 4 == 0) load(std::true_type());
+    else load(std::false_type());
+  };
+  auto prefetch = [&](int64_t row0) {
+    if (w < P1W) {
+      if (w < nu) load_rows(row0, w);
+    } else if (p2w) {
+      load_groups(row0, 0);
     }
   };
   // as in the 32-wide kernel: the rows and columns from 16 on are zero
-  auto log_entry = [&](int64_t st, int now) {
+  auto log_entry = [&](int64_t st, int now, int before) {
     double f[2];
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
@@ -1950,7 +1959,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
       if (c4 < 16)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-          const double dd = (double)S.phif[now][r][c4 + e] - (double)S.phif[now ^ 1][r][c4 + e];
+          const double dd = (double)S.phif[now][r][c4 + e] - (double)S.phif[before][r][c4 + e];
           d = fma(dd, dd, d);
         }
       f[q] = wave_sum(d);
@@ -1958,7 +1967,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
     if (lane == 0) a.frob[st] = f[0] + f[1];
   };
 
-  // wave 4: Phi and Phi^T in accumulator layout; mu_A, mu_B, mu_C of the rows 4 g + i and mu_C of row c
+  // OWNER: Phi and Phi^T in accumulator layout; mu_A, mu_B, mu_C of the rows 4 g + i and mu_C of row c
   floatx4 x = {}, xt = {}, ua = {}, ub = {}, uc = {};
   float uct = 0.f;
   auto new_phi = [&](int buf) {
@@ -1974,7 +1983,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
     const float m = swap_add32(ma, mb) + 0.f;  // m_A in the lower half, m_B in the upper
     if ((g & 1) == 0) S.mv[g >> 1][c] = m;
   };
-  if (w == 4) {
+  if (w == OWNER) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       x[i] = a.phi0[(4 * g + i) * kp + c];
@@ -1989,7 +1998,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
   prefetch(pos * a.bl);
   __syncthreads();
 
-  int cur = 0;
+  int cur = 0;       // S.phif[cur] holds Phi, the buffer before it (of three) the previous one
   int64_t st = 0;
   while (true) {
     const int64_t row0 = pos * a.bl;
@@ -1999,79 +2008,75 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
     if (renorm) rn = 0;
     const bool poll = pos == 0 && st + 1 < a.nsteps;
     int stop = 0;
-    if (poll && w == 7) stop = __hip_atomic_load(&a.ctl->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-    floatx4 ph = {}, pht = {};  // wave 4: Phi H and its transpose
-    // P_A, P_B, C_g; Phi H; the previous step's log entry
-    if (w < 4) {
+    if (poll && w == AUX) stop = __hip_atomic_load(&a.ctl->stop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    const float inv_b = 1.f / (float)nb;
+    floatx4 ph = {}, pht = {};  // OWNER: Phi H and its transpose
+    // P_A, P_B, C_g; Phi H
+    if (w < P1W) {
       const float mA = S.mv[0][c], mB = S.mv[1][c];
       const floatx4 phi = tile_frag(S.phi[lane]);
-      for (int tile = w; tile < nt; tile += 4) {
-        floatx4 xa[2], xb[2], pa[2] = {}, pb[2] = {};
+      for (int u = w; u < nu; u += P1W) {
+        const floatx4 xa = tile_frag(ra), xb = tile_frag(rb);
+        if (u + P1W < nu) load_rows(row0, u + P1W);
+        floatx4 pa = {}, pb = {};
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          xa[h] = tile_frag(ra[h]);
-          xb[h] = tile_frag(rb[h]);
+        for (int e = 0; e < 4; ++e) {
+          pa = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[e], phi[e], pa, 0, 0, 0);
+          pb = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[e], phi[e], pb, 0, 0, 0);
         }
-        if (tile + 4 < nt) load_tile(row0, tile + 4);
+        float cg[4], cs = 0.f;
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int h = 0; h < 2; ++h) {
-            pa[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[h][e], phi[e], pa[h], 0, 0, 0);
-            pb[h] = __builtin_amdgcn_mfma_f32_16x16x4f32(xb[h][e], phi[e], pb[h], 0, 0, 0);
-          }
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          float cg[4], cs = 0.f;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const int row = 32 * tile + 16 * h + 4 * g + e;
-            const float p = pa[h][e] + 0.f, r = pb[h][e] + 0.f;
-            const bool valid = row < nb;
-            const float ab = p * r;
-            {
+        for (int e = 0; e < 4; ++e) {
+          const float p = pa[e] + 0.f, r = pb[e] + 0.f;
+          const bool valid = 16 * u + 4 * g + e < nb;
+          const float ab = p * r;
+          {
 #pragma clang fp contract(off)
-              cs += valid ? ab : 0.f;
-            }
-            cg[e] = valid ? cg_value(a.c3, a.c1, p, r, ab, mA, mB) : 0.f;
+            cs += valid ? ab : 0.f;
           }
-          store4(cgt + c * ldc + 32 * tile + 16 * h + 4 * g, cg);
-          const float t = swap_add16(cs, cs);
-          const float u = swap_add32(t, t);
-          if (g == 0) S.cs[2 * tile + h][c] = u;
+          cg[e] = valid ? cg_value(a.c3, a.c1, p, r, ab, mA, mB) : 0.f;
         }
+        store4(cgt + c * ldc + 16 * u + 4 * g, cg);
+        const float t = swap_add16(cs, cs), v = swap_add32(t, t);
+        if (g == 0) S.cs[u][c] = v;
       }
-    } else if (w == 4) {
+    } else if (w == OWNER) {
       const floatx4 f = tile_frag(x), ft = tile_frag(xt);
       const floatx4 gr = tile_mm(f, f);
       const floatx4 fh = tile_frag(gr * gr);
       ph = tile_mm(ft, fh);
       pht = tile_mm(fh, ft);
-    } else if (w == 5 || w == 6) {
+    } else if (p2w) {
 #pragma unroll
       for (int u = 0; u < PF; ++u)
-        if (g0 + u < g1)
+        if (u < ng)
 #pragma unroll
           for (int h = 0; h < 2; ++h) yc[u][h] = tile_frag(yc[u][h]);
-    } else if (st > 0) {
-      log_entry(st - 1, cur);
     }
     __syncthreads();
     // the halves of Y_C^T C_g, c_mu
-    if (w == 5 || w == 6) {
+    if (p2w) {
       floatx4 acc = {};
+      const float* p = cgt + c * ldc + 32 * g0 + 4 * g;
+      for (int u0 = 0; u0 < ng; u0 += PF) {
+        if (u0 > 0) load_groups(row0, u0);
+        floatx4 y[PF][2];
 #pragma unroll
-      for (int u = 0; u < PF; ++u)
-        if (g0 + u < g1) {
-          const float* p = cgt + c * ldc + 32 * (g0 + u) + 4 * g;
-          const floatx4 y0 = *reinterpret_cast<const floatx4*>(p), y1 = *reinterpret_cast<const floatx4*>(p + 16);
-          tile_mma(acc, yc[u][0], tile_frag(y0));
-          tile_mma(acc, yc[u][1], tile_frag(y1));
+        for (int u = 0; u < PF; ++u) {
+          const float* q = p + 32 * min(u0 + u, ng - 1);
+          y[u][0] = *reinterpret_cast<const floatx4*>(q);
+          y[u][1] = *reinterpret_cast<const floatx4*>(q + 16);
         }
-      S.t[w - 5][lane] = acc;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) S.tr[w - 5][4 * g + i][c] = acc[i];
-    } else if (w == 7) {
+        for (int u = 0; u < PF; ++u)
+          if (u0 + u < ng)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) tile_mma(acc, u0 > 0 ? tile_frag(yc[u][h]) : yc[u][h], tile_frag(y[u][h]));
+      }
+      S.t[w - P2A][lane] = acc;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) S.tr[w - P2A][4 * g + i][c] = acc[i];
+    } else if (w == AUX) {
       float m[8];
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
@@ -2083,11 +2088,16 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
       if (g == 0) S.cmu[c] = cmu_value(a.c0, a.c1, S.mv[0][c], S.mv[1][c], ssum, nb);
     }
     __syncthreads();
-    // Phi~ and the renormalisation (wave 4) under the next step's loads
-    if (st + 1 < a.nsteps) prefetch(pos * a.bl);
-    if (poll && w == 7 && lane == 0) S.stop = stop;
-    if (w == 4) {
-      const float inv_b = 1.f / (float)nb, cmu = S.cmu[c];
+    // Phi~ and the renormalisation (OWNER) under the next step's loads and the previous step's log entry
+    const int next = cur == 2 ? 0 : cur + 1;
+    if (w != OWNER) {
+      if (st + 1 < a.nsteps) prefetch(pos * a.bl);
+      if (w == AUX) {
+        if (poll && lane == 0) S.stop = stop;
+        if (st > 0) log_entry(st - 1, cur, cur == 0 ? 2 : cur - 1);
+      }
+    } else {
+      const float cmu = S.cmu[c];
       const floatx4 cmut = *reinterpret_cast<const floatx4*>(&S.cmu[4 * g]);
       const floatx4 t0 = S.t[0][lane], t1 = S.t[1][lane];
       const floatx4 r0 = *reinterpret_cast<const floatx4*>(&S.tr[0][c][4 * g]);
@@ -2133,19 +2143,19 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small16_kernel(SmallArg
           }
         }
       }
-      new_phi(cur ^ 1);
+      new_phi(next);
     }
-    cur ^= 1;
+    cur = next;
     ++st;
     __syncthreads();
     if (st == a.nsteps || (poll && S.stop)) break;
   }
-  if (w == 7) {
-    log_entry(st - 1, cur);
+  if (w == AUX) {
+    log_entry(st - 1, cur, cur == 0 ? 2 : cur - 1);
     if (lane == 0) a.ctl->ran = st;
   }
-  float* phi_out = cur ? a.phi1 : a.phi0;
-  if (w == 4)
+  float* phi_out = (st & 1) ? a.phi1 : a.phi0;
+  if (w == OWNER)
 #pragma unroll
     for (int i = 0; i < 4; ++i) phi_out[(4 * g + i) * kp + c] = x[i];
 }
@@ -2445,7 +2455,7 @@ static int run_small(hipStream_t s, const StgdArgs& args, const void* YA, const 
   a.eta = args.eta;
   a.theta = args.theta;
   if (MODE == MM_F32 && a.k <= 16) {
-    hipLaunchKernelGGL(stgd_small16_kernel, dim3(1), dim3(kSmallThreads), small16_shm_bytes(a.b), s, a);
+    hipLaunchKernelGGL(stgd_small16_kernel, dim3(1), dim3(kSmall16Threads), small16_shm_bytes(a.b), s, a);
   } else {
     const void* fn = reinterpret_cast<const void*>(stgd_small_kernel<MODE, TY>);
     MMSB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)small_shm_bytes<MODE>(kSmallB)));
