@@ -33,8 +33,8 @@ struct StgdArgs {
   float* phit;          // [kp x kp] Phi~ after the gradient step; set per step
   float* cs_part;       // [b/32 x kp] per-row-tile column sums of P_A o P_B
   float* mab;           // [2 x kp] m_A, m_B
-  int32_t y_window;     // 0: Y holds all of X; 1: Y holds the current minibatch only (rows from 0), refilled
-                        // before each step by the caller's fill callback (checkpointed STGD)
+  int32_t y_window;     // 0: Y holds all of X; 1: Y holds the rows of as many whole steps as n_pad - b leaves room
+                        // for (one at least), refilled by the caller's fill callback (checkpointed STGD)
   int32_t frob_pre;     // 1: log ||Phi~ - Phi||^2 before the renormalisation (the reference's order,
                         // stpm.c:705-743 then the QR at :774-786); 0: ||Phi_next - Phi||^2 after it
   StgdStop* stop;       // null: every step runs; else the end test below, checked per step on the device
@@ -88,8 +88,8 @@ struct StgdTiming {
 // result on exit. frob_log[st] receives ||Phi_{t+1} - Phi_t||_F^2 of the st-th step of this call.
 // precision is MMSB_PREC_FP32 (Y as float) or MMSB_PREC_BF16 (Y as BF16). Without timing every
 // launch is capturable in a HIP graph (no memset nodes, no host synchronisation).
-// With args.y_window, fill(row0, nb) is called before each step's first launch to enqueue (on s) the
-// kernels that write rows [row0, row0 + nb) of X into the Y buffers.
+// With args.y_window, fill(row0, n) is called before the first launch of a step whose rows are not in the Y buffers, to
+// enqueue (on s) the kernels that write rows [row0, row0 + n) of X into them (from row 0).
 // With a renorm callback (the reference's QR mode), a renormalising step runs P1, P2, then
 // renorm(src = bufs.phit, dst = bufs.phia) -- launches that leave the orthonormal factor of Phi~ in
 // phia -- and a QRFIN kernel that makes it the next Phi (with its derived copies).

@@ -31,9 +31,8 @@
 // in FP32. In BF16 mode every k x k operand is written by the kernel that produces it both in
 // FP32 and as its (hi, lo) BF16 pair, so the MFMA loops load ready operands and convert nothing.
 // m_A and m_B of the next step are reduced from the tiles of the new Phi where it is written.
-// Y_A, Y_B, Y_C^T either hold all of X (row offset row0) or, for checkpointed runs, only the current
-// minibatch (row offset 0, Y_C^T with leading dimension b), refilled from CSR before each step by a
-// caller-supplied launch (StgdArgs::y_window).
+// Y_A, Y_B, Y_C^T either hold all of X (row offset row0) or, for checkpointed runs, only the minibatches of
+// the next steps, refilled from CSR by a caller-supplied launch (StgdArgs::y_window).
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
@@ -2484,7 +2483,7 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
   const int64_t spe = ceil_div(args.n_x, args.bl);
   const StepPlan P{args, B, YA, YB, YCt, ns_iters, ns_degree, KMODE == MM_BF16X3};
   StopArgs stop{args.stop, 0, args.thresh, args.iter_min, args.iter_max};
-  int64_t yrow0 = 0;
+  int64_t yrow0 = 0, win0 = 0, win1 = 0;  // rows [win0, win1) of X in the window
   int32_t nb = 0;
   auto launch = [&](int phase, int it) -> int {
     const dim3 grid(phase_tiles(phase, kp, args.b) * (phase == PH_P2S ? 4 : 1)), block(kThreads);
@@ -2525,10 +2524,17 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
     const int64_t gstep = step0 + st;
     const int64_t row0 = (gstep % spe) * args.bl;
     nb = (int32_t)std::min<int64_t>(args.bl, args.n_x - row0);
-    yrow0 = args.y_window ? 0 : row0;
+    yrow0 = row0 - win0;
     stop.st = st;
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[0], s));
-    if (args.y_window) MMSB_TRY(fill(row0, nb));
+    if (args.y_window && (row0 < win0 || row0 + nb > win1)) {
+      const int64_t in_epoch = std::min<int64_t>(spe - gstep % spe, timing ? 1 : nsteps - st);  // timed phases: step by step
+      const int64_t steps = std::max<int64_t>(1, std::min<int64_t>(in_epoch, (args.n_pad - args.b) / args.bl + 1));
+      win0 = row0;
+      win1 = std::min<int64_t>(row0 + steps * args.bl, args.n_x);
+      yrow0 = 0;
+      MMSB_TRY(fill(win0, (int32_t)(win1 - win0)));
+    }
     MMSB_TRY(launch(PH_P1, 0));
     if (timing) MMSB_HIP(hipEventRecord(timing->ev[1], s));
     MMSB_TRY(launch(p2_spread<DMODE>(args) ? PH_P2S : PH_P2, 0));
