@@ -17,6 +17,7 @@
 #include "dense.h"
 #include "mfma64.h"
 #include "philox.h"
+#include "wave.h"
 
 namespace mmsb {
 
@@ -1085,19 +1086,21 @@ __global__ __launch_bounds__(256) void chol_transpose_kernel(int32_t r, const do
   }
 }
 
-// Columns [c0, c0 + kTrinvCols) of X = L^{-1} by forward substitution, one thread per row k of X
-// (blockDim >= r): b_k starts as the unit vector entries; at step i the owner of row i finalises
-// x_i = b_i / L_ii and broadcasts it through LDS (double-buffered by step parity, one barrier per
-// step), and every row k > i subtracts L_ki x_i. L_ki = R[i][k] is read along row i of R (coalesced),
-// kTrinvRing steps ahead of its use. Rows of X above a column's diagonal stay exactly zero. Writes
+// Columns [c0, c0 + kTrinvCols) of X = L^{-1} by forward substitution in blocks of 16 rows, one thread per row k of X
+// (blockDim >= r) with the block's columns in registers: b_k starts as the unit vector entries; a block's 16 rows go to
+// LDS, wave 0 solves them against the diagonal block, one lane per column, and every row below subtracts
+// L_ki x_i for i = the 16 rows in turn. Each element sees the same operations in the same order as row-by-row
+// substitution, which took a barrier, a broadcast and their latency per row: 37 us at r = 110, now 26. L_ki = R[i][k] is
+// read along row i of R (coalesced), a block ahead. Rows of X above a column's diagonal stay exactly zero. Writes
 // row c of R^{-1} (= column c of X) for each of the block's columns.
 constexpr int kTrinvCols = 16;
-constexpr int kTrinvRing = 16;
 
-__global__ __launch_bounds__(1024) void trinv_cols_kernel(int32_t r, const double* __restrict__ R,
+template <int THREADS>
+__global__ __launch_bounds__(THREADS) void trinv_cols_kernel(int32_t r, const double* __restrict__ R,
                                                           double* __restrict__ Rinv) {
-  constexpr int C = kTrinvCols, D = kTrinvRing;
-  __shared__ double xb[2][C];
+  constexpr int C = kTrinvCols, D = 16;
+  constexpr bool AHEAD = THREADS <= 512;  // registers for the next block's L
+  __shared__ double bs[D][C + 1], xs[D][C], ds[D][D + 1], inv[D];
   const int k = threadIdx.x;
   const int c0 = blockIdx.x * C;
   double b[C];
@@ -1105,30 +1108,50 @@ __global__ __launch_bounds__(1024) void trinv_cols_kernel(int32_t r, const doubl
   for (int c = 0; c < C; ++c) b[c] = (k == c0 + c) ? 1.0 : 0.0;
   const double inv_kk = k < r ? 1.0 / R[(int64_t)k * r + k] : 0.0;
   auto lval = [&](int i) -> double { return (i < r && k > i && k < r) ? R[(int64_t)i * r + k] : 0.0; };
-  double ring[D];
+  double l[D];
 #pragma unroll
-  for (int d = 0; d < D; ++d) ring[d] = lval(c0 + d);
+  for (int d = 0; d < D; ++d) l[d] = lval(c0 + d);
   for (int ib = c0; ib < r; ib += D) {
+    if (k >= ib && k < ib + D) {  // the block's rows: right-hand sides, L and 1 / L_ii
+      const int q = k - ib;
+      inv[q] = inv_kk;
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-      const int i = ib + d;
-      if (i < r) {  // uniform over the block
-        const double lki = ring[d];
-        ring[d] = lval(i + D);
-        if (k == i) {
+      for (int c = 0; c < C; ++c) bs[q][c] = b[c];
 #pragma unroll
-          for (int c = 0; c < C; ++c) {
-            b[c] *= inv_kk;
-            xb[i & 1][c] = b[c];
-          }
-        }
-        __syncthreads();
-        if (k > i) {
+      for (int d = 0; d < D; ++d) ds[d][q] = l[d];
+    }
+    __syncthreads();
+    if (k < C) {
+      double x[D];
 #pragma unroll
-          for (int c = 0; c < C; ++c) b[c] = fma(-lki, xb[i & 1][c], b[c]);
-        }
+      for (int d = 0; d < D; ++d) x[d] = bs[d][k];
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        x[d] *= inv[d];
+        xs[d][k] = x[d];
+#pragma unroll
+        for (int e = d + 1; e < D; ++e) x[e] = fma(-ds[d][e], x[d], x[e]);
       }
     }
+    double ln[AHEAD ? D : 1];
+    if constexpr (AHEAD)
+#pragma unroll
+      for (int d = 0; d < D; ++d) ln[d] = lval(ib + D + d);
+    __syncthreads();
+    if (k >= ib + D) {
+#pragma unroll
+      for (int d = 0; d < D; ++d) {
+        asm volatile("" ::: "memory");  // one row of xs at a time in registers
+#pragma unroll
+        for (int c = 0; c < C; ++c) b[c] = fma(-l[d], xs[d][c], b[c]);
+      }
+    } else if (k >= ib) {
+#pragma unroll
+      for (int c = 0; c < C; ++c) b[c] = xs[k - ib][c];
+    }
+#pragma unroll
+    for (int d = 0; d < D; ++d) l[d] = AHEAD ? ln[d] : lval(ib + D + d);
+    __syncthreads();
   }
   if (k < r) {
 #pragma unroll
@@ -1137,8 +1160,126 @@ __global__ __launch_bounds__(1024) void trinv_cols_kernel(int32_t r, const doubl
   }
 }
 
+// R of a small matrix (r <= 128: the whole triangle in LDS) in one workgroup and one launch, in place of the shift, two
+// launches per panel and the transpose: the same operations in the same order (the trace as the tree of
+// chol_shift_kernel, the diagonal block by one wave with its rows in the lanes, the rows below one per thread, the
+// trailing triangle in 4 x 4 tiles), so R is bit-identical. Bound by the chain of 2 r square roots and divisions. At
+// r = 110: 65 us against 15 launches of 125 us. Reads G, leaves it as it is.
+constexpr int kCholSmall = 128;
+
+__global__ __launch_bounds__(kCholThreads) void chol_small_kernel(int32_t r, const double* __restrict__ G, double shift,
+                                                                  double* __restrict__ R, int32_t* __restrict__ status) {
+  extern __shared__ double Ls[];  // [r][ld], the lower triangle
+  __shared__ double sh;
+  const int ld = r | 1, t = threadIdx.x, w = t >> 6, lane = t & 63;
+  for (int i = w; i < r; i += kCholThreads / 64)
+    for (int l = lane; l <= i; l += 64) Ls[i * ld + l] = G[(int64_t)i * r + l];
+  __syncthreads();
+  if (w == 0) {
+    const double d0 = lane < r ? Ls[lane * ld + lane] : 0.0, d1 = lane + 64 < r ? Ls[(lane + 64) * ld + lane + 64] : 0.0;
+    const double v = shift * wave_sum(d0 + d1);
+    if (lane == 0) sh = v > 0.0 ? v : 1e-300;
+  }
+  __syncthreads();
+  if (t < r) Ls[t * ld + t] += sh;
+  __syncthreads();
+  int bad = 0;
+  for (int j0 = 0; j0 < r; j0 += kCholP) {
+    const int pb = min(kCholP, r - j0), base = j0 + pb, m = r - base;
+    if (w == 0) {  // lane a holds row a of the diagonal block
+      const int a = lane & (kCholP - 1);
+      double D[kCholP];
+#pragma unroll
+      for (int b = 0; b < kCholP; ++b) D[b] = (a < pb && b <= a) ? Ls[(j0 + a) * ld + j0 + b] : 0.0;
+#pragma unroll
+      for (int c = 0; c < kCholP; ++c) {
+        if (c < pb) {
+          const double d = read_lane(D[c], c);
+          const bool ok = d > 0.0;
+          if (!ok && !bad) bad = j0 + c + 1;
+          const double piv = ok ? sqrt(d) : 1.0;
+          D[c] = a == c ? piv : D[c] / piv;
+#pragma unroll
+          for (int b = c + 1; b < kCholP; ++b) {
+            const double l = read_lane(D[c], b);
+            if (a >= b) D[b] = fma(-D[c], l, D[b]);
+          }
+        }
+      }
+      if (lane < pb)
+#pragma unroll
+        for (int b = 0; b < kCholP; ++b)
+          if (b <= a) Ls[(j0 + a) * ld + j0 + b] = D[b];
+    }
+    __syncthreads();
+    if (t < m) {  // a row below: against the diagonal block
+      double* row = Ls + (base + t) * ld + j0;
+      double x[kCholP];
+#pragma unroll
+      for (int c = 0; c < kCholP; ++c) x[c] = row[c];
+#pragma unroll
+      for (int c = 0; c < kCholP; ++c) {
+        double v = x[c];
+        const double* L = Ls + (j0 + c) * ld + j0;
+#pragma unroll
+        for (int cc = 0; cc < c; ++cc) v = fma(-x[cc], L[cc], v);
+        x[c] = v / L[c];
+        row[c] = x[c];
+      }
+    }
+    __syncthreads();
+    const int nt = (m + 3) / 4;
+    for (int e = t; e < nt * (nt + 1) / 2; e += kCholThreads) {  // trailing tile (ti, tj), ti >= tj
+      int ti = (int)((sqrtf(8.f * (float)e + 1.f) - 1.f) * 0.5f);
+      if (ti * (ti + 1) / 2 > e) --ti;
+      if ((ti + 1) * (ti + 2) / 2 <= e) ++ti;
+      const int tj = e - ti * (ti + 1) / 2, i0 = base + 4 * ti, l0 = base + 4 * tj;
+      double acc[4][4] = {};
+#pragma unroll 4
+      for (int c = 0; c < kCholP; ++c) {
+        double x[4], y[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          x[u] = Ls[min(i0 + u, r - 1) * ld + j0 + c];
+          y[u] = Ls[min(l0 + u, r - 1) * ld + j0 + c];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) acc[u][v] = fma(x[u], y[v], acc[u][v]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int i = i0 + u, l = l0 + v;
+          if (i < r && l <= i) Ls[i * ld + l] -= acc[u][v];
+        }
+    }
+    __syncthreads();
+  }
+  for (int i = w; i < r; i += kCholThreads / 64)
+    for (int l = lane; l < r; l += 64) R[(int64_t)i * r + l] = l >= i ? Ls[l * ld + i] : 0.0;
+  if (t == 0) status[0] = bad;
+}
+
 int chol_inv(hipStream_t s, int32_t r, double* G, double shift, double* R, double* Rinv, int32_t* status) {
   MMSB_CHECK_ARG(r >= 1 && r <= 4096, "chol_inv: r=%d out of range", r);
+  auto inverse = [&]() {
+    const int threads = (r + 63) / 64 * 64;
+    const dim3 grid((r + kTrinvCols - 1) / kTrinvCols);
+    if (r <= 512) hipLaunchKernelGGL((trinv_cols_kernel<512>), grid, dim3(threads), 0, s, r, R, Rinv);
+    else hipLaunchKernelGGL((trinv_cols_kernel<1024>), grid, dim3(threads), 0, s, r, R, Rinv);
+  };
+  if (r <= kCholSmall) {
+    const void* fn = reinterpret_cast<const void*>(chol_small_kernel);
+    MMSB_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(double) * kCholSmall * (kCholSmall | 1)));
+    hipLaunchKernelGGL(chol_small_kernel, dim3(1), dim3(kCholThreads), sizeof(double) * r * (r | 1), s, r, G, shift, R, status);
+    MMSB_LAUNCH_CHECK();
+    inverse();
+    MMSB_LAUNCH_CHECK();
+    return MMSB_OK;
+  }
   hipLaunchKernelGGL(chol_shift_kernel, dim3(1), dim3(kCholThreads), 0, s, r, G, shift, status);
   MMSB_LAUNCH_CHECK();
   for (int j0 = 0; j0 < r; j0 += kCholP) {
@@ -1155,8 +1296,7 @@ int chol_inv(hipStream_t s, int32_t r, double* G, double shift, double* R, doubl
     const int nt = (r + 31) / 32;
     hipLaunchKernelGGL(chol_transpose_kernel, dim3(nt, nt), dim3(256), 0, s, r, G, R);
     MMSB_LAUNCH_CHECK();
-    const int threads = (r + 63) / 64 * 64;
-    hipLaunchKernelGGL(trinv_cols_kernel, dim3((r + kTrinvCols - 1) / kTrinvCols), dim3(threads), 0, s, r, R, Rinv);
+    inverse();
   } else if (r <= 2048)
     hipLaunchKernelGGL(trinv_kernel<8>, dim3(1), dim3(1024), 0, s, r, G, R, Rinv);
   else
