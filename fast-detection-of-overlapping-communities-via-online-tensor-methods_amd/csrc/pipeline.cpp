@@ -129,6 +129,7 @@ struct mmsb_ctx {
   bool y16_valid = false;
   bool have_phi = false;
   // stop request (forceExit_flag, stpm.c:61,754): set from any thread, honoured between epochs
+  int64_t epoch_runs[2][2][2] = {};  // whole epochs launched of each kind
   std::atomic<int> stop_req{0};
   std::atomic<StgdSmallCtl*> small_ctl{nullptr};  // pinned; its stop follows stop_req during a one-workgroup run
   // eigen / post
@@ -838,7 +839,10 @@ static int run_stgd_steps(mmsb_ctx* c, int64_t nsteps, int32_t precision, StgdTi
   };
   // Whole epochs that start at an epoch boundary replay a captured HIP graph of the epoch's
   // launches (one graph per precision, Phi ping-pong parity and end-test setting); anything else
-  // launches directly.
+  // launches directly, and so do the first kDirectEpochs epochs of a kind: capturing and instantiating a graph costs
+  // what several epochs of direct launches lose to it (29079 rows, k = 100, b = 1024: four epochs take 4.4 ms with
+  // graphs from the first and 3.9 - 4.1 ms this way, twelve 10.5 and 11.1, as many again 8.9).
+  constexpr int kDirectEpochs = 2;
   const bool renorm_aligned = c->cfg.renorm_every <= 1 || spe % c->cfg.renorm_every == 0;
   if (rule) TRY(stgd_set_i64(c->s, &c->stopctl->stop_at, INT64_MAX));
   int64_t done = 0;
@@ -871,7 +875,7 @@ static int run_stgd_steps(mmsb_ctx* c, int64_t nsteps, int32_t precision, StgdTi
     if (rule) TRY(stgd_set_i64(c->s, &c->stopctl->base, step0));
     const bool epoch_aligned =
         (step0 % spe == 0) && (nsteps - done >= spe) && renorm_aligned && c->cfg.use_graphs && !timing;
-    if (epoch_aligned) {
+    if (epoch_aligned && c->epoch_runs[precision][c->cur][rule ? 1 : 0]++ >= kDirectEpochs) {
       TRY(dalloc(c, c->frob_epoch, (size_t)spe));
       hipGraphExec_t& ge = c->epoch_graph[precision][c->cur][rule ? 1 : 0];
       if (!ge) {
