@@ -378,7 +378,7 @@ int64_t mmsb_get_size(mmsb_ctx* ctx, int32_t what);
 /* Blocks until all work of the context has finished. */
 int mmsb_sync(mmsb_ctx* ctx);
 /* Releases the process-wide resources the library keeps between calls -- the pinned staging of large
- * copies, the host-CSR SpMM's staging, slots and copy stream, the CSR sort temporaries -- and the
+ * copies, the host-CSR SpMM's staging, slots and copy stream, the CSR sort temporaries, device blocks of closed contexts -- and the
  * context of the program-level entry points (pre_proc / GPU_Task / post_proc). No counterpart in the
  * reference. Call it before the HIP runtime is torn down (the Python binding does so at interpreter
  * exit); mmsb_destroy of the last live context releases the same resources. Later calls re-create
