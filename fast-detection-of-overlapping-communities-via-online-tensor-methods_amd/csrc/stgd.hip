@@ -1849,13 +1849,12 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
     log_entry(st - 1, cur);
     if (lane == 0) a.ctl->ran = st;
   }
+  // all of Phi's buffer, as the phase kernels write it: a diverged run may have left anything in the padding
   float* phi_out = cur ? a.phi1 : a.phi0;
-  if (w < 4)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int r = 8 * w + 4 * h + e;
-      phi_out[r * kp + c] = S.phif[cur][r][c];
-    }
+  for (int e = threadIdx.x; e < kp * kp; e += kSmallThreads) {
+    const int r = e / kp, j = e % kp;
+    phi_out[e] = r < 32 && j < 32 ? S.phif[cur][r][j] : 0.f;
+  }
 }
 
 // ---- the same for k <= 16 in FP32: one 16 x 16 block -----------------------------------------------------
@@ -2153,10 +2152,11 @@ __global__ __launch_bounds__(kSmall16Threads, 1) void stgd_small16_kernel(SmallA
     log_entry(st - 1, cur, cur == 0 ? 2 : cur - 1);
     if (lane == 0) a.ctl->ran = st;
   }
-  float* phi_out = (st & 1) ? a.phi1 : a.phi0;
-  if (w == OWNER)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) phi_out[(4 * g + i) * kp + c] = x[i];
+  float* phi_out = (st & 1) ? a.phi1 : a.phi0;  // all of the buffer, as in the 32-wide kernel
+  for (int e = threadIdx.x; e < kp * kp; e += kSmall16Threads) {
+    const int r = e / kp, j = e % kp;
+    phi_out[e] = r < 16 && j < 16 ? S.phif[cur][r][j] : 0.f;
+  }
 }
 
 // ---- resolving the arguments (host) ------------------------------------------------------------------
