@@ -60,7 +60,8 @@ __device__ inline void block_m(const double (&ms)[NM], double (&part)[NM][256], 
 // pass over Phi for the three), turned into K_A, K_B, K_C in registers, with the column sums of B o C,
 // A o C, A o B and of the loss terms over the block's rows (cpart [rt][4][k]) and m = Phi^T mu (by the first row
 // of blocks). The ct * ct workgroups after them: H = (Phi^T Phi)^o2 and the sum of (Phi^T Phi)^o3 per block
-// (gpart). Two workgroups per CU: the 64 x 64 form needs the cap at 256 registers for it (502 -> 395 us per call
+// (gpart). Rows from nb and columns from k on stay out of the sums: an infinite entry of Phi makes NaN of their
+// zeros. Two workgroups per CU: the 64 x 64 form needs the cap at 256 registers for it (502 -> 395 us per call
 // at k = 500). The element-wise pass this replaces ran k threads over all nb rows (1.49 ms of 3.73 at k = 500,
 // nb = 4000; 0.35 of 0.83 ms at k = 100, nb = 1024), and the products one vector-ALU launch each.
 template <int T, typename TY>
@@ -91,8 +92,10 @@ __global__ __launch_bounds__(256, 2) void adj_products_kernel(int32_t nb, int32_
     double s = 0.0;
     each_elem<T>([&](int r, int c, int u, int v, int gi) {
       const double x = acc[u][v][gi];
-      s = fma(x * x, x, s);
-      if (i0 + r < k && j0 + c < k) H[(int64_t)(i0 + r) * k + j0 + c] = x * x;
+      if (i0 + r < k && j0 + c < k) {
+        s = fma(x * x, x, s);
+        H[(int64_t)(i0 + r) * k + j0 + c] = x * x;
+      }
     });
     __syncthreads();
     sm.red[threadIdx.x] = s;
@@ -117,15 +120,17 @@ __global__ __launch_bounds__(256, 2) void adj_products_kernel(int32_t nb, int32_
   each_elem<T>([&](int r, int c, int u, int v, int g) {
     const double a = acc[0][u][v][g], b = acc[1][u][v][g], cc = acc[2][u][v][g];
     const double ma = sm.e.m[0][c], mb = sm.e.m[1][c], mc = sm.e.m[2][c];
-    s[v][0] += b * cc;
-    s[v][1] += a * cc;
-    s[v][2] += a * b;
-    s[v][3] += c3 * a * b * cc + c1 * (a * b * mc + a * mb * cc + ma * b * cc);
-    if (x0 + r < nb && c0 + c < k) {
-      const int64_t o = (x0 + r) * k + c0 + c;
-      KA[o] = c3 * b * cc + c1 * (b * mc + mb * cc);
-      KB[o] = c3 * a * cc + c1 * (a * mc + ma * cc);
-      KC[o] = c3 * a * b + c1 * (a * mb + ma * b);
+    if (x0 + r < nb) {
+      s[v][0] += b * cc;
+      s[v][1] += a * cc;
+      s[v][2] += a * b;
+      s[v][3] += c3 * a * b * cc + c1 * (a * b * mc + a * mb * cc + ma * b * cc);
+      if (c0 + c < k) {
+        const int64_t o = (x0 + r) * k + c0 + c;
+        KA[o] = c3 * b * cc + c1 * (b * mc + mb * cc);
+        KB[o] = c3 * a * cc + c1 * (a * mc + ma * cc);
+        KC[o] = c3 * a * b + c1 * (a * mb + ma * b);
+      }
     }
   });
   block_colsum<T, 4>(s, sm.e.red, cpart + (int64_t)tr * 4 * k, k, c0);
