@@ -1583,6 +1583,17 @@ __device__ inline void small_new_phi(SmallShm<MODE>& S, int buf, const float v[1
   }
 }
 
+// Clears the buffer of the next Phi ([64 x 64]) outside the T x T block that the run writes: the phase kernels and batches
+// that go on from it take all of it, and a diverged run may have left anything there. (The current Phi's is clean:
+// whatever leaves a Phi writes or has cleared the whole buffer.) Done while the first loads are on their way: 0.2 us
+// of a run's 16-21 for one step. As part of the stores at a run's end it cost 1-2 % of every step (registers of the loop).
+constexpr int kSmallKp = 64;
+template <int T>
+__device__ inline void small_clear(const SmallArgs& a) {
+  for (int e = threadIdx.x; e < kSmallKp * kSmallKp / 4; e += blockDim.x)
+    if (e / (kSmallKp / 4) >= T || e % (kSmallKp / 4) * 4 >= T) reinterpret_cast<float4*>(a.phi1)[e] = make_float4(0.f, 0.f, 0.f, 0.f);
+}
+
 template <int MODE, typename TY>
 __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs a) {
   extern __shared__ __attribute__((aligned(16))) unsigned char small_raw[];
@@ -1654,6 +1665,7 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
     small_new_phi<MODE>(S, 0, v);
   }
   prefetch(pos * a.bl);
+  small_clear<32>(a);
   __syncthreads();
 
   int cur = 0;
@@ -1849,12 +1861,13 @@ __global__ __launch_bounds__(kSmallThreads, 1) void stgd_small_kernel(SmallArgs 
     log_entry(st - 1, cur);
     if (lane == 0) a.ctl->ran = st;
   }
-  // all of Phi's buffer, as the phase kernels write it: a diverged run may have left anything in the padding
   float* phi_out = cur ? a.phi1 : a.phi0;
-  for (int e = threadIdx.x; e < kp * kp; e += kSmallThreads) {
-    const int r = e / kp, j = e % kp;
-    phi_out[e] = r < 32 && j < 32 ? S.phif[cur][r][j] : 0.f;
-  }
+  if (w < 4)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 8 * w + 4 * h + e;
+      phi_out[r * kp + c] = S.phif[cur][r][c];
+    }
 }
 
 // ---- the same for k <= 16 in FP32: one 16 x 16 block -----------------------------------------------------
@@ -1909,6 +1922,7 @@ __global__ __launch_bounds__(kSmall16Threads, 1) void stgd_small16_kernel(SmallA
   Small16Shm& S = *reinterpret_cast<Small16Shm*>(small_raw);
   constexpr int P1W = 8, OWNER = 8, P2A = 9, P2B = 10, AUX = 11;  // roles of the waves
   constexpr int PF = 4;                                          // P2: groups of 32 minibatch rows loaded ahead
+  small_clear<16>(a);
   const int w = wave_id(), lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
   const int kp = a.kp, b = a.b, nt = b / 32, nu = b / 16, ldc = b + 4;
   const float* ya = static_cast<const float*>(a.ya);
@@ -2152,11 +2166,10 @@ __global__ __launch_bounds__(kSmall16Threads, 1) void stgd_small16_kernel(SmallA
     log_entry(st - 1, cur, cur == 0 ? 2 : cur - 1);
     if (lane == 0) a.ctl->ran = st;
   }
-  float* phi_out = (st & 1) ? a.phi1 : a.phi0;  // all of the buffer, as in the 32-wide kernel
-  for (int e = threadIdx.x; e < kp * kp; e += kSmall16Threads) {
-    const int r = e / kp, j = e % kp;
-    phi_out[e] = r < 16 && j < 16 ? S.phif[cur][r][j] : 0.f;
-  }
+  float* phi_out = (st & 1) ? a.phi1 : a.phi0;
+  if (w == OWNER)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) phi_out[(4 * g + i) * kp + c] = x[i];
 }
 
 // ---- resolving the arguments (host) ------------------------------------------------------------------
@@ -2418,7 +2431,7 @@ static bool p2_spread(const StgdArgs& a) {
 }
 
 bool stgd_small_fits(const StgdArgs& a) {
-  return a.k <= 32 && a.kp == 64 && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
+  return a.k <= 32 && a.kp == kSmallKp && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
 }
 
 template <int MODE, typename TY>
