@@ -13,6 +13,7 @@
 
 #include "common.h"
 #include "dense.h"
+#include "devmem.h"
 #include "xfer.h"
 
 namespace mmsb {
@@ -59,7 +60,7 @@ hipError_t scratch_take(SortScratch& s, int i, size_t bytes, T** out) {
     if (s.p[i]) (void)hipFree(s.p[i]);
     s.p[i] = nullptr;
     s.bytes[i] = 0;
-    const hipError_t e = hipMalloc(&s.p[i], bytes);
+    const hipError_t e = dev_malloc(&s.p[i], bytes);
     if (e != hipSuccess) return e;
     s.bytes[i] = bytes;
   }

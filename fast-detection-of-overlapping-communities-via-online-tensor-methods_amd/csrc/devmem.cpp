@@ -27,6 +27,17 @@ void drop(DevCache& c) {
   c.kept.clear();
   c.bytes = 0;
 }
+
+// hipMalloc, once more without the kept blocks if it fails.
+hipError_t malloc_or_drop(DevCache& c, void** p, size_t bytes) {
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess && !c.kept.empty()) {
+    (void)hipGetLastError();
+    drop(c);
+    e = hipMalloc(p, bytes);
+  }
+  return e;
+}
 }  // namespace
 
 hipError_t dev_alloc(void** p, size_t bytes) {
@@ -45,14 +56,16 @@ hipError_t dev_alloc(void** p, size_t bytes) {
     c.kept.erase(it);
     return hipSuccess;
   }
-  e = hipMalloc(p, bytes);
-  if (e != hipSuccess && !c.kept.empty()) {
-    (void)hipGetLastError();
-    drop(c);
-    e = hipMalloc(p, bytes);
-  }
+  e = malloc_or_drop(c, p, bytes);
   if (e == hipSuccess) c.live[*p] = {dev, bytes};
   return e;
+}
+
+hipError_t dev_malloc(void** p, size_t bytes) {
+  *p = nullptr;
+  DevCache& c = dev_cache();
+  std::lock_guard<std::mutex> lock(c.mu);
+  return malloc_or_drop(c, p, bytes);
 }
 
 void dev_free(void* p) {
@@ -69,6 +82,16 @@ void dev_free(void* p) {
   } else {
     (void)hipFree(p);
   }
+}
+
+void dev_release(void* p) {
+  if (!p) return;
+  DevCache& c = dev_cache();
+  {
+    std::lock_guard<std::mutex> lock(c.mu);
+    if (c.live.erase(p) == 0) return;
+  }
+  (void)hipFree(p);
 }
 
 size_t dev_cached_bytes() {

@@ -176,7 +176,7 @@ static void dfree(mmsb_ctx* c, T*& p) {
   (void)hipStreamSynchronize(c->s);
   auto it = std::find(c->allocs.begin(), c->allocs.end(), (void*)p);
   if (it != c->allocs.end()) c->allocs.erase(it);
-  dev_free(p);
+  dev_release(p);
   p = nullptr;
 }
 
@@ -1115,7 +1115,7 @@ extern "C" int mmsb_batch_autotune(mmsb_batch* b, int32_t* best_grid, double* be
   if (b->save.empty())
     for (mmsb_ctx* c : b->ctx) {
       float* q = nullptr;
-      HCHK(hipMalloc(&q, sizeof(float) * (size_t)c->kp * c->kp));
+      HCHK(dev_malloc(&q, sizeof(float) * (size_t)c->kp * c->kp));
       b->save.push_back(q);
     }
   for (size_t i = 0; i < b->ctx.size(); ++i) {
@@ -1747,11 +1747,11 @@ extern "C" int mmsb_grad(mmsb_ctx* c, int64_t row0, int32_t nrows, const double*
   hipError_t e = hipSuccess;
   const size_t ybytes = sizeof(float) * (size_t)nrows * kp;
   for (float** p : {&ya, &yb, &yc})
-    if (e == hipSuccess) e = hipMalloc(p, ybytes);
-  if (e == hipSuccess) e = hipMalloc(&dphi, sizeof(double) * k * k);
-  if (e == hipSuccess) e = hipMalloc(&dgrad, sizeof(double) * k * k);
-  if (e == hipSuccess) e = hipMalloc(&dloss, sizeof(double));
-  if (e == hipSuccess) e = hipMalloc(&work, wb);
+    if (e == hipSuccess) e = dev_malloc(p, ybytes);
+  if (e == hipSuccess) e = dev_malloc(&dphi, sizeof(double) * k * k);
+  if (e == hipSuccess) e = dev_malloc(&dgrad, sizeof(double) * k * k);
+  if (e == hipSuccess) e = dev_malloc(&dloss, sizeof(double));
+  if (e == hipSuccess) e = dev_malloc(&work, wb);
   if (e != hipSuccess) {
     cleanup();
     return set_error(MMSB_ERR_NOMEM, "grad: %s", hipGetErrorString(e));

@@ -21,6 +21,7 @@
 #include <vector>
 
 #include "dense.h"
+#include "devmem.h"
 #include "host_util.h"
 #include "mmsb_stpm.h"
 #include "xfer.h"
@@ -101,10 +102,10 @@ int ensure_slot(Slot& sl, int64_t rows, int64_t nnz, bool vals) {
     sl.vals = nullptr;
     sl.rows_cap = std::max(rows, sl.rows_cap);
     sl.nnz_cap = std::max(nnz, sl.nnz_cap);
-    SHIP(hipMalloc(&sl.rowptr, sizeof(int32_t) * (size_t)(sl.rows_cap + 1)));
-    SHIP(hipMalloc(&sl.order, sizeof(int32_t) * (size_t)sl.rows_cap));
-    SHIP(hipMalloc(&sl.colidx, sizeof(int32_t) * (size_t)std::max<int64_t>(sl.nnz_cap, 1)));
-    if (vals) SHIP(hipMalloc(&sl.vals, sizeof(float) * (size_t)std::max<int64_t>(sl.nnz_cap, 1)));
+    SHIP(dev_malloc(&sl.rowptr, sizeof(int32_t) * (size_t)(sl.rows_cap + 1)));
+    SHIP(dev_malloc(&sl.order, sizeof(int32_t) * (size_t)sl.rows_cap));
+    SHIP(dev_malloc(&sl.colidx, sizeof(int32_t) * (size_t)std::max<int64_t>(sl.nnz_cap, 1)));
+    if (vals) SHIP(dev_malloc(&sl.vals, sizeof(float) * (size_t)std::max<int64_t>(sl.nnz_cap, 1)));
   }
   const size_t hb = sizeof(int32_t) * (size_t)(2 * sl.rows_cap + 1) + sizeof(int32_t) * (size_t)sl.nnz_cap +
                     (sl.vals ? sizeof(float) * (size_t)sl.nnz_cap : 0);

@@ -41,6 +41,7 @@
 #include <vector>
 
 #include "common.h"
+#include "devmem.h"
 #include "stgd.h"
 #include "wave.h"
 
@@ -2725,7 +2726,7 @@ int stgd_batch_plan(StgdBatch*& out, int32_t precision, const std::vector<StgdBa
   hipError_t e;
   auto put = [](auto** dst, const auto& src) -> hipError_t {
     const size_t bytes = sizeof(src[0]) * src.size();
-    const hipError_t me = hipMalloc(dst, bytes);
+    const hipError_t me = dev_malloc(dst, bytes);
     return me != hipSuccess ? me : hipMemcpy(*dst, src.data(), bytes, hipMemcpyHostToDevice);
   };
   if ((e = put(&b->d_args, args)) != hipSuccess || (e = put(&b->d_first, first)) != hipSuccess ||
