@@ -1039,9 +1039,9 @@ __device__ inline void quad_mm(floatx4& acc, const float* a, int64_t lda, const 
 
 // P2 of an FP32 step in 16 x 16 tiles, four times the workgroups: of a 32 x 32 tile the two waves that take Y_C^T C_g
 // pass MFMAs in a row for 6.8 us at b = 1024 while most compute units have no tile (16 tiles at k = 100). P2 at k = 100,
-// b = 1024 (2048): 4.3 (8.1) us against 10.9 (20.5).
+// b = 1024 (2048): 4.3 (8.1) us against 10.9 (20.5). Two waves take each of the two products: builds with eight waves per
+// workgroup have no such tiles.
 __device__ __forceinline__ void p2_quad_tile(const P2Args& a, int tile, StgdSmem& sm) {
-  static_assert(kWaves == 4, "two waves for each of the two products");
   const int kp = a.kp, nq = kp / 16;
   const int w = wave_id(), lane = threadIdx.x & 63;
   const int64_t i0 = (int64_t)(tile / nq) * 16, j0 = (int64_t)(tile % nq) * 16;
@@ -1272,7 +1272,10 @@ __device__ __forceinline__ void phase_tile(const typename ArgsOf<PHASE>::type& a
   constexpr bool SPLIT = KMODE == MM_BF16X3;
   if constexpr (PHASE == PH_P1) p1_tile<DMODE, KMODE, TY, TPH>(a, tile, sm, log);
   else if constexpr (PHASE == PH_P2) p2_tile<DMODE, KMODE, TY, TPH>(a, tile, sm);
-  else if constexpr (PHASE == PH_P2S) p2_quad_tile(a, tile, sm);
+  else if constexpr (PHASE == PH_P2S) {
+    static_assert(PHASE == PH_P2S && kWaves == 4, "four waves per tile");
+    p2_quad_tile(a, tile, sm);
+  }
   else if constexpr (PHASE == PH_GRAM) gram_tile<KMODE>(a, tile, sm);
   else if constexpr (PHASE == PH_QPOLY) qpoly_tile<KMODE>(a, tile, sm);
   else if constexpr (PHASE == PH_UPDATE) update_tile<KMODE>(a, tile, sm);
@@ -2428,11 +2431,11 @@ static bool step_renorms(int64_t gstep, int32_t renorm_every, int32_t ns_iters) 
 constexpr int kQuadTiles = 100;  // of 32 x 32: kp <= 320
 template <int DMODE>
 static bool p2_spread(const StgdArgs& a) {
-  return DMODE == MM_F32 && !a.frob_pre && phase_tiles(PH_P2, a.kp, a.b) <= kQuadTiles;
+  return DMODE == MM_F32 && kWaves == 4 && !a.frob_pre && phase_tiles(PH_P2, a.kp, a.b) <= kQuadTiles;
 }
 
-bool stgd_small_fits(const StgdArgs& a) {
-  return a.k <= 32 && a.kp == kSmallKp && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
+bool stgd_small_fits(const StgdArgs& a) {  // the one-workgroup kernels add in the order of four-wave tiles
+  return kWaves == 4 && a.k <= 32 && a.kp == kSmallKp && a.b <= kSmallB && !a.y_window && !a.stop && !a.frob_pre;
 }
 
 template <int MODE, typename TY>
@@ -2515,7 +2518,7 @@ static int run_steps(hipStream_t s, const StgdArgs& args, const void* YA, const 
       MMSB_PHASE(PH_P1)
       MMSB_PHASE(PH_P2)
       case PH_P2S:
-        if constexpr (DMODE == MM_F32) {
+        if constexpr (DMODE == MM_F32 && kWaves == 4) {
           if (stop.stop)
             hipLaunchKernelGGL((stgd_phase_kernel<DMODE, KMODE, TY, TPH, PH_P2S, true>), grid, block, 0, s, a.p2, stop);
           else
