@@ -122,14 +122,18 @@ struct mmsb_ctx {
   int64_t frob_cap = 0, steps_done = 0;
   bf16_bits *YA16 = nullptr, *YB16 = nullptr, *YCt16 = nullptr;
   double* frob_epoch = nullptr;            // per-epoch log written by captured epochs
-  // captured epochs, [precision][cur][end test on]
-  hipGraphExec_t epoch_graph[2][2][2] = {{{nullptr, nullptr}, {nullptr, nullptr}}, {{nullptr, nullptr}, {nullptr, nullptr}}};
+  // whole epochs of each kind, [precision][cur][end test on]: how many were run since the settings changed, and the graph
+  // that the later ones replay
+  struct EpochKind {
+    int64_t runs = 0;
+    hipGraphExec_t graph = nullptr;
+  };
+  EpochKind epoch_kind[2][2][2];
   StgdStop* stopctl = nullptr;             // device state of the per-step end test (stpm.c:747-765)
   float *phiT = nullptr, *phitT = nullptr, *phiaT = nullptr;
   bool y16_valid = false;
   bool have_phi = false;
   // stop request (forceExit_flag, stpm.c:61,754): set from any thread, honoured between epochs
-  int64_t epoch_runs[2][2][2] = {};  // whole epochs launched of each kind
   std::atomic<int> stop_req{0};
   std::atomic<StgdSmallCtl*> small_ctl{nullptr};  // pinned; its stop follows stop_req during a one-workgroup run
   // eigen / post
@@ -180,16 +184,16 @@ static void dfree(mmsb_ctx* c, T*& p) {
   p = nullptr;
 }
 
-// Captured epoch graphs hold the step parameters and buffer addresses in their kernel arguments.
+// Captured epoch graphs hold the step parameters and buffer addresses in their kernel arguments. The epochs count anew
+// from here: a learning-rate schedule that changes them every epoch captures none.
 static int drop_epoch_graphs(mmsb_ctx* c) {
   HCHK(hipStreamSynchronize(c->s));
-  for (auto& plane : c->epoch_graph)
+  for (auto& plane : c->epoch_kind)
     for (auto& row : plane)
-      for (hipGraphExec_t& g : row)
-        if (g) {
-          HCHK(hipGraphExecDestroy(g));
-          g = nullptr;
-        }
+      for (auto& kind : row) {
+        if (kind.graph) HCHK(hipGraphExecDestroy(kind.graph));
+        kind = {};
+      }
   return MMSB_OK;
 }
 
@@ -839,7 +843,7 @@ static int run_stgd_steps(mmsb_ctx* c, int64_t nsteps, int32_t precision, StgdTi
   };
   // Whole epochs that start at an epoch boundary replay a captured HIP graph of the epoch's
   // launches (one graph per precision, Phi ping-pong parity and end-test setting); anything else
-  // launches directly, and so do the first kDirectEpochs epochs of a kind: capturing and instantiating a graph costs
+  // launches directly, and so do the first kDirectEpochs epochs of a kind under the same settings: capturing and instantiating a graph costs
   // what several epochs of direct launches lose to it (29079 rows, k = 100, b = 1024: four epochs take 4.4 ms with
   // graphs from the first and 3.9 - 4.1 ms this way, twelve 10.5 and 11.1, as many again 8.9).
   constexpr int kDirectEpochs = 2;
@@ -875,9 +879,10 @@ static int run_stgd_steps(mmsb_ctx* c, int64_t nsteps, int32_t precision, StgdTi
     if (rule) TRY(stgd_set_i64(c->s, &c->stopctl->base, step0));
     const bool epoch_aligned =
         (step0 % spe == 0) && (nsteps - done >= spe) && renorm_aligned && c->cfg.use_graphs && !timing;
-    if (epoch_aligned && c->epoch_runs[precision][c->cur][rule ? 1 : 0]++ >= kDirectEpochs) {
+    auto& kind = c->epoch_kind[precision][c->cur][rule ? 1 : 0];
+    if (epoch_aligned && kind.runs++ >= kDirectEpochs) {
       TRY(dalloc(c, c->frob_epoch, (size_t)spe));
-      hipGraphExec_t& ge = c->epoch_graph[precision][c->cur][rule ? 1 : 0];
+      hipGraphExec_t& ge = kind.graph;
       if (!ge) {
         hipGraph_t g = nullptr;
         int cur = c->cur;
@@ -1506,10 +1511,10 @@ extern "C" void mmsb_destroy(mmsb_ctx* c) {
   if (!c) return;
   (void)hipSetDevice(c->cfg.device);
   if (c->s) (void)hipStreamSynchronize(c->s);
-  for (auto& plane : c->epoch_graph)
+  for (auto& plane : c->epoch_kind)
     for (auto& row : plane)
-      for (hipGraphExec_t& g : row)
-        if (g) (void)hipGraphExecDestroy(g);
+      for (auto& kind : row)
+        if (kind.graph) (void)hipGraphExecDestroy(kind.graph);
   if (!c->allocs.empty()) (void)hipDeviceSynchronize();  // a batch's stream may still use the blocks
   for (void* p : c->allocs) dev_free(p);
   if (StgdSmallCtl* ctl = c->small_ctl.load()) (void)hipHostFree(ctl);
