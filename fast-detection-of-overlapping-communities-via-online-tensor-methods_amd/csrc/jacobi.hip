@@ -301,11 +301,20 @@ static int run_sweeps_rm(hipStream_t s, int32_t r, double* A, double* Vw, int32_
   return MMSB_OK;
 }
 
+// Largest r whose 2B columns of A (and of V when it is wanted) fit in the 160 KiB of LDS.
+template <int B, bool WV>
+constexpr int sweep_r_max() { return (160 * 1024 - 256) / (int)(sizeof(double) * 2 * (WV ? 2 : 1) * B); }
+
+// Smallest r that comes to blocks of B columns: jacobi_svd takes blocks twice as wide while they are allowed and fit.
+template <int B, bool WV>
+constexpr int sweep_r_min() { return 2 * B <= MMSB_JACOBI_BMAX ? sweep_r_max<2 * B, WV>() + 1 : 1; }
+
 template <int B, bool WV>
 static int run_sweeps(hipStream_t s, int32_t r, double* A, double* Vw, int32_t* counters) {
   if constexpr (B >= 4) {  // columns in registers: up to 20 entries per lane
-#define MMSB_RM(RM, MIN) \
-  if (r <= 64 * RM) return run_sweeps_rm<B, WV, RM, MIN>(s, r, A, Vw, counters);
+#define MMSB_RM(RM, MIN)                                                            \
+  if constexpr (MIN <= sweep_r_max<B, WV>() && 64 * RM >= sweep_r_min<B, WV>())      \
+    if (r <= 64 * RM) return run_sweeps_rm<B, WV, RM, MIN>(s, r, A, Vw, counters);
     MMSB_RM(1, 1)
     MMSB_RM(2, 65)
     MMSB_RM(4, 129)
@@ -315,7 +324,8 @@ static int run_sweeps(hipStream_t s, int32_t r, double* A, double* Vw, int32_t* 
     MMSB_RM(20, 769)
 #undef MMSB_RM
   }
-  return run_sweeps_rm<B, WV, 0, 0>(s, r, A, Vw, counters);
+  if constexpr (B < 4 || sweep_r_max<B, WV>() > 64 * 20) return run_sweeps_rm<B, WV, 0, 0>(s, r, A, Vw, counters);
+  return set_error(MMSB_ERR_ARG, "jacobi: no form for r=%d in blocks of %d columns", r, B);
 }
 
 int jacobi_svd(hipStream_t s, int32_t r, double* A, double* U, double* sigma, double* V, void* work, int32_t* sweeps_out) {

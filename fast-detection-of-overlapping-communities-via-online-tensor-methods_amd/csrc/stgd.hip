@@ -2402,11 +2402,6 @@ int stgd_set_i64(hipStream_t s, int64_t* p, int64_t v) {
   return MMSB_OK;
 }
 
-__global__ void zero_f64_kernel(int64_t n, double* p) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t < n) p[t] = 0.0;
-}
-
 __global__ void f32_to_bf16_kernel(int64_t n, const float* __restrict__ in, __bf16* __restrict__ out) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (t < n) out[t] = (__bf16)in[t];
