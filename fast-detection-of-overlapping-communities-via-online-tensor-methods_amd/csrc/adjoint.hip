@@ -419,7 +419,7 @@ size_t grad_workspace_bytes(int32_t k, int32_t nb) {
 // 64 x 64 blocks read each operand half as often as 32 x 32 ones but leave CUs idle on small problems: they are
 // taken for the products once they make 192 workgroups, and for the contraction above k = 256 (below it the
 // k x k output has at most 16 of them): k = 500, nb = 4000 takes 387 us with 64 x 64 products, 431 with 32 x 32.
-// The contraction's rows are cut into S slices of at least 64 rows, about 512 workgroups in all. A whole call
+// The contraction's rows are cut into S slices of about 64 rows or more (nb = 65: 32 and 33), about 512 workgroups in all. A whole call
 // (three launches instead of 22): k = 100, nb = 1024 in FP32 828 -> 49 us, of which 28 in kernels; k = 500,
 // nb = 4000 in FP64 3.73 -> 0.39 ms, 32 TFLOP/s of FP64 MFMA.
 struct AdjShape {

@@ -69,9 +69,10 @@ int csr_rowsum(hipStream_t s, int32_t m, const int32_t* rowptr, const float* val
 
 // ---- C[p x q] (FP64) = alpha * A^T B, A [n x p], B [n x q] row-major ------------------------
 // The rows are cut into slices; each slice's partial tile of C goes to a workspace and a second kernel sums the
-// slices in order (deterministic result). The slice count is a function of the shape alone and every form below
-// adds the rows of a slice one after another (the MFMA forms four after four), so the form chosen for a call --
-// by how many workgroups its tiles make -- does not change a bit of C.
+// slices in order (deterministic result). The slice count is a function of the shape alone, and so is whether a
+// product with a vector over many rows takes tn_vec_kernel (four interleaved chains, slices of its own). Every other form
+// adds the rows of a slice one after another (the MFMA forms four after four), so which of them is chosen for a call -- by
+// how many workgroups its tiles make -- does not change a bit of C.
 // General form: 64 x 64 tiles, 16-row slabs of A and B through LDS as FP64, a 4 x 4 register tile per thread.
 template <typename TA, typename TB>
 __global__ __launch_bounds__(256) void tn_partial_kernel(int64_t n, int32_t p, int32_t q, const TA* __restrict__ A,

@@ -1354,9 +1354,9 @@ __global__ __launch_bounds__(kThreads, PHASE == PH_P1 ? 3 : 1) void stgd_phase_k
 //   waves 5, 6  Y_C^T C_g over the two halves of the minibatch
 //   wave 7      c_mu; the log entry of the previous step
 // The rows of Y of the next step are loaded during the Newton-Schulz iterations. One compute unit bounds the
-// minibatch: b = 512 takes about 9 us per step, beyond it (and beyond the LDS that holds C_g) the phase kernels
-// spread the work. At k = 10, b = 100 it takes 6.5 us (the phase kernels 27); the whole detection of a graph of 1000
-// nodes, 200 epochs, 57 -> 20 ms (FP32 at k <= 16 goes to stgd_small16_kernel).
+// minibatch: at b = 512 a step takes 8.7 us in BF16 and 16.1 in FP32 (k = 32; the phase kernels 23.0 and 24.3), beyond it
+// (and beyond the LDS that holds C_g) the phase kernels spread the work. At b = 100: 7.2 us in FP32 (k = 20) and 5.9 in
+// BF16 (k = 10), the phase kernels 23.2 and 22.5. FP32 at k <= 16 goes to stgd_small16_kernel.
 constexpr int kSmallB = 512;        // largest padded minibatch
 constexpr int kSmallThreads = 512;
 
